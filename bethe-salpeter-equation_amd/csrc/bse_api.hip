@@ -849,17 +849,32 @@ static int twostage_tridiag(bse_ctx* ctx, int n, void* H, int fp32, const double
     const int64_t ncnt = bse_chase_counters(n);
     int* prog = BUF(int, S_BPROG, ncnt + 4);
     HCK(bse_launch_zero_words(st, (ncnt + 4) / 2, prog));
-    int ncu = 0;
-    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess) ncu = 64;
-    // one workgroup per CU at most (all resident, so every waiter's
-    // predecessor runs); BSE_CHASE_GRID sets the count for measurements
-    int cgrid = std::max(1, ncu - 16);
-    if (const char* g = getenv("BSE_CHASE_GRID")) cgrid = std::max(1, std::min(atoi(g), ncu));
-    HCK(bse_launch_chase(st, n, b, AB, ldab, y, d, e, prog, prog + ncnt, cgrid));
-    HCK(hipEventRecord(tv[2], st));
     int err = 0;
-    HCK(hipMemcpyAsync(&err, prog + ncnt, sizeof(int), hipMemcpyDeviceToHost, st));
-    HCK(hipStreamSynchronize(st));
+    // band resident in LDS, one workgroup per 32 rows; BSE_CHASE=tasks (or a
+    // band with more workgroups than the device holds, or a device that did
+    // not hold them together) takes one wave per sweep instead
+    const char* che = getenv("BSE_CHASE");
+    const int64_t mel = (che && !strcmp(che, "tasks")) ? 0 : bse_chase_resident_workspace(n, b, ldab, ctx->device);
+    if (mel > 0) {
+        double2* msg = BUF(double2, S_BMSG, mel);
+        HCK(bse_launch_chase_resident(st, ctx->device, n, b, AB, ldab, y, d, e, msg, prog + ncnt));
+        HCK(hipEventRecord(tv[2], st));
+        HCK(hipMemcpyAsync(&err, prog + ncnt, sizeof(int), hipMemcpyDeviceToHost, st));
+        HCK(hipStreamSynchronize(st));
+        if (err == 2) HCK(bse_launch_zero_words(st, (ncnt + 4) / 2, prog));
+    }
+    if (mel <= 0 || err == 2) {
+        int ncu = 0;
+        if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess) ncu = 64;
+        // one workgroup per CU at most (all resident, so every waiter's
+        // predecessor runs); BSE_CHASE_GRID sets the count for measurements
+        int cgrid = std::max(1, ncu - 16);
+        if (const char* g = getenv("BSE_CHASE_GRID")) cgrid = std::max(1, std::min(atoi(g), ncu));
+        HCK(bse_launch_chase(st, n, b, AB, ldab, y, d, e, prog, prog + ncnt, cgrid));
+        HCK(hipEventRecord(tv[2], st));
+        HCK(hipMemcpyAsync(&err, prog + ncnt, sizeof(int), hipMemcpyDeviceToHost, st));
+        HCK(hipStreamSynchronize(st));
+    }
     float ms1 = 0.f, ms2 = 0.f;
     HCK(hipEventElapsedTime(&ms1, tv[0], tv[1]));
     HCK(hipEventElapsedTime(&ms2, tv[1], tv[2]));

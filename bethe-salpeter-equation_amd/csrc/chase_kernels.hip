@@ -35,6 +35,9 @@
 // Band storage: AB[c * ldab + d] = A(c + d, c), 0 <= d <= 2b (FP64).
 #include "bse_common.hpp"
 #include <cfloat>
+#include <mutex>
+
+extern "C" hipError_t bse_launch_zero_words(hipStream_t, int64_t, void*);
 
 #define CH_B 32                  // largest band half-width
 #define CH_W 4                   // sweeps (waves) per workgroup
@@ -64,7 +67,7 @@ __device__ inline Refl make_refl(double2 alpha, double ss) {
         const double nrm = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + ss);
         r.beta = (alpha.x >= 0.0) ? -nrm : nrm;
         r.tau = cmk((r.beta - alpha.x) / r.beta, -alpha.y / r.beta);
-        r.scal = cdiv(cmk(1.0, 0.0), cmk(alpha.x - r.beta, alpha.y));
+        r.scal = crecip(cmk(alpha.x - r.beta, alpha.y));
     }
     return r;
 }
@@ -371,6 +374,438 @@ __global__ __launch_bounds__(64 * CH_W) void k_chase(ChaseArgs a)
         }
         if (!alive) break;
     }
+}
+
+// ---------------------------------------------------------------------------
+// Bulge chasing with the band resident in LDS: workgroup k owns the blocks
+// D_k and X_k of every sweep instead of one sweep's blocks all along the
+// band.  From sweep s to sweep s + 1 its window moves down by one row and
+// one column, so with rows and columns kept at (index mod 32) nothing moves
+// in LDS; what a window lacks comes from its neighbours:
+//   right (k -> k + 1)  the reflector v_k, tau_k of sweep s, applied from
+//                       the right to X_{k+1};
+//   left (k + 1 -> k)   the first row of X_{k+1} and D_{k+1}(0, 0) (and the
+//                       first entry of its segment of y) after sweep s: the
+//                       row that enters D_k and X_k for sweep s + 1.  Of it
+//                       X_k sees only X_{k+1}(0, 0) = beta_{k+1} (the rest
+//                       of that row lies outside D_{k-1}), which is sent as
+//                       soon as it is known.
+// X_k's entering column is the first column of D_k (sweep s), handed over
+// inside the workgroup.  Rows past the matrix are zero and stay zero (a zero
+// column gives H = I), so no block is cut.
+//
+// Wave 0 (X) computes x = X_k H_{k-1} e_1, its reflector, sends v_k and beta_k
+// and then finishes X_k; wave 1 (D) applies H_k to D_k and y meanwhile.  Lane
+// (h, i) holds row i of the block, columns 16 h .. 16 h + 15.
+//
+// The rate is set by the cycle v_k(s) -> v_{k+1}(s) -> v_k(s + 1), two
+// messages and two 32 x 32 matrix-vector products with a reflector each.  A
+// message is one 16-byte store per lane and one polled 16-byte load: every
+// 8 bytes carry 4 bytes of data and the sweep's number, so the data itself
+// says when it is there, and no store has to complete before a flag is
+// written (0.44 us one way inside an XCD, 0.6 us across XCDs, measured).
+// A v or beta slot is written for sweep s + 1 only after its reader has
+// answered sweep s; row and D slots, read later in the sweep, have two
+// copies by the sweep's parity.
+//
+// Measured: 3.5 us per sweep (N = 4624: 16.2 ms, N = 6720: 23.8 ms) and
+// 4.2 us at N = 20736 (86.5 ms; 648 workgroups, so waves share SIMDs), against
+// 18 us per sweep (83, 121 and 374 ms) for k_chase above, one wave per sweep
+// with the band in device-coherent memory.
+//
+// Every workgroup must be resident (each waits on both neighbours): they meet
+// at a counter first (chase_meet) and leave together when that does not
+// happen in time, with the band, y, d and e untouched; the host then runs
+// k_chase, whose workgroups only ever wait on earlier ones.  k_chase also
+// serves bands with more workgroups than the device holds (n above 32768 on
+// 256 CUs with four workgroups each).
+// ---------------------------------------------------------------------------
+#define CHS_LD 33                             // LDS stride of a block's columns
+#define CHS_SPIN (1u << 23)                   // polls (each a memory round trip) before a wait is given up
+#define CHS_MEET_TICKS 200000000ull           // 2 s of the 100 MHz clock
+#define CHS_ABORT 0x80000000u
+
+struct ChaseSysArgs {
+    int n, ldab, npos;
+    const double2* AB;
+    double2* y;          // may be null; in and out
+    double* d;
+    double* e;
+    bse_i4v* msg;        // npos x CHS_SLOT words, zeroed
+    unsigned* meet;      // arrivals (zeroed)
+    int* err;            // 0; 1: a wait was given up; 2: not every workgroup became resident
+};
+// words (16 bytes) of one workgroup's inbox
+#define CHS_V 0                               // 64: v_{k-1} (its unit first entry replaced by tau)
+#define CHS_BETA 64                           // 1: beta_{k+1}
+#define CHS_ROW 65                            // 2 x 64: first row of X_{k+1}
+#define CHS_D 193                             // 2 x 3: D_{k+1}(0,0), y
+#define CHS_SLOT 200
+
+__device__ inline bse_i4v chs_word(double v, int tag) {
+    const bse_i4v w = {__double2loint(v), tag, __double2hiint(v), tag};
+    return w;
+}
+__device__ inline bool chs_here(bse_i4v w, int tag) { return w[1] == tag && w[3] == tag; }
+__device__ inline double chs_value(bse_i4v w) { return __hiloint2double(w[2], w[0]); }
+
+// a + its partner in the other half of the wave, in the same order in both
+__device__ inline double chs_half_sum(double a) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(a), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(a), false, false);
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+// the lower half's value in both halves
+__device__ inline double chs_lower(double a) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(a), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(a), false, false);
+    return __hiloint2double((int)hi[0], (int)lo[0]);
+}
+__device__ inline double2 chs_half_sum2(double2 a) { return cmk(chs_half_sum(a.x), chs_half_sum(a.y)); }
+__device__ inline double2 chs_lower2(double2 a) { return cmk(chs_lower(a.x), chs_lower(a.y)); }
+
+// All workgroups resident?  An arrival adds one; a workgroup that has waited
+// too long sets CHS_ABORT, and only while the count is short (compare and
+// swap), so either every workgroup sees the full count or every one leaves.
+__device__ inline bool chase_meet(unsigned* meet, unsigned npos, int* err) {
+    unsigned v = __hip_atomic_fetch_add(meet, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+    const unsigned long long t0 = wall_clock64();
+    for (;;) {
+        if (v & CHS_ABORT) break;
+        if (v == npos) return true;
+        if (wall_clock64() - t0 > CHS_MEET_TICKS) {
+            unsigned want = v;
+            if (__hip_atomic_compare_exchange_strong(meet, &want, v | CHS_ABORT, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT))
+                break;
+            v = want;
+            continue;
+        }
+        __builtin_amdgcn_s_sleep(4);
+        v = __hip_atomic_load(meet, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __hip_atomic_store(err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return false;
+}
+
+// One failed poll: true when the wait is to be given up.
+__device__ inline bool chs_give_up(unsigned& spins, int* err) {
+    ++spins;
+    if ((spins & 1023u) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return true;
+    if (spins > CHS_SPIN) {
+        __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return true;
+    }
+    return false;
+}
+
+__global__ __launch_bounds__(128, 2) void k_chase_resident(ChaseSysArgs a)
+{
+    // consecutive k on one XCD (workgroups go to the XCDs in turn)
+    const int per = gridDim.x >> 3;
+    const int k = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (k >= a.npos) return;
+    __shared__ double2 sX[CH_B * CHS_LD], sD[CH_B * CHS_LD];
+    __shared__ double2 sVin[CH_B], sS[CH_B];              // wave 0: incoming v, v^H X
+    __shared__ double2 sV[2][CH_B], sTau[2];              // v_k, tau_k by parity of the sweep
+    __shared__ double2 sCol[2][CH_B];                     // first column of D_k by parity
+    __shared__ double2 sR[CH_B], sU[CH_B], sW[2];         // wave 1: entering row, u, (D(0,0), y)
+    __shared__ double2 sY[CH_B];
+    __shared__ int fV, fD, go;
+    const int n = a.n, b = CH_B, ldab = a.ldab;
+    const int lane = threadIdx.x & 63, i = lane & 31, h = lane >> 5;
+    const int base = 1 + k * b;                           // first row of D_k in sweep 0
+    const __amdgpu_buffer_rsrc_t rab = bse_rsrc(a.AB, (int)((int64_t)n * ldab * 16));
+    const __amdgpu_buffer_rsrc_t rin = bse_rsrc(a.msg + (int64_t)k * CHS_SLOT, CHS_SLOT * 16);
+    const __amdgpu_buffer_rsrc_t rright = bse_rsrc(a.msg + (int64_t)min(k + 1, a.npos - 1) * CHS_SLOT, CHS_SLOT * 16);
+    const __amdgpu_buffer_rsrc_t rleft = bse_rsrc(a.msg + (int64_t)max(k - 1, 0) * CHS_SLOT, CHS_SLOT * 16);
+    // sweep 0's blocks: A(r, c) of the band, zero outside it and the matrix
+    auto band = [&](int r, int c) -> double2 {
+        const bool ok = c >= 0 && r < n && r >= c && r - c <= b;
+        return bufld<double2>::ld<0>(rab, ok ? (c * ldab + r - c) * 16 : CH_OOB, 0);
+    };
+    for (int e = threadIdx.x; e < b * b; e += 128) {
+        const int r = e & 31, c = e >> 5;
+        const int at = ((c + 1) & 31) * CHS_LD + ((r + 1) & 31);
+        sX[at] = (k > 0) ? band(base + r, base - b + c) : cmk(0, 0);
+        sD[at] = band(base + r, base + c);               // r >= c only
+    }
+    if (threadIdx.x < b) {
+        // X_k's last column in sweep 0 (k = 0: column 0 of the matrix), as an
+        // entering column: entry r at sCol[1][r + 1], the last one is beta's
+        const int r = threadIdx.x;
+        const double2 x = band(base + r, (k > 0) ? base - 1 : 0);
+        sCol[1][(r + 1) & 31] = x;                       // slot 0: the last entry
+        sY[(r + 1) & 31] = (a.y && base + r < n) ? a.y[base + r] : cmk(0, 0);
+    }
+    if (threadIdx.x == 0) {
+        fV = 0;
+        fD = 0;
+    }
+    double d0 = 0.0;
+    if (k == 0 && threadIdx.x == 0) d0 = band(0, 0).x;
+    __syncthreads();
+    if (threadIdx.x == 0) go = chase_meet(a.meet, (unsigned)a.npos, a.err) ? 1 : 0;
+    __syncthreads();
+    if (!go) return;
+    if (k == 0 && threadIdx.x == 0) a.d[0] = d0;
+    const int last = n - 2 - k * b;                      // last sweep with a row in D_k
+    const int rlast = last - b;                          // ... in D_{k+1}
+    unsigned spins = 0;
+    if (threadIdx.x < 64) {
+        // ------------------------------------------------ wave 0: X_k
+        for (int s = 0; s <= last; ++s) {
+            const int o = (s + 1) & 31, tag = s + 1, par = s & 1;
+            const int pr = (i + o) & 31;
+            const bool right = s <= rlast;               // workgroup k + 1 takes part in this sweep
+            const bool rprev = s > 0 && s - 1 <= rlast;  // ... took part in the previous one
+            double2 xr[16], vc[16];
+            if (k > 0) {
+                // columns 16 h + q < 31 are in LDS whatever the neighbours do
+#pragma unroll
+                for (int q = 0; q < 16; ++q) {
+                    const int pc = (16 * h + q + o) & 31;
+                    xr[q] = sX[pc * CHS_LD + pr];
+                    if (i == 31 && s > 0) xr[q] = cmk(0, 0);
+                }
+            }
+            // v_{k-1}, beta_{k+1} of the previous sweep, the first column of D_k
+            double vw = 0.0, bw = 0.0;
+            for (spins = 0;;) {
+                asm volatile("" ::: "memory");
+                const bse_i4v wv = __builtin_amdgcn_raw_buffer_load_b128(rin, (CHS_V + 2 * i + h) * 16, 0, CH_SC1);
+                const bse_i4v wb = __builtin_amdgcn_raw_buffer_load_b128(rin, CHS_BETA * 16, 0, CH_SC1);
+                const int fd = __hip_atomic_load(&fD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                const bool ok = (k == 0 || chs_here(wv, tag)) && (!rprev || chs_here(wb, s)) && fd >= s;
+                vw = chs_value(wv);
+                bw = rprev ? chs_value(wb) : 0.0;
+                if (__all(ok)) break;
+                if (chs_give_up(spins, a.err)) return;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            const double2 top = sCol[par ^ 1][(i + 1) & 31];         // entry i + 1 of D_k's first column
+            const double2 ent = (i < 31) ? top : (s == 0 ? top : cmk(bw, 0.0));
+            double2 x, tt = cmk(0, 0);
+            if (k > 0) {
+                reinterpret_cast<double*>(sVin)[2 * i + h] = vw;
+                wave_lds_sync();
+                if (h == 1) xr[15] = ent;
+                double2 t0 = cmk(0, 0), t1 = cmk(0, 0);
+#pragma unroll
+                for (int q = 0; q < 16; ++q) vc[q] = sVin[16 * h + q];
+                const double2 tau = sVin[0];
+                if (h == 0) vc[0] = cmk(1.0, 0.0);
+#pragma unroll
+                for (int q = 0; q < 16; q += 2) {
+                    cfma(t0, xr[q], vc[q]);
+                    cfma(t1, xr[q + 1], vc[q + 1]);
+                }
+                tt = cmul(tau, chs_half_sum2(cadd(t0, t1)));
+                xr[0] = csub(xr[0], cmul(tt, cconj(vc[0])));
+                x = chs_lower2(xr[0]);
+            } else {
+                x = ent;
+            }
+            const double ss = wave_sum_dpp((i >= 1 && h == 0) ? cabs2(x) : 0.0);
+            const double2 alpha = cmk(__hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x.x), 0),
+                                                       __builtin_amdgcn_readlane(__double2loint(x.x), 0)),
+                                      __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x.y), 0),
+                                                       __builtin_amdgcn_readlane(__double2loint(x.y), 0)));
+            const Refl r = make_refl(alpha, ss);
+            const double2 v = (i == 0) ? cmk(1.0, 0.0) : cmul(x, r.scal);
+            const double2 out = (i == 0) ? r.tau : v;
+            if (right)
+                __builtin_amdgcn_raw_buffer_store_b128(chs_word(h == 0 ? out.x : out.y, tag), rright,
+                                                       (CHS_V + 2 * i + h) * 16, 0, CH_SC1);
+            if (k > 0 && lane == 0)
+                __builtin_amdgcn_raw_buffer_store_b128(chs_word(r.beta, tag), rleft, CHS_BETA * 16, 0, CH_SC1);
+            if (k == 0 && lane == 0) a.e[s] = r.beta;
+            if (h == 0) sV[par][i] = v;
+            if (lane == 0) sTau[par] = r.tau;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            if (lane == 0) __hip_atomic_store(&fV, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (k == 0) continue;
+            // the other columns of X H_{k-1}
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                if (q > 0) xr[q] = csub(xr[q], cmul(tt, cconj(vc[q])));
+                sX[((16 * h + q + o) & 31) * CHS_LD + pr] = xr[q];
+            }
+            wave_lds_sync();
+            // v^H X: lane (h, i) sums rows 16 h .. 16 h + 15 of column i
+            double2 s0 = cmk(0, 0), s1 = cmk(0, 0);
+#pragma unroll
+            for (int q = 0; q < 16; q += 2) {
+                const int r0 = 16 * h + q;
+                cfmac(s0, sV[par][r0], sX[pr * CHS_LD + ((r0 + o) & 31)]);
+                cfmac(s1, sV[par][r0 + 1], sX[pr * CHS_LD + ((r0 + 1 + o) & 31)]);
+            }
+            const double2 sc = chs_half_sum2(cadd(s0, s1));
+            if (h == 0) sS[i] = sc;
+            wave_lds_sync();
+            const double2 f = cmul(cconj(r.tau), v);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const double2 xn = csub(xr[q], cmul(f, sS[16 * h + q]));
+                xr[q] = (q == 0 && h == 0) ? ((i == 0) ? cmk(r.beta, 0.0) : cmk(0, 0)) : xn;
+                sX[((16 * h + q + o) & 31) * CHS_LD + pr] = xr[q];
+            }
+            wave_lds_sync();
+            // the first row to the left: word 2 c + (real, imaginary)
+            {
+                const double2 rw = sX[(((lane >> 1) + o) & 31) * CHS_LD + o];
+                __builtin_amdgcn_raw_buffer_store_b128(chs_word((lane & 1) ? rw.y : rw.x, tag), rleft,
+                                                       (CHS_ROW + 64 * par + lane) * 16, 0, CH_SC1);
+            }
+        }
+    } else {
+        // ------------------------------------------------ wave 1: D_k and y
+        for (int s = 0; s <= last; ++s) {
+            const int o = (s + 1) & 31, tag = s + 1, par = s & 1;
+            const int pr = (i + o) & 31;
+            const bool rprev = s > 0 && s - 1 <= rlast;
+            // the entering row (sweep s - 1 of workgroup k + 1) and v_k
+            double rw = 0.0, dw = 0.0;
+            for (spins = 0;;) {
+                asm volatile("" ::: "memory");
+                const bse_i4v w0 = __builtin_amdgcn_raw_buffer_load_b128(rin, (CHS_ROW + 64 * (par ^ 1) + lane) * 16, 0,
+                                                                         CH_SC1);
+                const bse_i4v w1 = __builtin_amdgcn_raw_buffer_load_b128(
+                    rin, (CHS_D + 3 * (par ^ 1) + min(lane, 2)) * 16, 0, CH_SC1);
+                const int fv = __hip_atomic_load(&fV, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                const bool ok = (!rprev || (chs_here(w0, s) && chs_here(w1, s))) && fv >= tag;
+                rw = rprev ? chs_value(w0) : 0.0;
+                dw = rprev ? chs_value(w1) : 0.0;
+                if (__all(ok)) break;
+                if (chs_give_up(spins, a.err)) return;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            reinterpret_cast<double*>(sR)[lane] = rw;
+            if (lane < 3) reinterpret_cast<double*>(sW)[lane == 0 ? 0 : lane + 1] = dw;   // sW = (D(0,0), -), y
+            wave_lds_sync();
+            const double2 v = sV[par][i], tau = sTau[par];
+            // row i of D_k: the lower triangle as stored, the upper one from it;
+            // row and column 31 are the entering ones (all of them in LDS in sweep 0)
+            double2 t[16];
+            double2 w0 = cmk(0, 0), w1 = cmk(0, 0);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int c = 16 * h + q, pc = (c + o) & 31;
+                const bool low = i >= c;
+                double2 z = low ? sD[pc * CHS_LD + pr] : sD[pr * CHS_LD + pc];
+                if (s > 0 && (i == 31 || c == 31)) {
+                    const int m = (i == 31) ? c : i;                 // the other index
+                    z = (m == 31) ? cmk(sW[0].x, 0.0) : sR[(m + 1) & 31];
+                }
+                if (!low) z.y = -z.y;
+                t[q] = z;
+                if (q & 1) cfma(w1, z, sV[par][c]);
+                else cfma(w0, z, sV[par][c]);
+            }
+            const double2 wv = chs_half_sum2(cadd(w0, w1));
+            const double2 yy = (i == 31 && s > 0) ? sW[1] : sY[pr];
+            const double gam = wave_sum_dpp(h == 0 ? v.x * wv.x + v.y * wv.y : 0.0);
+            const double2 dot = wave_sum_c(h == 0 ? cmul(cconj(v), yy) : cmk(0, 0));
+            const double2 u = csub(cmul(tau, wv), cscale(v, 0.5 * cabs2(tau) * gam));
+            const double2 yn = csub(yy, cmul(cmul(cconj(tau), v), dot));
+            if (h == 0) {
+                sU[i] = u;
+                sY[pr] = yn;
+            }
+            wave_lds_sync();
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int c = 16 * h + q, pc = (c + o) & 31;
+                double2 z = csub(t[q], cadd(cmul(u, cconj(sV[par][c])), cmul(v, cconj(sU[c]))));
+                if (i == c) z.y = 0.0;
+                if (i >= c) sD[pc * CHS_LD + pr] = z;
+                if (q == 0) {
+                    // the first column is wave 0's entering column, D(0,0) and
+                    // y's first entry go to the left (or are final)
+                    if (h == 0) sCol[par][i] = z;
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+                    if (lane == 0) __hip_atomic_store(&fD, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    if (k > 0) {
+                        // lanes 0..2 of row 0 .. 2: broadcast row 0's values first
+                        const double z0 = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(z.x), 0),
+                                                           __builtin_amdgcn_readlane(__double2loint(z.x), 0));
+                        const double y0 = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(yn.x), 0),
+                                                           __builtin_amdgcn_readlane(__double2loint(yn.x), 0));
+                        const double y1 = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(yn.y), 0),
+                                                           __builtin_amdgcn_readlane(__double2loint(yn.y), 0));
+                        if (lane < 3)
+                            __builtin_amdgcn_raw_buffer_store_b128(chs_word(lane == 0 ? z0 : (lane == 1 ? y0 : y1), tag),
+                                                                   rleft, (CHS_D + 3 * par + lane) * 16, 0, CH_SC1);
+                    } else if (lane == 0) {
+                        a.d[s + 1] = z.x;
+                        if (a.y) a.y[s + 1] = yn;
+                    }
+                }
+            }
+            wave_lds_sync();
+        }
+    }
+}
+
+// Workgroups of the resident form, 0 when it does not apply (another
+// half-bandwidth, or more workgroups than the device holds at once).
+static int chase_resident_grid(int n, int b, int ldab, int device)
+{
+    if (b != CH_B || n < 2 || (int64_t)n * ldab * 16 >= ((int64_t)1 << 31)) return 0;
+    const int npos = (n - 2) / CH_B + 1;
+    const int grid = 8 * (int)ceil_div64(npos, 8);
+    int per_cu = 0, ncu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_chase_resident, 128, 0) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+        return 0;
+    return (int64_t)grid <= (int64_t)per_cu * ncu ? grid : 0;
+}
+
+// 16-byte words of the messages and the meeting counter.
+extern "C" int64_t bse_chase_resident_workspace(int n, int b, int ldab, int device)
+{
+    if (chase_resident_grid(n, b, ldab, device) == 0) return 0;
+    return (int64_t)((n - 2) / CH_B + 1) * CHS_SLOT + 1;
+}
+
+// Two of these kernels at once could each hold half of the device and wait
+// for the rest, so the launches on one device follow one another: each waits
+// for the event of the one before.
+struct ChaseQueue {
+    std::mutex m;
+    hipEvent_t done = nullptr;
+};
+static ChaseQueue& chase_queue(int device)
+{
+    static ChaseQueue q[64];
+    return q[device & 63];
+}
+
+// err receives 0, 1 (a wait was given up) or 2 (the workgroups did not become
+// resident together: AB, y, d and e are as they were).
+extern "C" hipError_t bse_launch_chase_resident(hipStream_t st, int device, int n, int b, const double2* AB,
+                                                int ldab, double2* y, double* d, double* e, double2* ws, int* err)
+{
+    const int grid = chase_resident_grid(n, b, ldab, device);
+    if (grid == 0) return hipErrorInvalidValue;
+    const int npos = (n - 2) / CH_B + 1;
+    const int64_t words = (int64_t)npos * CHS_SLOT;
+    hipError_t rc = bse_launch_zero_words(st, 2 * (words + 1), ws);
+    if (rc != hipSuccess) return rc;
+    const ChaseSysArgs args{n, ldab, npos, AB, y, d, e, reinterpret_cast<bse_i4v*>(ws),
+                            reinterpret_cast<unsigned*>(ws + words), err};
+    ChaseQueue& q = chase_queue(device);
+    const std::lock_guard<std::mutex> lock(q.m);
+    if (!q.done) {
+        rc = hipEventCreateWithFlags(&q.done, hipEventDisableTiming);
+        if (rc != hipSuccess) return rc;
+    } else {
+        rc = hipStreamWaitEvent(st, q.done, 0);
+        if (rc != hipSuccess) return rc;
+    }
+    hipLaunchKernelGGL(k_chase_resident, dim3((unsigned)grid), dim3(128), 0, st, args);
+    rc = hipGetLastError();
+    return rc == hipSuccess ? hipEventRecord(q.done, st) : rc;
 }
 
 extern "C" int64_t bse_chase_counters(int n) { return n > 1 ? n - 1 : 1; }
