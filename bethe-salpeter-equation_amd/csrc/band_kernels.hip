@@ -407,8 +407,7 @@ __device__ inline void lds_unit_lower_inv(hh_sq& L, hh_sq& X, int k)
 }
 // The LU runs in place in W: the multipliers (L1 below the unit diagonal)
 // replace W's strict lower part, U (diagonal u_jj, upper -d_c W(j, c)) its
-// upper part, so W, Ui and Li are the only LDS matrices (the kernels that
-// call this fit beside a running trailing update).
+// upper part.
 __device__ __attribute__((always_inline)) inline void hh_reconstruct_lds(
     int m, int b, int k, hh_sq& W, hh_sq& Ui, hh_sq& Li, double2* d, double2* ud,
     const double2* __restrict__ Rfin, double2* __restrict__ V, double2* __restrict__ Tp,
@@ -596,160 +595,279 @@ __global__ __launch_bounds__(256) void k_cq_reduce(int ng, const double2* __rest
     G[e] = acc;
 }
 
-// The Gram matrix G (Gp, summed by k_cq_reduce) into sG, then its Cholesky
-// factor in place (lower triangle).
-// pass 1 also checks |G - I| <= 0.1.  Returns false (uniformly) on failure.
-__device__ bool cq_sum_chol(int ng, const double2* __restrict__ Gp, int pass, hh_sq& sG, double* diag0,
-                            int* fl)
+// The 32 x 32 factorisations below keep the matrix in registers, thread
+// (g, i) = (tid / 32, tid % 32) holding row i, columns 4 g .. 4 g + 3, and
+// eliminate it by 32 rank-one steps.  A step publishes its pivot column and
+// row in LDS, takes one workgroup barrier, and updates all 32 x 32 entries:
+// the trailing block, and in the columns already eliminated (whose entries
+// are no longer needed) the inverse of the factor, which obeys the same
+// recurrence.  So a factor and its inverse cost 32 short steps instead of the
+// 32 three-barrier steps and 32 dependent LDS rows of a factorisation
+// followed by a triangular inverse.  One workgroup, bound by the latency of
+// the steps: the two kernels of a panel took 70 + 152 us that way and take
+// 17 + 45 us now (N = 4624; half of the second kernel is its four
+// 32 x 32 products and their loads).
+
+// 1/x and 1/sqrt(x) of a positive normal x: the hardware estimates (about
+// 2^-24) and two Newton steps each, which end within 1-2 ulp; the compiler's
+// exactly rounded division and square root have about twice the dependent
+// latency, which every step of the factorisations below would wait for.
+__device__ inline double cq_rcp(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.0), r);
+    return fma(r, fma(-x, r, 1.0), r);
+}
+__device__ inline double cq_rsq(double x) {
+    double r = __builtin_amdgcn_rsq(x);
+    r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
+    return fma(0.5 * r, fma(-x * r, r, 1.0), r);
+}
+
+// c ? a : b on the components (a conditional on the vectors themselves selects
+// between their addresses and puts both in scratch memory).
+__device__ inline double2 csel(bool c, double2 a, double2 b) { return cmk(c ? a.x : b.x, c ? a.y : b.y); }
+
+// G (e = i + 32 c in Gs, summed by k_cq_reduce) = L L^H.  L is left in sL
+// (lower triangle, zeros above), L^{-1} in a (row i, columns 4 g ..; zeros
+// above the diagonal).  With near_one it also checks |G - I| <= 0.1.
+// Returns false (uniformly) when G is not numerically positive definite.
+__device__ inline bool cq_factor(const double2* __restrict__ Gs, bool near_one, hh_sq& sL, double2 (&sRow)[2][BR_B],
+                                 double* diag0, double* rs, int* fl, double2 (&a)[4])
 {
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, i = tid & 31, g = tid >> 5;
+    bool ok = true;
     if (tid == 0) *fl = 0;
-    // G summed by k_cq_reduce (ng = 1: Gp is G itself)
-    (void)ng;
+    __syncthreads();
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int e = tid + 256 * u, i = e % BR_B, j = e / BR_B;
-        const double2 x = Gp[e];
-        sG[i][j] = x;
-        if (i == j) diag0[i] = x.x;
+    for (int q = 0; q < 4; ++q) {
+        const int c = 4 * g + q;
+        const double2 x = Gs[i + BR_B * c];
+        a[q] = x;
+        if (i == c) diag0[i] = x.x;
+        if (near_one && !(fabs(x.x - (i == c ? 1.0 : 0.0)) <= 0.1 && fabs(x.y) <= 0.1)) *fl = 1;
+    }
+    // not unrolled: straight-line code runs once and would wait for the
+    // instruction cache at every line
+#pragma unroll 1
+    for (int jb = 0; jb < BR_B / 4; ++jb) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int j = 4 * jb + u;
+            if (g == jb) sL[i][j] = a[u];
+            if (i == j) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) sRow[j & 1][4 * g + q] = a[q];
+            }
+            __syncthreads();
+            // every LDS read of the step is issued before the first is used
+            const double d = sL[j][j].x;
+            const double2 col = sL[i][j];
+            const double top = diag0[j];
+            double2 pr[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) pr[q] = sRow[j & 1][4 * g + q];
+            // a zero or lost pivot: the result is dropped at the end
+            ok = ok && d > 1e-12 * top && top > 0.0;
+            const double2 m = cscale(col, cq_rcp(d));
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int c = 4 * g + q;
+                const double2 p = pr[q];
+                const double2 z = csel(c == j, cmk(-m.x, -m.y), csub(a[q], cmul(m, p)));
+                a[q] = csel(i > j, z, csel(i == j && c == j, cmk(1.0, 0.0), a[q]));
+            }
+        }
+    }
+    if (tid < BR_B) rs[tid] = 1.0 / sqrt(sL[tid][tid].x);
+    __syncthreads();
+    if (!ok || *fl) return false;                    // LDS values only: uniform
+    // the published columns hold L D: scale; rows of L^{-1} likewise
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int c = 4 * g + q;
+        sL[i][c] = cscale(sL[i][c], (i >= c) ? rs[c] : 0.0);
+        a[q] = cscale(a[q], (i >= c) ? rs[i] : 0.0);
     }
     __syncthreads();
-    if (pass == 1) {
-        for (int e = tid; e < BR_B * BR_B; e += 256) {
-            const int i = e % BR_B, j = e / BR_B;
-            const double2 x = csub(sG[i][j], cmk(i == j ? 1.0 : 0.0, 0.0));
-            if (!(fabs(x.x) <= 0.1 && fabs(x.y) <= 0.1)) *fl = 1;
-        }
-        __syncthreads();
-    }
-    // right-looking Cholesky, the trailing update spread over the workgroup
-    for (int j = 0; j < BR_B; ++j) {
-        if (*fl) break;                                   // uniform
-        const double dj = sG[j][j].x;
-        if (!(dj > 1e-12 * diag0[j] && diag0[j] > 0.0)) {
-            __syncthreads();
-            if (tid == 0) *fl = 1;
-            __syncthreads();
-            break;
-        }
-        const double ljj = sqrt(dj);
-        __syncthreads();                                  // every thread has read sG[j][j]
-        if (tid > j && tid < BR_B) sG[tid][j] = cscale(sG[tid][j], 1.0 / ljj);
-        if (tid == j) sG[j][j] = cmk(ljj, 0.0);
-        __syncthreads();
-        for (int e = tid; e < BR_B * BR_B; e += 256) {
-            const int i = e % BR_B, c = e / BR_B;
-            if (c > j && i >= c) sG[i][c] = csub(sG[i][c], cmul(sG[i][j], cconj(sG[c][j])));
-        }
-        __syncthreads();
-    }
-    __syncthreads();
-    return *fl == 0;
+    return true;
 }
 
-// Ri = R^{-1} for R = L^H (L lower in sL).
-__device__ void cq_rinv(hh_sq& sL, hh_sq& Ri)
+// First factorisation: R1 = L^H (upper, ld b) and R1^{-1} to global.
+__global__ __launch_bounds__(256) void k_cq_chol1(const double2* __restrict__ Gs, double2* __restrict__ R1,
+                                                  double2* __restrict__ R1i, int* __restrict__ flag,
+                                                  int* __restrict__ fail)
 {
-    if (threadIdx.x < 64) lds_upper_inv(sL, true, Ri, BR_B);
-    __syncthreads();
-}
-
-// First factorisation: R1 (upper, ld b) and R1^{-1} to global.
-__global__ __launch_bounds__(256) void k_cq_chol1(int ng, const double2* __restrict__ Gp,
-                                                  double2* __restrict__ R1, double2* __restrict__ R1i,
-                                                  int* __restrict__ flag, int* __restrict__ fail)
-{
-    __shared__ hh_sq sG, Ri;
-    __shared__ double diag0[BR_B];
+    __shared__ hh_sq sL;
+    __shared__ double2 sRow[2][BR_B];
+    __shared__ double diag0[BR_B], rs[BR_B];
     __shared__ int fl;
-    if (!cq_sum_chol(ng, Gp, 0, sG, diag0, &fl)) {
+    double2 a[4];
+    if (!cq_factor(Gs, false, sL, sRow, diag0, rs, &fl, a)) {
         if (threadIdx.x == 0) {
             flag[0] = 1;
             *fail = 1;
         }
         return;
     }
-    cq_rinv(sG, Ri);
-    for (int e = threadIdx.x; e < BR_B * BR_B; e += 256) {
-        const int i = e % BR_B, j = e / BR_B;
-        R1[e] = (i <= j) ? cconj(sG[j][i]) : cmk(0, 0);
-        R1i[e] = Ri[i][j];
+    const int i = threadIdx.x & 31, g = threadIdx.x >> 5;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int c = 4 * g + q;
+        R1[i + BR_B * c] = cconj(sL[c][i]);
+        R1i[c + BR_B * i] = cconj(a[q]);
     }
     if (threadIdx.x == 0) flag[1] = 1;
 }
 
-// Second factorisation and the Householder form: R = R2 R1 -> Rf; the top
-// block W = Q1(0:32, :) R2^{-1}; hh_reconstruct_lds; Mp = R2^{-1} Mlow for
-// the rows below (V = Q1 Mp there).  Nothing is written when it fails.
-__global__ __launch_bounds__(256) void k_cq_chol2(int m, int b, int ng, const double2* __restrict__ Gp,
+// Second factorisation and the Householder form.  R = R2 R1; W = Q1(0:32, :)
+// R2^{-1} is the top block of Q.  LU of E - Q D, d_j = -conj(w_j)/|w_j| from the
+// running Schur entry w_j (Ballard et al. 2014): u_jj = 1 + |w_j|, U(j, c) =
+// -d_c W(j, c), multipliers -d_j W(i, j) / u_jj.  With What = U (-D)^{-1} (row
+// j of W, diagonal -u_jj / d_j), -D U^{-1} = What^{-1}, whose column j is known
+// at step j: x = d_j S(:, j) / u_jj with S = What^{-1} What accumulated from the
+// same pivot rows.  Step j therefore is, with f_i = d_j W(i, j) / u_jj (rows
+// above j: S(i, j)) and f_j = -d_j / u_jj,
+//   a(i, c) += f_i W(j, c)   (c > j; also c < j in the rows below j)
+//   a(j, c)  = f_j W(j, c)   (c > j),   a(:, j) = f,
+// and leaves L1^{-1} below the diagonal and What^{-1} on and above it.
+// Out: V rows 0 .. 31 = L1; T = U L1^{-H}; Mp = R2^{-1} What^{-1} (V = Q1 Mp below);
+// R' = D^H R into the band store.  Nothing is written when it fails.
+__global__ __launch_bounds__(256) void k_cq_chol2(int m, int b, const double2* __restrict__ Gs,
                                                   const double2* __restrict__ Q1, const double2* __restrict__ R1,
-                                                  double2* __restrict__ Rf, double2* __restrict__ V,
-                                                  double2* __restrict__ Tp, double2* __restrict__ Mp,
-                                                  double2* __restrict__ AB, int ldab, int c0,
-                                                  int* __restrict__ flag, int* __restrict__ fail)
+                                                  double2* __restrict__ V, double2* __restrict__ Tp,
+                                                  double2* __restrict__ Mp, double2* __restrict__ AB, int ldab,
+                                                  int c0, int* __restrict__ flag, int* __restrict__ fail)
 {
-    __shared__ hh_sq W, Ui, Li;
-    __shared__ double2 d[BR_B], ud[BR_B];
-    __shared__ double diag0[BR_B];
+    __shared__ hh_sq sL, sRi, sW, sC;
+    __shared__ double2 sRow[2][BR_B], sd[BR_B];
+    __shared__ double diag0[BR_B], rs[BR_B], su[BR_B];
     __shared__ int fl;
     if (flag[1] == 0) return;
-    // Cholesky of G2 in W, R2^{-1} in Li
-    if (!cq_sum_chol(ng, Gp, 1, W, diag0, &fl)) {
-        if (threadIdx.x == 0) {
+    const int tid = threadIdx.x, i = tid & 31, g = tid >> 5;
+    double2 q1[4], r1[4], a[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        q1[q] = Q1[i + (int64_t)(4 * g + q) * m];
+        r1[q] = R1[i + BR_B * (4 * g + q)];
+    }
+    if (!cq_factor(Gs, true, sL, sRow, diag0, rs, &fl, a)) {
+        if (tid == 0) {
             flag[0] = 1;
             *fail = 1;
         }
         return;
     }
-    cq_rinv(W, Li);
-    for (int e = threadIdx.x; e < BR_B * BR_B; e += 256) Ui[e % BR_B][e / BR_B] = R1[e];
-    __syncthreads();
-    // R = R2 R1 (both upper; R2(i, l) = conj(W(l, i))) into Rf
-    for (int e = threadIdx.x; e < BR_B * BR_B; e += 256) {
-        const int i = e % BR_B, j = e / BR_B;
-        double2 s = cmk(0, 0);
-        for (int l = i; l <= j; ++l) cfma(s, cconj(W[l][i]), Ui[l][j]);
-        Rf[e] = (i <= j) ? s : cmk(0, 0);
-    }
-    __syncthreads();
-    // the top 32 x 32 block of Q1 into Ui, then the top block of
-    // Q = Q1 R2^{-1} into W; R2^{-1} is kept in registers (4 entries per
-    // thread) while the reconstruction uses Li
-    for (int e = threadIdx.x; e < BR_B * BR_B; e += 256) {
-        const int i = e % BR_B, j = e / BR_B;
-        Ui[i][j] = Q1[i + (int64_t)j * m];
-    }
-    __syncthreads();
-    double2 r2i[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int e = threadIdx.x + 256 * u, i = e % BR_B, j = e / BR_B;
-        double2 t = cmk(0, 0);
-        for (int l = 0; l <= j; ++l) cfma(t, Ui[i][l], Li[l][j]);
-        W[i][j] = t;
-        r2i[u] = Li[i][j];
+    for (int q = 0; q < 4; ++q) {
+        const int c = 4 * g + q;
+        sRi[c][i] = cconj(a[q]);                     // R2^{-1}
+        sW[i][c] = q1[q];
     }
     __syncthreads();
-    hh_reconstruct_lds(m, b, BR_B, W, Ui, Li, d, ud, Rf, V, Tp, nullptr, AB, ldab, c0);
+    // the top block of Q, rows of Q1 times R2^{-1} (upper triangular)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) a[q] = cmk(0, 0);
+#pragma unroll 1
+    for (int l = 0; l < 4 * g + 4; ++l) {
+        const double2 x = sW[i][l];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) cfma(a[q], x, sRi[l][4 * g + q]);
+    }
     __syncthreads();
-    // Mlow = -D U^{-1} into W, R2^{-1} back into Li, then Mp = R2^{-1} Mlow
-    for (int e = threadIdx.x; e < BR_B * BR_B; e += 256) {
-        const int i = e % BR_B, j = e / BR_B;
-        W[i][j] = cmul(cmk(-d[i].x, -d[i].y), Ui[i][j]);
+    // not unrolled: straight-line code runs once and would wait for the
+    // instruction cache at every line
+#pragma unroll 1
+    for (int jb = 0; jb < BR_B / 4; ++jb) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int j = 4 * jb + u;
+            if (g == jb) sC[i][j] = a[u];
+            if (i == j) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) sW[j][4 * g + q] = a[q];
+            }
+            __syncthreads();
+            const double2 wj = sC[j][j], col = sC[i][j];
+            double2 pr[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) pr[q] = sW[j][4 * g + q];
+            // d_j / u_jj = -conj(w) / (|w| + |w|^2); a |w| below 1e-140 (whose
+            // square would underflow) counts as zero: d_j = u_jj = 1
+            const double a2 = cabs2(wj);
+            const double2 sc = csel(a2 > 1e-280, cscale(cmk(-wj.x, wj.y), cq_rcp(fma(a2, cq_rsq(a2), a2))), cmk(1.0, 0.0));
+            const double2 f = csel(i == j, cmk(-sc.x, -sc.y), cmul(sc, col));
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int c = 4 * g + q;
+                const double2 p = pr[q];
+                double2 z = csel(i == j, cmk(0, 0), a[q]);
+                cfma(z, f, p);
+                a[q] = csel(c == j, f, csel(c > j || i > j, z, a[q]));
+            }
+        }
+    }
+    __syncthreads();
+    if (tid < BR_B) {
+        const double2 w = sC[tid][tid];
+        const double a2 = cabs2(w), aw = sqrt(a2);
+        sd[tid] = csel(a2 > 1e-280, cmk(-w.x / aw, w.y / aw), cmk(1.0, 0.0));
+        su[tid] = (a2 > 1e-280) ? 1.0 + aw : 1.0;
+    }
+    __syncthreads();
+    // V's top rows: multipliers -d_c W(i, c) / u_cc from the published columns
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int c = 4 * g + q;
+        V[i + (int64_t)c * m] = csel(i > c, cscale(cmul(sd[c], sC[i][c]), -1.0 / su[c]), cmk(i == c ? 1.0 : 0.0, 0.0));
+    }
+    __syncthreads();
+    // U into sW; L1^{-1} strictly below, What^{-1} on and above the diagonal of sC
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int c = 4 * g + q;
+        const double2 w = sW[i][c];
+        sW[i][c] = csel(c > i, cmul(cmk(-sd[c].x, -sd[c].y), w), cmk(c == i ? su[i] : 0.0, 0.0));
+        sC[i][c] = a[q];
+    }
+    __syncthreads();
+    double2 t[4], mp[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) t[q] = mp[q] = cmk(0, 0);
+#pragma unroll 1
+    for (int l = 0; l < 4 * g + 4; ++l) {
+        const double2 u = sW[i][l], r = sRi[i][l];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int c = 4 * g + q;
+            const double2 li = csel(l < c, sC[c][l], cmk(l == c ? 1.0 : 0.0, 0.0));
+            cfma(t[q], u, cconj(li));
+            cfma(mp[q], r, csel(l <= c, sC[l][c], cmk(0, 0)));
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int c = 4 * g + q;
+        Tp[i + c * b] = csel(i <= c, t[q], cmk(0, 0));
+        Mp[i + c * b] = csel(i <= c, mp[q], cmk(0, 0));
+        sW[i][c] = r1[q];
+    }
+    __syncthreads();
+    // R' = D^H R2 R1: rows s .. s + 31 of columns c0 .. c0 + 31
+#pragma unroll
+    for (int q = 0; q < 4; ++q) t[q] = cmk(0, 0);
+#pragma unroll 1
+    for (int l = 0; l < 4 * g + 4; ++l) {
+        const double2 x = cconj(sL[l][i]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) cfma(t[q], x, sW[l][4 * g + q]);
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int e = threadIdx.x + 256 * u;
-        Li[e % BR_B][e / BR_B] = r2i[u];
+    for (int q = 0; q < 4; ++q) {
+        const int c = 4 * g + q, gr = c0 + b + i, gc = c0 + c;
+        AB[(int64_t)gc * ldab + (gr - gc)] = csel(i <= c, cmul(cconj(sd[i]), t[q]), cmk(0, 0));
     }
-    __syncthreads();
-    for (int e = threadIdx.x; e < BR_B * BR_B; e += 256) {
-        const int i = e % BR_B, j = e / BR_B;
-        double2 s = cmk(0, 0);
-        for (int l = i; l < BR_B; ++l) cfma(s, Li[i][l], W[l][j]);
-        Mp[i + j * b] = s;
-    }
-    if (threadIdx.x == 0) flag[2] = 1;
+    if (tid == 0) flag[2] = 1;
 }
 
 // ---------------------------------------------------------------------------
@@ -1114,7 +1232,7 @@ extern "C" hipError_t bse_band_gather_tail(hipStream_t st, int fp32, int n, int 
 
 // Workspace of one panel QR of an m-row panel (complex elements): leaf R and
 // tau, tree levels (V, tau, R per node; X pieces), the thin Q, then the
-// CholeskyQR2 partial Gram matrices, R1, R1^{-1}, R, Mp and two flags.
+// CholeskyQR2 partial Gram matrices, R1, R1^{-1}, Mp and three flags.
 extern "C" int64_t bse_tsqr_workspace(int m, int b) {
     int64_t el = 0;
     int nin = tsqr_nblk(m);
@@ -1126,7 +1244,7 @@ extern "C" int64_t bse_tsqr_workspace(int m, int b) {
         nin = nn;
     }
     el += (int64_t)m * b;                                 // Q_thin (Q1 on the fast path)
-    el += (int64_t)CQ_G * BR_B * BR_B + 4 * BR_B * BR_B + 1;
+    el += (int64_t)CQ_G * BR_B * BR_B + 3 * BR_B * BR_B + 1;
     return el + 64;
 }
 
@@ -1184,7 +1302,6 @@ extern "C" hipError_t bse_band_panel_qr(hipStream_t st, int m, int b, double2* P
     double2* Gp = p; p += (int64_t)CQ_G * BR_B * BR_B;
     double2* R1 = p; p += BR_B * BR_B;
     double2* R1i = p; p += BR_B * BR_B;
-    double2* Rf = p; p += BR_B * BR_B;
     double2* Mp = p; p += BR_B * BR_B;
     int* flags = reinterpret_cast<int*>(p);     // [0]: TSQR needed, [1], [2]: factorisations done
     const bool fast = (b == BR_B && m >= 2 * BR_B);
@@ -1195,14 +1312,14 @@ extern "C" hipError_t bse_band_panel_qr(hipStream_t st, int m, int b, double2* P
         hipLaunchKernelGGL(k_cq_gram<0>, dim3((unsigned)g), dim3(256), 0, st, m, (const double2*)P, Gp, flags);
         hipLaunchKernelGGL(k_cq_reduce, dim3(BR_B * BR_B / 256), dim3(256), 0, st, g, (const double2*)Gp, Gs,
                            (const int*)flags, -1);
-        hipLaunchKernelGGL(k_cq_chol1, dim3(1), dim3(256), 0, st, 1, (const double2*)Gs, R1, R1i, flags, fail);
+        hipLaunchKernelGGL(k_cq_chol1, dim3(1), dim3(256), 0, st, (const double2*)Gs, R1, R1i, flags, fail);
         hipLaunchKernelGGL(k_rows_small, dim3((unsigned)ceil_div64(m, 64)), dim3(256), 0, st, m, 0, BR_B, BR_B, BR_B,
                            (const double2*)P, (const double2*)R1i, Q, 0, (const int*)(flags + 1));
         hipLaunchKernelGGL(k_cq_gram<1>, dim3((unsigned)g), dim3(256), 0, st, m, (const double2*)Q, Gp, flags);
         hipLaunchKernelGGL(k_cq_reduce, dim3(BR_B * BR_B / 256), dim3(256), 0, st, g, (const double2*)Gp, Gs,
                            (const int*)flags, 1);
-        hipLaunchKernelGGL(k_cq_chol2, dim3(1), dim3(256), 0, st, m, b, 1, (const double2*)Gs,
-                           (const double2*)Q, (const double2*)R1, Rf, Vout, Tp, Mp, AB, ldab, c0, flags, fail);
+        hipLaunchKernelGGL(k_cq_chol2, dim3(1), dim3(256), 0, st, m, b, (const double2*)Gs, (const double2*)Q,
+                           (const double2*)R1, Vout, Tp, Mp, AB, ldab, c0, flags, fail);
         hipLaunchKernelGGL(k_rows_small, dim3((unsigned)ceil_div64(m - k, 64)), dim3(256), 0, st, m, k, BR_B, k, b,
                            (const double2*)Q, (const double2*)Mp, Vout, 0, (const int*)(flags + 2));
         gate = flags;
