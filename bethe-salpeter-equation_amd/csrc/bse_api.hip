@@ -554,7 +554,7 @@ static int64_t hemv_partials(int code, int n, int s0) {
 // them makes the column step's reduce slower).
 // ---------------------------------------------------------------------------
 int autotune_hemv(bse_ctx* ctx, int fp32, int n, const void* H, double2* v, double2* Yr,
-                  double2* Yc) {
+                  double2* Yc, int min_nt) {
     unsigned char* tab = ctx->hemv_ch[fp32];
     // BSE_HEMV_CODE=<code> pins one variant for every trailing size (for
     // measurements of a single variant)
@@ -567,7 +567,7 @@ int autotune_hemv(bse_ctx* ctx, int fp32, int n, const void* H, double2* v, doub
     hipStream_t st = ctx->st;
     bool zeroed = false;
     for (int b = 6; b < BSE_HEMV_BUCKETS && (1 << b) <= n - 1; ++b) {
-        if (tab[b] != 0) continue;
+        if (tab[b] != 0 || (2 << b) <= min_nt) continue;
         if (!zeroed) {
             HCK(hipMemsetAsync(v, 0, sizeof(double2) * n, st));
             zeroed = true;
@@ -1036,8 +1036,27 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     Tall = BUF(double2, S_TALL, (size_t)std::max(npan, 1) * nb * nb);
     double2* Gram = BUF(double2, S_GRAM, (size_t)std::max(npan, 1) * 64 * 64);   // one block per panel
     double2* alpha2 = BUF(double2, S_ALPHA2, 64);
+    // panels that run in one launch each (BSE_TRD_PANEL=0, and a pinned hemv
+    // variant, keep the per-column launches); the matrix is kept, so that the
+    // reduction can be repeated without them should the device not hold all
+    // their workgroups at once
+    const char* pne = getenv("BSE_TRD_PANEL");
+    const int pnwg = ((pne && pne[0] == '0') || getenv("BSE_HEMV_CODE")) ? 0 : bse_panel_workgroups(ctx->device, fp32);
+    PanelRun prun{ctx->device, n, pnwg, nullptr, pnwg > 0 ? bse_panel_workspace(n, pnwg) : 0, nullptr};
+    const size_t hbytes = (size_t)tiled_elems(n) * (fp32 ? sizeof(float2) : sizeof(double2));
+    void* H0 = nullptr;
+    if (prun.ws_el > 0) {
+        prun.first = bse_panel_first(n, pnwg);
+        prun.ws = BUF(double2, S_PNMSG, prun.ws_el);
+        prun.err = BUF(int, S_PNERR, 4);
+        H0 = BUF(char, S_BH0, hbytes);
+        HCK(bse_launch_zero_words(st, 2 * prun.ws_el, prun.ws));
+        HCK(bse_launch_zero_words(st, 2, prun.err));
+        HCK(hipMemcpyAsync(H0, H, hbytes, hipMemcpyDeviceToDevice, st));
+    }
+    const int panel_first = prun.ws_el > 0 ? prun.first : n;
     {
-        int rc = autotune_hemv(ctx, fp32, n, H, acol, Yr, Yc);
+        int rc = autotune_hemv(ctx, fp32, n, H, acol, Yr, Yc, n - panel_first);
         if (rc) return rc;
         rc = autotune_her2k(ctx, fp32, Yr, sizeof(double2) * (size_t)yr_el, Vst, Wp,
                             std::min<int64_t>(vs_el, (int64_t)n * nb), alpha2);
@@ -1046,12 +1065,26 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     double* hsys = BUF(double, S_HSYS, 32);   // one HetrdSys (device copy)
     HCK(bse_hetrd(st, fp32, n, H, nb, d, e, tauh, Vst, Tall, Wp, alpha2, Gram, acol, Yr, Yc, t12,
                   part, scal, counter, pev, ctx->hemv_ch[fp32], ctx->her2k_valu[fp32] >= 0 ? ctx->her2k_valu[fp32] : 1,
-                  hsys));
+                  hsys, prun.ws_el > 0 ? &prun : nullptr));
+    if (prun.ws_el > 0) {
+        int perr = 0;
+        HCK(hipMemcpyAsync(&perr, prun.err, sizeof(int), hipMemcpyDeviceToHost, st));
+        HCK(hipStreamSynchronize(st));
+        if (perr) {
+            HCK(hipMemcpyAsync(H, H0, hbytes, hipMemcpyDeviceToDevice, st));
+            int rc = autotune_hemv(ctx, fp32, n, H, acol, Yr, Yc);
+            if (rc) return rc;
+            HCK(bse_hetrd(st, fp32, n, H, nb, d, e, tauh, Vst, Tall, Wp, alpha2, Gram, acol, Yr, Yc, t12, part, scal,
+                          counter, nullptr, ctx->hemv_ch[fp32], ctx->her2k_valu[fp32] >= 0 ? ctx->her2k_valu[fp32] : 1,
+                          hsys, nullptr));
+        }
+    }
     if (pev) {
         HCK(hipStreamSynchronize(st));
         double ms = 0.0, bytes = 0.0;
         const double es = fp32 ? 8.0 : 16.0;
-        for (int c = 0; c < n - 1; ++c) {
+        const int ncol = std::min(n - 1, panel_first);      // the other columns have no such launch
+        for (int c = 0; c < ncol; ++c) {
             float t = 0.f;
             HCK(hipEventElapsedTime(&t, pev[2 * c], pev[2 * c + 1]));
             ms += t;
@@ -1060,7 +1093,7 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
         }
         ctx->hemv_ms = ms;
         ctx->hemv_bytes = bytes;
-        ctx->hemv_launches = n - 1;
+        ctx->hemv_launches = ncol;
     }
     const int64_t skws = (int64_t)64 * 1024 * 1024 / sizeof(double2) * 8;   // 512 MiB split-K workspace cap
     sk_el = std::min<int64_t>(skws, std::max<int64_t>((int64_t)64 * nb * std::max(n_vectors, 64), (int64_t)nb * nb * 512));

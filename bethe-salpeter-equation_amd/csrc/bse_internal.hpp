@@ -11,6 +11,16 @@
 #include <string>
 #include <vector>
 
+// Panels of the one-stage reduction that run in one launch each: from column
+// first on, nwg workgroups at most, messages and counters in ws (zeroed), err
+// (zeroed) as in resident.hpp.
+struct PanelRun {
+    int device, first, nwg;
+    double2* ws;
+    int64_t ws_el;
+    int* err;
+};
+
 // ---- kernel launchers implemented in the other translation units ----------
 extern "C" {
 hipError_t bse_launch_tb_states(hipStream_t, int, int, int, const double*, const double2*,
@@ -43,7 +53,14 @@ hipError_t bse_launch_tile_pad_zero(hipStream_t, int, int64_t, void*);
 void bse_hetrd_workspace(int, int, int64_t*, int64_t*, int64_t*, int64_t*);
 hipError_t bse_hetrd(hipStream_t, int, int, void*, int, double*, double*, double2*, double2*,
                      double2*, double2*, double2*, double2*, double2*, double2*, double2*, double2*,
-                     double*, double*, unsigned int*, hipEvent_t*, const unsigned char*, int, void*);
+                     double*, double*, unsigned int*, hipEvent_t*, const unsigned char*, int, void*,
+                     const PanelRun*);
+// panel kernel of the one-stage reduction (panel_kernels.hip)
+int bse_panel_workgroups(int, int);
+int bse_panel_first(int, int);
+int64_t bse_panel_workspace(int, int);
+hipError_t bse_launch_panel(hipStream_t, int, int, int, int, int, const void*, double2*, double2*, double2*, double2*,
+                            double*, double*, double2*, double2*, int64_t, int*);
 hipError_t bse_launch_hemv(hipStream_t, int, int, int, int, const void*, const double2*, double2*,
                            double2*);
 hipError_t bse_launch_last_diag(hipStream_t, int, int, const void*, double*);
@@ -280,7 +297,7 @@ enum Slot {
     S_RS, S_RHS, S_RX, S_RG, S_RHG, S_RC, S_RSMALL,
     S_GDHR, S_GDEPS, S_GDCOEF, S_GDP, S_GDPV, S_GDRHO, S_GDDE, S_GDW, S_GY, S_GOUT,
     S_SGFB, S_SGFA, S_SGX, S_SGU, S_SGB, S_SGV, S_SGPART, S_APPLYP, S_MEMB, S_KMAP, S_KINV, S_TBK, S_TBH, S_TBR, S_TBE, S_TBC,
-    S_BAB, S_BAB0, S_BPAN, S_BTSQR, S_BUPD, S_BPROG, S_BMSG, S_BII, S_BZERO, S_BH0, S_BFAIL,
+    S_BAB, S_BAB0, S_BPAN, S_BTSQR, S_BUPD, S_BPROG, S_BMSG, S_PNMSG, S_PNERR, S_BII, S_BZERO, S_BH0, S_BFAIL,
     // grouped back-transform: panel offsets, workspace
     S_BTVOFF, S_BTWS,
     // full BSE: coupling block, M / its Cholesky factor, W = L^H s3 L, tile
@@ -520,4 +537,4 @@ void batch_destroy(bse_ctx* ctx);
 
 // Autotuner of the tridiagonalisation's hemv chunk length (bse_api.hip).
 int autotune_hemv(bse_ctx* ctx, int fp32, int n, const void* H, double2* v, double2* Yr,
-                  double2* Yc);
+                  double2* Yc, int min_nt = 0);

@@ -34,6 +34,7 @@
 //
 // Band storage: AB[c * ldab + d] = A(c + d, c), 0 <= d <= 2b (FP64).
 #include "bse_common.hpp"
+#include "resident.hpp"
 #include <cfloat>
 #include <mutex>
 
@@ -162,7 +163,7 @@ __device__ inline void chase_post(const ChaseArgs& a, int s, int val, int lane, 
 // device-scope cache policy.  A masked-off element gets an offset past the
 // descriptor's range, which the hardware turns into a zero load or a
 // dropped store, so no access needs a branch.
-#define CH_SC1 16
+#define CH_SC1 RS_COHERENT
 #define CH_OOB ((int)0xFFFFFFF0u)
 template <int COH> struct ChaseMem {
     __amdgpu_buffer_rsrc_t rab, ry;
@@ -414,16 +415,13 @@ __global__ __launch_bounds__(64 * CH_W) void k_chase(ChaseArgs a)
 // with the band in device-coherent memory.
 //
 // Every workgroup must be resident (each waits on both neighbours): they meet
-// at a counter first (chase_meet) and leave together when that does not
+// at a counter first (rs_meet) and leave together when that does not
 // happen in time, with the band, y, d and e untouched; the host then runs
 // k_chase, whose workgroups only ever wait on earlier ones.  k_chase also
 // serves bands with more workgroups than the device holds (n above 32768 on
 // 256 CUs with four workgroups each).
 // ---------------------------------------------------------------------------
 #define CHS_LD 33                             // LDS stride of a block's columns
-#define CHS_SPIN (1u << 23)                   // polls (each a memory round trip) before a wait is given up
-#define CHS_MEET_TICKS 200000000ull           // 2 s of the 100 MHz clock
-#define CHS_ABORT 0x80000000u
 
 struct ChaseSysArgs {
     int n, ldab, npos;
@@ -442,13 +440,6 @@ struct ChaseSysArgs {
 #define CHS_D 193                             // 2 x 3: D_{k+1}(0,0), y
 #define CHS_SLOT 200
 
-__device__ inline bse_i4v chs_word(double v, int tag) {
-    const bse_i4v w = {__double2loint(v), tag, __double2hiint(v), tag};
-    return w;
-}
-__device__ inline bool chs_here(bse_i4v w, int tag) { return w[1] == tag && w[3] == tag; }
-__device__ inline double chs_value(bse_i4v w) { return __hiloint2double(w[2], w[0]); }
-
 // a + its partner in the other half of the wave, in the same order in both
 __device__ inline double chs_half_sum(double a) {
     const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(a), false, false);
@@ -463,41 +454,6 @@ __device__ inline double chs_lower(double a) {
 }
 __device__ inline double2 chs_half_sum2(double2 a) { return cmk(chs_half_sum(a.x), chs_half_sum(a.y)); }
 __device__ inline double2 chs_lower2(double2 a) { return cmk(chs_lower(a.x), chs_lower(a.y)); }
-
-// All workgroups resident?  An arrival adds one; a workgroup that has waited
-// too long sets CHS_ABORT, and only while the count is short (compare and
-// swap), so either every workgroup sees the full count or every one leaves.
-__device__ inline bool chase_meet(unsigned* meet, unsigned npos, int* err) {
-    unsigned v = __hip_atomic_fetch_add(meet, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
-    const unsigned long long t0 = wall_clock64();
-    for (;;) {
-        if (v & CHS_ABORT) break;
-        if (v == npos) return true;
-        if (wall_clock64() - t0 > CHS_MEET_TICKS) {
-            unsigned want = v;
-            if (__hip_atomic_compare_exchange_strong(meet, &want, v | CHS_ABORT, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT))
-                break;
-            v = want;
-            continue;
-        }
-        __builtin_amdgcn_s_sleep(4);
-        v = __hip_atomic_load(meet, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __hip_atomic_store(err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return false;
-}
-
-// One failed poll: true when the wait is to be given up.
-__device__ inline bool chs_give_up(unsigned& spins, int* err) {
-    ++spins;
-    if ((spins & 1023u) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return true;
-    if (spins > CHS_SPIN) {
-        __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return true;
-    }
-    return false;
-}
 
 __global__ __launch_bounds__(128, 2) void k_chase_resident(ChaseSysArgs a)
 {
@@ -545,7 +501,7 @@ __global__ __launch_bounds__(128, 2) void k_chase_resident(ChaseSysArgs a)
     double d0 = 0.0;
     if (k == 0 && threadIdx.x == 0) d0 = band(0, 0).x;
     __syncthreads();
-    if (threadIdx.x == 0) go = chase_meet(a.meet, (unsigned)a.npos, a.err) ? 1 : 0;
+    if (threadIdx.x == 0) go = rs_meet(a.meet, (unsigned)a.npos, a.err) ? 1 : 0;
     __syncthreads();
     if (!go) return;
     if (k == 0 && threadIdx.x == 0) a.d[0] = d0;
@@ -576,11 +532,11 @@ __global__ __launch_bounds__(128, 2) void k_chase_resident(ChaseSysArgs a)
                 const bse_i4v wv = __builtin_amdgcn_raw_buffer_load_b128(rin, (CHS_V + 2 * i + h) * 16, 0, CH_SC1);
                 const bse_i4v wb = __builtin_amdgcn_raw_buffer_load_b128(rin, CHS_BETA * 16, 0, CH_SC1);
                 const int fd = __hip_atomic_load(&fD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                const bool ok = (k == 0 || chs_here(wv, tag)) && (!rprev || chs_here(wb, s)) && fd >= s;
-                vw = chs_value(wv);
-                bw = rprev ? chs_value(wb) : 0.0;
+                const bool ok = (k == 0 || rs_here(wv, tag)) && (!rprev || rs_here(wb, s)) && fd >= s;
+                vw = rs_value(wv);
+                bw = rprev ? rs_value(wb) : 0.0;
                 if (__all(ok)) break;
-                if (chs_give_up(spins, a.err)) return;
+                if (rs_give_up(spins, a.err)) return;
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
             const double2 top = sCol[par ^ 1][(i + 1) & 31];         // entry i + 1 of D_k's first column
@@ -615,10 +571,10 @@ __global__ __launch_bounds__(128, 2) void k_chase_resident(ChaseSysArgs a)
             const double2 v = (i == 0) ? cmk(1.0, 0.0) : cmul(x, r.scal);
             const double2 out = (i == 0) ? r.tau : v;
             if (right)
-                __builtin_amdgcn_raw_buffer_store_b128(chs_word(h == 0 ? out.x : out.y, tag), rright,
+                __builtin_amdgcn_raw_buffer_store_b128(rs_word(h == 0 ? out.x : out.y, tag), rright,
                                                        (CHS_V + 2 * i + h) * 16, 0, CH_SC1);
             if (k > 0 && lane == 0)
-                __builtin_amdgcn_raw_buffer_store_b128(chs_word(r.beta, tag), rleft, CHS_BETA * 16, 0, CH_SC1);
+                __builtin_amdgcn_raw_buffer_store_b128(rs_word(r.beta, tag), rleft, CHS_BETA * 16, 0, CH_SC1);
             if (k == 0 && lane == 0) a.e[s] = r.beta;
             if (h == 0) sV[par][i] = v;
             if (lane == 0) sTau[par] = r.tau;
@@ -654,7 +610,7 @@ __global__ __launch_bounds__(128, 2) void k_chase_resident(ChaseSysArgs a)
             // the first row to the left: word 2 c + (real, imaginary)
             {
                 const double2 rw = sX[(((lane >> 1) + o) & 31) * CHS_LD + o];
-                __builtin_amdgcn_raw_buffer_store_b128(chs_word((lane & 1) ? rw.y : rw.x, tag), rleft,
+                __builtin_amdgcn_raw_buffer_store_b128(rs_word((lane & 1) ? rw.y : rw.x, tag), rleft,
                                                        (CHS_ROW + 64 * par + lane) * 16, 0, CH_SC1);
             }
         }
@@ -673,11 +629,11 @@ __global__ __launch_bounds__(128, 2) void k_chase_resident(ChaseSysArgs a)
                 const bse_i4v w1 = __builtin_amdgcn_raw_buffer_load_b128(
                     rin, (CHS_D + 3 * (par ^ 1) + min(lane, 2)) * 16, 0, CH_SC1);
                 const int fv = __hip_atomic_load(&fV, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                const bool ok = (!rprev || (chs_here(w0, s) && chs_here(w1, s))) && fv >= tag;
-                rw = rprev ? chs_value(w0) : 0.0;
-                dw = rprev ? chs_value(w1) : 0.0;
+                const bool ok = (!rprev || (rs_here(w0, s) && rs_here(w1, s))) && fv >= tag;
+                rw = rprev ? rs_value(w0) : 0.0;
+                dw = rprev ? rs_value(w1) : 0.0;
                 if (__all(ok)) break;
-                if (chs_give_up(spins, a.err)) return;
+                if (rs_give_up(spins, a.err)) return;
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
             reinterpret_cast<double*>(sR)[lane] = rw;
@@ -734,7 +690,7 @@ __global__ __launch_bounds__(128, 2) void k_chase_resident(ChaseSysArgs a)
                         const double y1 = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(yn.y), 0),
                                                            __builtin_amdgcn_readlane(__double2loint(yn.y), 0));
                         if (lane < 3)
-                            __builtin_amdgcn_raw_buffer_store_b128(chs_word(lane == 0 ? z0 : (lane == 1 ? y0 : y1), tag),
+                            __builtin_amdgcn_raw_buffer_store_b128(rs_word(lane == 0 ? z0 : (lane == 1 ? y0 : y1), tag),
                                                                    rleft, (CHS_D + 3 * par + lane) * 16, 0, CH_SC1);
                     } else if (lane == 0) {
                         a.d[s + 1] = z.x;
@@ -768,17 +724,27 @@ extern "C" int64_t bse_chase_resident_workspace(int n, int b, int ldab, int devi
     return (int64_t)((n - 2) / CH_B + 1) * CHS_SLOT + 1;
 }
 
-// Two of these kernels at once could each hold half of the device and wait
-// for the rest, so the launches on one device follow one another: each waits
-// for the event of the one before.
-struct ChaseQueue {
+// The resident kernels' launches on one device follow one another: see
+// resident.hpp.
+struct ResidentQueue {
     std::mutex m;
     hipEvent_t done = nullptr;
 };
-static ChaseQueue& chase_queue(int device)
+static ResidentQueue& resident_queue(int device)
 {
-    static ChaseQueue q[64];
+    static ResidentQueue q[64];
     return q[device & 63];
+}
+hipError_t resident_launch(int device, hipStream_t st, const std::function<hipError_t()>& launch)
+{
+    ResidentQueue& q = resident_queue(device);
+    const std::lock_guard<std::mutex> lock(q.m);
+    hipError_t rc;
+    if (!q.done) rc = hipEventCreateWithFlags(&q.done, hipEventDisableTiming);
+    else rc = hipStreamWaitEvent(st, q.done, 0);
+    if (rc != hipSuccess) return rc;
+    rc = launch();
+    return rc == hipSuccess ? hipEventRecord(q.done, st) : rc;
 }
 
 // err receives 0, 1 (a wait was given up) or 2 (the workgroups did not become
@@ -794,18 +760,10 @@ extern "C" hipError_t bse_launch_chase_resident(hipStream_t st, int device, int 
     if (rc != hipSuccess) return rc;
     const ChaseSysArgs args{n, ldab, npos, AB, y, d, e, reinterpret_cast<bse_i4v*>(ws),
                             reinterpret_cast<unsigned*>(ws + words), err};
-    ChaseQueue& q = chase_queue(device);
-    const std::lock_guard<std::mutex> lock(q.m);
-    if (!q.done) {
-        rc = hipEventCreateWithFlags(&q.done, hipEventDisableTiming);
-        if (rc != hipSuccess) return rc;
-    } else {
-        rc = hipStreamWaitEvent(st, q.done, 0);
-        if (rc != hipSuccess) return rc;
-    }
-    hipLaunchKernelGGL(k_chase_resident, dim3((unsigned)grid), dim3(128), 0, st, args);
-    rc = hipGetLastError();
-    return rc == hipSuccess ? hipEventRecord(q.done, st) : rc;
+    return resident_launch(device, st, [&]() -> hipError_t {
+        hipLaunchKernelGGL(k_chase_resident, dim3((unsigned)grid), dim3(128), 0, st, args);
+        return hipGetLastError();
+    });
 }
 
 extern "C" int64_t bse_chase_counters(int n) { return n > 1 ? n - 1 : 1; }

@@ -44,8 +44,7 @@
 // in the batched path also the compact-WY factor, which the single-matrix
 // path forms for all panels after the last column) before the trailing
 // update.
-#include "bse_common.hpp"
-#include <cstdlib>
+#include "bse_internal.hpp"
 
 struct HetrdCol {
     int n;            // matrix size (tiled lower storage, bse_common.hpp)
@@ -1419,14 +1418,16 @@ static_assert(sizeof(HetrdSys) <= 256, "HetrdSys must fit the 256-byte device sl
 // microsecond per launch).  Tall receives one nb x nb compact-WY factor per panel,
 // formed in one launch after the last column from the per-panel Gram blocks
 // (G: ceil((n-1)/nb) blocks of 64 x 64); prof_ev (optional) gets 2 events per
-// column around the hemv launch.
+// column around the hemv launch.  With run (nb = 32), the panels from column
+// run->first on take one launch each (panel_kernels.hip) in place of three
+// per column.
 extern "C" hipError_t bse_hetrd(hipStream_t st, int fp32, int n, void* A, int nb,
                                 double* d, double* e, double2* tau, double2* Vstore,
                                 double2* Tall, double2* Wp, double2* alpha2,
                                 double2* G, double2* acol, double2* Yr, double2* Yc, double2* t12,
                                 double* part, double* scal, unsigned int* counter,
                                 hipEvent_t* prof_ev, const unsigned char* ch_table, int her2k_kind,
-                                void* d_sys)
+                                void* d_sys, const PanelRun* run)
 {
     if (nb < 1 || nb > 32 || n < 1 || !d_sys) return hipErrorInvalidValue;
     hipError_t err;
@@ -1438,7 +1439,10 @@ extern "C" hipError_t bse_hetrd(hipStream_t st, int fp32, int n, void* A, int nb
         if ((err = hipMemcpyAsync(d_sys, &x, sizeof(x), hipMemcpyHostToDevice, st)) != hipSuccess)
             return err;
         const int ntile = tile_count(n);
-        for (int c = 0; c < n - 1; ++c) {
+        // columns before `first` by the per-column launches, the panels from
+        // there on in one launch each, followed by their trailing update
+        const int first = run ? run->first : n;
+        for (int c = 0; c < std::min(n - 1, first); ++c) {
             const int code = hemv_ch_for(ch_table, n - c - 1);
             err = column_launch(st, fp32, c, nb, 1, n, d_sys, code, prof_ev ? prof_ev[2 * c] : nullptr,
                                 prof_ev ? prof_ev[2 * c + 1] : nullptr);
@@ -1447,6 +1451,16 @@ extern "C" hipError_t bse_hetrd(hipStream_t st, int fp32, int n, void* A, int nb
             if (c != j0 + nbp - 1) continue;
             const int64_t nT = (j0 + nbp < n) ? ntile - ((j0 + nbp) >> 6) : 0;
             if ((err = bse_hetrd_batch_panel(st, fp32, c, nb, 1, d_sys, nT, her2k_kind)) != hipSuccess)
+                return err;
+        }
+        for (int j0 = first; j0 < n - 1; j0 += nb) {
+            const int p = j0 / nb, nbp = std::min(nb, n - 1 - j0);
+            double2* Vp = Vstore + panel_voff(n, nb, p);
+            if ((err = bse_launch_panel(st, run->device, fp32, n, j0, run->nwg, A, Vp, Wp, alpha2,
+                                        G + (int64_t)p * 64 * 64, d, e, tau, run->ws, run->ws_el, run->err)) != hipSuccess)
+                return err;
+            if ((err = bse_launch_her2k(st, fp32, her2k_kind, n, j0 + nbp, A, Vp, Wp, n - j0, j0, nbp, alpha2)) !=
+                hipSuccess)
                 return err;
         }
         const int npan = (int)ceil_div64(n - 1, nb);

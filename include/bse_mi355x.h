@@ -288,8 +288,9 @@ int  bse_stage_times(const bse_ctx* ctx, double* ms, int n);
  * recording on for later calls; out (may be NULL, else 9 doubles) receives,
  * for the last bse_eigh:
  *   one-stage reduction: [0] total time in ms of the Hermitian matrix-vector
- *     kernel, [1] its algorithmic bytes (lower triangle of every trailing
- *     block), [2] launches, [4] = 0;
+ *     kernel, [1] its algorithmic bytes (lower triangle of its trailing
+ *     blocks), [2] launches, [4] = 0 (the columns of panels that run in one
+ *     launch each have no such launch and are not counted);
  *   two-stage reduction: [0] ms, [1] = 1 when the products ran on FP32
  *     matrix cores, [2] launches, [3] algorithmic flops of the panels'
  *     rank-2k update (8 m (m+1) k per panel), [4] = 1, and [5] ms, [6] flops
