@@ -608,24 +608,13 @@ __global__ __launch_bounds__(256) void k_cq_reduce(int ng, const double2* __rest
 // 17 + 45 us now (N = 4624; half of the second kernel is its four
 // 32 x 32 products and their loads).
 
-// 1/x and 1/sqrt(x) of a positive normal x: the hardware estimates (about
-// 2^-24) and two Newton steps each, which end within 1-2 ulp; the compiler's
-// exactly rounded division and square root have about twice the dependent
-// latency, which every step of the factorisations below would wait for.
-__device__ inline double cq_rcp(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(r, fma(-x, r, 1.0), r);
-    return fma(r, fma(-x, r, 1.0), r);
-}
+// 1/sqrt(x) of a positive normal x, as rcp_nr: every step of the
+// factorisations below would wait for an exactly rounded one.
 __device__ inline double cq_rsq(double x) {
     double r = __builtin_amdgcn_rsq(x);
     r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
     return fma(0.5 * r, fma(-x * r, r, 1.0), r);
 }
-
-// c ? a : b on the components (a conditional on the vectors themselves selects
-// between their addresses and puts both in scratch memory).
-__device__ inline double2 csel(bool c, double2 a, double2 b) { return cmk(c ? a.x : b.x, c ? a.y : b.y); }
 
 // G (e = i + 32 c in Gs, summed by k_cq_reduce) = L L^H.  L is left in sL
 // (lower triangle, zeros above), L^{-1} in a (row i, columns 4 g ..; zeros
@@ -659,16 +648,24 @@ __device__ inline bool cq_factor(const double2* __restrict__ Gs, bool near_one, 
                 for (int q = 0; q < 4; ++q) sRow[j & 1][4 * g + q] = a[q];
             }
             __syncthreads();
-            // every LDS read of the step is issued before the first is used
+            // every LDS read of the step is issued before the first is used.
+            // The pivot row beyond the pivot is the column's conjugate: taken
+            // from the upper triangle, with the real part as the pivot, its
+            // rounding differences from the lower one would grow fourfold a step
             const double d = sL[j][j].x;
             const double2 col = sL[i][j];
             const double top = diag0[j];
             double2 pr[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) pr[q] = sRow[j & 1][4 * g + q];
-            // a zero or lost pivot: the result is dropped at the end
-            ok = ok && d > 1e-12 * top && top > 0.0;
-            const double2 m = cscale(col, cq_rcp(d));
+            for (int q = 0; q < 4; ++q) {
+                const int c = 4 * g + q;
+                const double2 x = sL[c][j], y = sRow[j & 1][c];
+                pr[q] = csel(c > j, cconj(x), y);
+            }
+            // a zero, lost or (for rcp_nr) too small pivot: the result is dropped
+            // at the end
+            ok = ok && d > 1e-12 * top && d > 1e-290;
+            const double2 m = cscale(col, rcp_nr(d));
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int c = 4 * g + q;
@@ -794,7 +791,7 @@ __global__ __launch_bounds__(256) void k_cq_chol2(int m, int b, const double2* _
             // d_j / u_jj = -conj(w) / (|w| + |w|^2); a |w| below 1e-140 (whose
             // square would underflow) counts as zero: d_j = u_jj = 1
             const double a2 = cabs2(wj);
-            const double2 sc = csel(a2 > 1e-280, cscale(cmk(-wj.x, wj.y), cq_rcp(fma(a2, cq_rsq(a2), a2))), cmk(1.0, 0.0));
+            const double2 sc = csel(a2 > 1e-280, cscale(cmk(-wj.x, wj.y), rcp_nr(fma(a2, cq_rsq(a2), a2))), cmk(1.0, 0.0));
             const double2 f = csel(i == j, cmk(-sc.x, -sc.y), cmul(sc, col));
 #pragma unroll
             for (int q = 0; q < 4; ++q) {

@@ -1046,10 +1046,17 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     const size_t hbytes = (size_t)tiled_elems(n) * (fp32 ? sizeof(float2) : sizeof(double2));
     void* H0 = nullptr;
     if (prun.ws_el > 0) {
+        int no = BSE_OK;
+        H0 = buf(ctx, S_BH0, hbytes, &no);
+        if (!H0) {
+            (void)hipGetLastError();
+            prun.ws_el = 0;                 // no room for the copy: per-column launches
+        }
+    }
+    if (prun.ws_el > 0) {
         prun.first = bse_panel_first(n, pnwg);
         prun.ws = BUF(double2, S_PNMSG, prun.ws_el);
         prun.err = BUF(int, S_PNERR, 4);
-        H0 = BUF(char, S_BH0, hbytes);
         HCK(bse_launch_zero_words(st, 2 * prun.ws_el, prun.ws));
         HCK(bse_launch_zero_words(st, 2, prun.err));
         HCK(hipMemcpyAsync(H0, H, hbytes, hipMemcpyDeviceToDevice, st));

@@ -169,6 +169,10 @@ __host__ __device__ inline double2 crecip(double2 a) {
     const double r = 1.0 / (a.x * a.x + a.y * a.y);
     return make_double2(a.x * r, -a.y * r);
 }
+// 1 / a where size, a few times |a| at most, says whether |a|^2 can be formed.
+__device__ inline double2 crecip_safe(double2 a, double size) {
+    return (size > 1e-145 && size < 1e150) ? crecip(a) : cdiv(make_double2(1.0, 0.0), a);
+}
 // Block reduction of a double over blockDim.x threads (multiple of 64, <= 1024).
 // Every thread receives the total.  Deterministic order.
 __device__ inline double block_sum(double v, double* sh /* >= 16 doubles */) {
@@ -225,6 +229,19 @@ __device__ inline bool last_block_ticket(unsigned int* counter, unsigned int nbl
 //   f64 (v_mfma_f64_16x16x4):                                  row = (l/16) + 4 r
 __device__ inline int mfma16_row_f32(int lane, int r) { return 4 * (lane >> 4) + r; }
 __device__ inline int mfma16_row_f64(int lane, int r) { return (lane >> 4) + 4 * r; }
+
+// 1/x of a positive normal x: the hardware estimate (about 2^-24) and two
+// Newton steps, which end within 1-2 ulp at half the dependent latency of the
+// compiler's exactly rounded division.
+__device__ inline double rcp_nr(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.0), r);
+    return fma(r, fma(-x, r, 1.0), r);
+}
+
+// c ? a : b on the components (a conditional on the vectors themselves selects
+// between their addresses and puts both in scratch memory).
+__device__ inline double2 csel(bool c, double2 a, double2 b) { return cmk(c ? a.x : b.x, c ? a.y : b.y); }
 
 __host__ __device__ inline int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }
 

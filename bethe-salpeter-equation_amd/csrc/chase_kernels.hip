@@ -68,7 +68,7 @@ __device__ inline Refl make_refl(double2 alpha, double ss) {
         const double nrm = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + ss);
         r.beta = (alpha.x >= 0.0) ? -nrm : nrm;
         r.tau = cmk((r.beta - alpha.x) / r.beta, -alpha.y / r.beta);
-        r.scal = crecip(cmk(alpha.x - r.beta, alpha.y));
+        r.scal = crecip_safe(cmk(alpha.x - r.beta, alpha.y), nrm);
     }
     return r;
 }

@@ -378,7 +378,7 @@ __global__ __launch_bounds__(PN_THREADS) void k_trd_panel(PanelArgs a)
                 const double nr = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + xn2);
                 beta = (alpha.x >= 0.0) ? -nr : nr;
                 tau = cmk((beta - alpha.x) / beta, -alpha.y / beta);
-                sc = crecip(cmk(alpha.x - beta, alpha.y));
+                sc = crecip_safe(cmk(alpha.x - beta, alpha.y), nr);
             }
         } else {
             double2 xp = cmk(0, 0), D = cmk(0, 0);
