@@ -1,119 +1,126 @@
 // Small dense FP64 linear algebra for the Rayleigh-Ritz refinement (K8):
 // everything lives in one workgroup's LDS (n <= 64).
 //
-// * Hermitian eigensolver: cyclic Jacobi with the Brent-Luk parallel ordering
-//   (n/2 disjoint rotations per step, n-1 steps per sweep), each rotation the
-//   complex 2x2 Jacobi rotation of Golub & Van Loan sec. 8.5, applied as a
-//   block J^H A J.
+// * Hermitian eigensolver: cyclic Jacobi in the round-robin order (n/2 disjoint
+//   rotations per step, n-1 steps per sweep), each rotation the complex 2x2
+//   Jacobi rotation of Golub & Van Loan sec. 8.5, applied as a block J^H A J.
 // * Rayleigh-Ritz with SVQB basis stabilisation (Stathopoulos & Wu 2002): for
 //   a basis S (not orthonormal) with G = S^H S and Hs = S^H H S, eig G =
 //   U diag(s) U^H, P = U diag(s^-1/2) (dropping s < tol s_max), eig of
 //   P^H Hs P = Y diag(l) Y^H, coefficients C = P Y of the lowest k Ritz pairs.
-#include "bse_common.hpp"
+#include "jacobi.hpp"
 
 #define SD_MAX 40
 
-// Jacobi on the LDS matrix A (ld SD_MAX), eigenvectors into V.  n <= SD_MAX.
-// On exit the diagonal of A holds the eigenvalues (unsorted).  One thread per
-// (pair, row) task: blockDim.x >= SD_JACOBI_THREADS.  A step reads A and
-// writes the rotated columns into A2, then reads A2 and writes the rotated
-// rows back into A, so no phase reads an entry another thread writes; every
-// thread forms its pair's rotation from A itself and keeps it for both
-// phases (two barriers per step).
-#define SD_JACOBI_THREADS ((SD_MAX / 2) * SD_MAX)
-__device__ void sd_jacobi(int n, double2 (*A)[SD_MAX + 1], double2 (*V)[SD_MAX + 1])
+// Jacobi on the LDS matrix A (ld SD_LD), eigenvectors into V.  n <= SD_MAX; rows and
+// columns from n up to the next even number are set to zero (such a pair does
+// not rotate).  On exit the diagonal of A holds the eigenvalues (unsorted).
+// A step rotates n/2 disjoint pairs: thread (P, Q) of the first waves forms
+// both pairs' rotations itself, reads the 2 x 2 block of A in the rows of pair
+// P and columns of pair Q and writes J_P^H B J_Q into the other copy of A, so a
+// step takes one barrier.  The other waves rotate V by the rotations of the
+// step before, which the threads (P, P) left in LDS: they form none themselves,
+// and the first waves have one SIMD each to themselves but for their few
+// products.  Bound by the latency of a step (LDS reads, two reciprocal square
+// roots, LDS writes, a barrier).  The Rayleigh-Ritz of order 32 took 1.29 ms
+// with two barriers, square roots and divisions per step and one task per
+// (pair, row), 0.76 ms with V's threads forming their rotations too, 0.53 ms now.
+#define SD_LD (SD_MAX + 1)
+#define SD_PAIRS (SD_MAX / 2)
+#define SD_JACOBI_THREADS 1024
+static_assert(SD_PAIRS * SD_PAIRS + 63 < SD_JACOBI_THREADS, "threads left for V");
+__device__ void sd_jacobi(int n, double2 (*A)[SD_LD], double2 (*V)[SD_LD])
 {
-    __shared__ double2 A2[SD_MAX][SD_MAX + 1];
+    __shared__ double2 A2[SD_MAX][SD_LD];
+    __shared__ JacobiRot rot[2][SD_PAIRS];
     __shared__ double sh[32];
     const int tid = threadIdx.x, nt = blockDim.x;
-    const int m = (n + 1) & ~1;   // even number of slots; slot n (if n odd) is a dummy
+    const int m = (n + 1) & ~1, h = m / 2;
     for (int e = tid; e < SD_MAX * SD_MAX; e += nt) {
         const int i = e / SD_MAX, j = e % SD_MAX;
         V[i][j] = cmk(i == j ? 1.0 : 0.0, 0.0);
+        if ((i >= n || j >= n) && i < m && j < m) A[i][j] = cmk(0, 0);
     }
-    // round-robin order at step r of a sweep: slot 0 holds 0, slot i >= 1
-    // holds ((i - 1 - r) mod (m - 1)) + 1 (slots 1.. shift right by one per
-    // step; after m - 1 steps the order is the identity again)
-    auto slot = [m](int i, int r) { return i == 0 ? 0 : ((i - 1 - r) % (m - 1) + (m - 1)) % (m - 1) + 1; };
     __syncthreads();
     double fro = 0.0;
     for (int e = tid; e < n * n; e += nt) fro += cabs2(A[e / n][e % n]);
     fro = block_sum(fro, sh);
-    const bool act = tid < (m / 2) * n;
-    const int t = act ? tid / n : 0, i = act ? tid % n : 0;
+    // pair j of step r: {m - 1, r} (j = 0) or {(r + j), (r - j)} mod (m - 1)
+    auto pair = [m](int j, int r, int& p, int& q) {
+        int u = (j == 0) ? m - 1 : r + j, v = r - j;
+        if (j > 0 && u >= m - 1) u -= m - 1;
+        if (v < 0) v += m - 1;
+        p = min(u, v);
+        q = max(u, v);
+    };
+    const int va = (h * h + 63) & ~63;               // first thread of V's waves
+    const bool act = tid < h * h;
+    int last = -1, cur = 0;                          // step whose rotations V still waits for
+    auto rotate_v = [&](int r, const JacobiRot* js) {
+        for (int t = tid - va; t < h * n; t += nt - va) {
+            int p, q;
+            const int j = t / n, i = t % n;
+            pair(j, r, p, q);
+            const JacobiRot rt = js[j];
+            const double2 v0 = V[i][p], v1 = V[i][q];
+            V[i][p] = csub(cscale(v0, rt.c), cmulc(rt.s, v1));
+            V[i][q] = cadd(cmul(rt.s, v0), cscale(v1, rt.c));
+        }
+    };
+    const int P = act ? tid / h : 0, Q = act ? tid % h : 0;
+    double2 (*X)[SD_LD] = A;
+    double2 (*Y)[SD_LD] = A2;
     for (int sweep = 0; sweep < 30; ++sweep) {
         double off = 0.0;
         for (int e = tid; e < n * n; e += nt) {
             const int r = e / n, j = e % n;
-            if (r != j) off += cabs2(A[r][j]);
+            if (r != j) off += cabs2(X[r][j]);
         }
         off = block_sum(off, sh);
         if (off <= 1e-30 * fro) break;
-        for (int step = 0; step < m - 1; ++step) {
-            // pair t of this step: (slot t, slot m-1-t); rotation from A
-            int p = slot(t, step), q = slot(m - 1 - t, step);
-            if (p > q) { const int x = p; p = q; q = x; }
-            double c = 1.0, s = 0.0;
-            double2 u = cmk(1.0, 0.0);
-            if (act && q < n) {
-                const double2 apq = A[p][q];
-                const double absa = sqrt(cabs2(apq));
-                if (absa > 0.0) {
-                    const double app = A[p][p].x, aqq = A[q][q].x;
-                    u = cmk(apq.x / absa, -apq.y / absa);
-                    const double theta = (aqq - app) / (2.0 * absa);
-                    double tt = 1.0 / (fabs(theta) + sqrt(theta * theta + 1.0));
-                    if (theta < 0.0) tt = -tt;
-                    c = 1.0 / sqrt(1.0 + tt * tt);
-                    s = tt * c;
-                }
-            }
-            const bool rot = act && q < n && s != 0.0;
-            // columns: (A J)(i, {p, q}) into A2, V J in place, with
-            // J = [[c, s], [-s u, c u]] on (p, q); other pairs copied
+        for (int r = 0; r < m - 1; ++r) {
             if (act) {
-                const double2 aip = A[i][p];
-                if (rot) {
-                    const double2 aiq = A[i][q];
-                    const double2 su = cscale(u, s), cu = cscale(u, c);
-                    A2[i][p] = csub(cscale(aip, c), cmul(aiq, su));
-                    A2[i][q] = cadd(cscale(aip, s), cmul(aiq, cu));
-                    const double2 vip = V[i][p], viq = V[i][q];
-                    V[i][p] = csub(cscale(vip, c), cmul(viq, su));
-                    V[i][q] = cadd(cscale(vip, s), cmul(viq, cu));
-                } else {
-                    A2[i][p] = aip;
-                    if (q < n) A2[i][q] = A[i][q];
+                int p1, q1, p2, q2;
+                pair(P, r, p1, q1);
+                pair(Q, r, p2, q2);
+                const JacobiRot rp = jacobi_rot(X[p1][p1].x, X[q1][q1].x, X[p1][q1]);
+                const JacobiRot rq = jacobi_rot(X[p2][p2].x, X[q2][q2].x, X[p2][q2]);
+                const double2 a00 = X[p1][p2], a01 = X[p1][q2], a10 = X[q1][p2], a11 = X[q1][q2];
+                const double2 b00 = csub(cscale(a00, rq.c), cmulc(rq.s, a01)), b01 = cadd(cmul(rq.s, a00), cscale(a01, rq.c));
+                const double2 b10 = csub(cscale(a10, rq.c), cmulc(rq.s, a11)), b11 = cadd(cmul(rq.s, a10), cscale(a11, rq.c));
+                double2 c00 = csub(cscale(b00, rp.c), cmul(rp.s, b10)), c01 = csub(cscale(b01, rp.c), cmul(rp.s, b11));
+                double2 c10 = cadd(cmulc(rp.s, b00), cscale(b10, rp.c)), c11 = cadd(cmulc(rp.s, b01), cscale(b11, rp.c));
+                if (P == Q) {
+                    rot[cur][P] = rp;
+                    c00 = cmk(a00.x - rp.dl, 0.0);
+                    c11 = cmk(a11.x + rp.dl, 0.0);
+                    c01 = c10 = cmk(0, 0);
                 }
+                Y[p1][p2] = c00;
+                Y[p1][q2] = c01;
+                Y[q1][p2] = c10;
+                Y[q1][q2] = c11;
             }
+            if (tid >= va && last >= 0) rotate_v(last, rot[cur ^ 1]);
+            last = r;
+            cur ^= 1;
             __syncthreads();
-            // rows: J^H (A J) back into A; the rotated pair's off-diagonal
-            // entries are set to zero and its diagonal to real
-            if (act) {
-                const int j = i;
-                const double2 bpj = A2[p][j];
-                if (rot) {
-                    const double2 bqj = A2[q][j];
-                    const double2 uc = cconj(u);
-                    double2 np = csub(cscale(bpj, c), cmul(bqj, cscale(uc, s)));
-                    double2 nq = cadd(cscale(bpj, s), cmul(bqj, cscale(uc, c)));
-                    if (j == q) { np = cmk(0, 0); nq.y = 0.0; }
-                    if (j == p) { nq = cmk(0, 0); np.y = 0.0; }
-                    A[p][j] = np;
-                    A[q][j] = nq;
-                } else {
-                    A[p][j] = bpj;
-                    if (q < n) A[q][j] = A2[q][j];
-                }
-            }
-            __syncthreads();
+            double2 (*t)[SD_LD] = X;
+            X = Y;
+            Y = t;
         }
+    }
+    if (tid >= va && last >= 0) rotate_v(last, rot[cur ^ 1]);
+    __syncthreads();
+    if (X != A) {
+        for (int e = tid; e < n * n; e += nt) A[e / n][e % n] = X[e / n][e % n];
+        __syncthreads();
     }
 }
 
 // Sort the Jacobi result ascending: writes eigenvalues to w[0..n) and the
 // permutation to perm[0..n) (shared).
-__device__ void sd_sort(int n, double2 (*A)[SD_MAX + 1], double* w, int* perm)
+__device__ void sd_sort(int n, double2 (*A)[SD_LD], double* w, int* perm)
 {
     __shared__ double tmp[SD_MAX];
     if (threadIdx.x == 0) {
@@ -139,9 +146,9 @@ __global__ __launch_bounds__(SD_JACOBI_THREADS) void k_small_rr(int m, int k, co
                                                  double* __restrict__ evals,
                                                  double2* __restrict__ C, int* __restrict__ info)
 {
-    __shared__ double2 A[SD_MAX][SD_MAX + 1];
-    __shared__ double2 V[SD_MAX][SD_MAX + 1];
-    __shared__ double2 P[SD_MAX][SD_MAX + 1];
+    __shared__ double2 A[SD_MAX][SD_LD];
+    __shared__ double2 V[SD_MAX][SD_LD];
+    __shared__ double2 P[SD_MAX][SD_LD];
     __shared__ double w[SD_MAX];
     __shared__ int perm[SD_MAX];
     __shared__ int rank;

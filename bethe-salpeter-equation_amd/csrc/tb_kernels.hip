@@ -25,7 +25,7 @@
 // one matrix rather than taking one each: 257 matrices of order 8 took
 // 1.27 ms (of order 16: 11 ms) with one thread per matrix and its arrays in
 // scratch memory, 0.047 ms (0.16 ms) now.
-#include "bse_common.hpp"
+#include "jacobi.hpp"
 
 #define TB_MAXORB BSE_MAXORB
 #define TB_WAVES 4             // waves per workgroup
@@ -35,40 +35,6 @@
 __device__ inline void tb_sync() {
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup", "local");
     __builtin_amdgcn_wave_barrier();
-}
-
-// 1/sqrt(x), x > 0: the hardware estimate and two Newton steps (1-2 ulp).
-__device__ inline double tb_rsq(double x) {
-    double r = __builtin_amdgcn_rsq(x);
-    r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
-    return fma(0.5 * r, fma(-x * r, r, 1.0), r);
-}
-
-// Rotation of columns p, q:  p' = c p - conj(s) q,  q' = s p + c q, that
-// zeroes A(p, q) = a; dl = what a(p, p) loses and a(q, q) gains.
-struct TbRot { double c, dl; double2 s; };
-__device__ inline TbRot tb_rot(double app, double aqq, double2 a) {
-    // h = (a_qq - a_pp)/2, r = sqrt(h^2 + |a|^2), c^2 = (r + |h|)/(2 r),
-    // s = sign(h) a / (2 r c); the pair is scaled by its size so that no
-    // square leaves the range
-    TbRot t;
-    const double h0 = 0.5 * (aqq - app);
-    const double big = fmax(fabs(h0), fmax(fabs(a.x), fabs(a.y)));
-    const bool act = (a.x != 0.0 || a.y != 0.0) && big > 0.0;
-    int ex;
-    (void)frexp(act ? big : 1.0, &ex);
-    const double h = ldexp(h0, -ex);
-    const double2 z = cmk(ldexp(a.x, -ex), ldexp(a.y, -ex));
-    const double g2 = cabs2(z);
-    const double ir = tb_rsq(act ? fma(h, h, g2) : 1.0);
-    const double c2 = fma(0.5 * fabs(h), ir, 0.5);
-    const double ic = tb_rsq(c2);
-    const double f = copysign(0.5 * ir * ic, h);
-    t.c = act ? c2 * ic : 1.0;
-    t.s = act ? cscale(z, f) : cmk(0, 0);
-    // |a| tan = sign(h) |a|^2 / (|h| + r)
-    t.dl = act ? ldexp(g2 * f * ic, ex) : 0.0;
-    return t;
 }
 
 template <int MP> struct TbShape {
@@ -203,8 +169,8 @@ __global__ __launch_bounds__(64 * TB_WAVES) void k_tb_states(
             int p1, q1, p2, q2;
             pair(P, p1, q1);
             pair(Q, p2, q2);
-            const TbRot rp = tb_rot(A[at(p1, p1)].x, A[at(q1, q1)].x, A[at(p1, q1)]);
-            const TbRot rq = tb_rot(A[at(p2, p2)].x, A[at(q2, q2)].x, A[at(p2, q2)]);
+            const JacobiRot rp = jacobi_rot(A[at(p1, p1)].x, A[at(q1, q1)].x, A[at(p1, q1)]);
+            const JacobiRot rq = jacobi_rot(A[at(p2, p2)].x, A[at(q2, q2)].x, A[at(p2, q2)]);
             const double2 a00 = A[at(p1, p2)], a01 = A[at(p1, q2)], a10 = A[at(q1, p2)], a11 = A[at(q1, q2)];
             const double2 v00 = V[at(P, p2)], v01 = V[at(P, q2)], v10 = V[at(P + MP, p2)], v11 = V[at(P + MP, q2)];
             // columns of pair Q, then rows of pair P (J^H from the left)
