@@ -276,68 +276,122 @@ extern "C" hipError_t bse_launch_rows_from_reference(hipStream_t st, int64_t N, 
 // Y <- Q Y (adjoint = 0; decreasing order, T), with Q = prod_p (I - V_p T_p V_p^H)
 // from the packed FP64 reflector store (panel p at nb (p n - nb p (p-1)/2),
 // ld n - p nb) and the per-panel compact-WY factors (nb x nb, ld nb).
-// One workgroup (APQ_THREADS threads; 512 keep the 32 partial dots of a
-// thread in registers, 1024 spill them) per vector walks all panels; for
-// each it forms w1 = V^H y (wave sums), w2 = T^(H) w1 and y -= V w2.  For the small
-// matrices of the batched sweep, where one vector is a few MB of reflector
-// reads, this replaces three GEMM launches per panel.  nb <= 32.
+// One workgroup per vector walks all panels; for each it forms w1 = V^H y,
+// w2 = T^(H) w1 and y -= V w2.  For the small matrices of the batched sweep,
+// where one vector is a few MB of reflector reads, this replaces three GEMM
+// launches per panel.  nb <= 32.
+//
+// The chain of panels is the bound, so a panel is kept to three barriers and
+// three trips to the cache.  In the dots the lower eight waves take reflectors
+// 0 .. 15 and the upper ones 16 .. 31 (a thread's 16 loads are in flight
+// together and everything fits its 128 registers); the 32 real sums of a wave
+// are folded by halves (lane pairs 32 apart exchange 16 values, then 8, ...:
+// 32 exchanges instead of 192).  T is read with the dots and multiplied from
+// LDS by one wave.  N = 1600: 1000 us a vector with T read element by element
+// inside its product and six exchanges per sum, 300 us this way.
 // ---------------------------------------------------------------------------
 #define APQ_NB 32
-#ifndef APQ_THREADS
-#define APQ_THREADS 512
-#endif
+#define APQ_THREADS 1024
+template <int O>
+__device__ __forceinline__ void apq_fold(double (&v)[APQ_NB], int lane) {
+    constexpr int h = O / 2;
+    const bool up = (lane & O) != 0;
+#pragma unroll
+    for (int i = 0; i < h; ++i) {
+        const double keep = up ? v[h + i] : v[i], give = up ? v[i] : v[h + i];
+        v[i] = keep + __shfl_xor(give, O, 64);
+    }
+}
 __global__ __launch_bounds__(APQ_THREADS) void k_apply_q(int n, int nb, const double2* __restrict__ Vstore,
                                                  const double2* __restrict__ Tall,
                                                  double2* __restrict__ Y, int64_t ldy, int adjoint)
 {
-    constexpr int NW = APQ_THREADS / 64;
-    __shared__ double2 s_red[NW][APQ_NB];
-    __shared__ double2 s_w1[APQ_NB], s_w2[APQ_NB];
+    constexpr int NW = APQ_THREADS / 64, HB = APQ_NB / 2, HR = APQ_THREADS / 2;
+    __shared__ double s_red[NW][APQ_NB];
+    __shared__ double2 s_T[APQ_NB][APQ_NB + 1], s_w1[APQ_NB], s_w2[APQ_NB];
     double2* y = Y + (int64_t)blockIdx.x * ldy;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int npan = (int)ceil_div64(n - 1, nb);
     for (int pp = 0; pp < npan; ++pp) {
         const int p = adjoint ? pp : npan - 1 - pp;
         const int j0 = p * nb, m = n - j0, nbp = min(nb, n - 1 - j0);
         const double2* V = Vstore + (int64_t)nb * ((int64_t)p * n - (int64_t)nb * p * (p - 1) / 2);
         const double2* T = Tall + (size_t)p * nb * nb;
-        double2 acc[APQ_NB];
+        {
+            // s_T[k][l] multiplies w1[k] in w2[l]; T is upper triangular
+            const int a = tid & 31, c = tid >> 5;
+            const double2 x = T[min(a, nb - 1) + min(c, nb - 1) * nb];
+            const bool in = a <= c && c < nbp;
+            if (adjoint) s_T[a][c] = cmk(in ? x.x : 0.0, in ? -x.y : 0.0);
+            else s_T[c][a] = cmk(in ? x.x : 0.0, in ? x.y : 0.0);
+        }
+        // dots: reflectors l0 .. l0 + 15 of the rows of this half
+        // (a wave's: scalar column addresses)
+        const int l0 = __builtin_amdgcn_readfirstlane(w) >= NW / 2 ? HB : 0;
+        double v[APQ_NB];
 #pragma unroll
-        for (int l = 0; l < APQ_NB; ++l) acc[l] = cmk(0, 0);
-        for (int r = threadIdx.x; r < m; r += APQ_THREADS) {
+        for (int l = 0; l < APQ_NB; ++l) v[l] = 0.0;
+        for (int r = tid & (HR - 1); r < m; r += HR) {
             const double2 yr = y[j0 + r];
 #pragma unroll
-            for (int l = 0; l < APQ_NB; ++l)
-                if (l < nbp) cfmac(acc[l], V[r + (int64_t)l * m], yr);
-        }
+            for (int b = 0; b < HB; b += 8) {
+                double2 x[8];
 #pragma unroll
-        for (int l = 0; l < APQ_NB; ++l) {
-            const double x = wave_sum(acc[l].x), z = wave_sum(acc[l].y);
-            if (lane == 0) s_red[w][l] = cmk(x, z);
-        }
-        __syncthreads();
-        if (threadIdx.x < APQ_NB) {
-            const int l = threadIdx.x;
-            double2 t = s_red[0][l];
-            for (int ww = 1; ww < NW; ++ww) t = cadd(t, s_red[ww][l]);
-            s_w1[l] = t;
-        }
-        __syncthreads();
-        if (threadIdx.x < nbp) {
-            const int l = threadIdx.x;
-            double2 s = cmk(0, 0);
-            if (adjoint) {
-                for (int k = 0; k <= l; ++k) cfmac(s, T[k + l * nb], s_w1[k]);
-            } else {
-                for (int k = l; k < nbp; ++k) cfma(s, T[l + k * nb], s_w1[k]);
+                for (int l = 0; l < 8; ++l) x[l] = (V + (int64_t)min(l0 + b + l, nbp - 1) * m)[r];
+#pragma unroll
+                for (int l = 0; l < 8; ++l) {
+                    double2 s = cmk(v[b + l], v[HB + b + l]);
+                    cfmac(s, x[l], yr);
+                    v[b + l] = s.x;
+                    v[HB + b + l] = s.y;
+                }
             }
-            s_w2[l] = s;
+        }
+        // fold by halves: lane bits 5 .. 1 choose the sum, bit 0 is added last
+        apq_fold<32>(v, lane);
+        apq_fold<16>(v, lane);
+        apq_fold<8>(v, lane);
+        apq_fold<4>(v, lane);
+        apq_fold<2>(v, lane);
+        v[0] += __shfl_xor(v[0], 1, 64);
+        if ((lane & 1) == 0) s_red[w][lane >> 1] = v[0];
+        __syncthreads();
+        if (w == 0) {
+            // lane: sum (lane & 31) of half lane >> 5 over that half's waves
+            double t = 0.0;
+#pragma unroll
+            for (int u = 0; u < NW / 2; ++u) t += s_red[(lane >> 5) * (NW / 2) + u][lane & 31];
+            const int l = (lane >> 5) * HB + (lane & (HB - 1));
+            double* dst = (double*)&s_w1[l];
+            dst[(lane & HB) ? 1 : 0] = l < nbp ? t : 0.0;
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            // w2[l]: each half-wave multiplies 16 of the terms
+            double2 s = cmk(0, 0);
+#pragma unroll 4
+            for (int q = 0; q < HB; ++q) {
+                const int k = (lane >> 5) * HB + q;
+                cfma(s, s_T[k][lane & 31], s_w1[k]);
+            }
+            s.x += __shfl_xor(s.x, 32, 64);
+            s.y += __shfl_xor(s.y, 32, 64);
+            if (lane < APQ_NB) s_w2[lane] = s;
         }
         __syncthreads();
-        for (int r = threadIdx.x; r < m; r += APQ_THREADS) {
+        for (int r = tid; r < m; r += APQ_THREADS) {
             double2 s = cmk(0, 0);
-            for (int l = 0; l < nbp; ++l) cfma(s, V[r + (int64_t)l * m], s_w2[l]);
-            y[j0 + r] = csub(y[j0 + r], s);
+            const double2 yr = y[j0 + r];
+            // w2 is zero beyond nbp
+#pragma unroll 1
+            for (int h = 0; h < APQ_NB; h += HB) {
+                double2 x[HB];
+#pragma unroll
+                for (int l = 0; l < HB; ++l) x[l] = (V + (int64_t)min(h + l, nbp - 1) * m)[r];
+#pragma unroll
+                for (int l = 0; l < HB; ++l) cfma(s, x[l], s_w2[h + l]);
+            }
+            y[j0 + r] = csub(yr, s);
         }
         __syncthreads();
     }
