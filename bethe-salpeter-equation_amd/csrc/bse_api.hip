@@ -677,6 +677,11 @@ static int autotune_her2k(bse_ctx* ctx, int fp32, void* scratch, size_t scratch_
 // reflectors in S_VSTORE / S_TALL (ctx->band_panels).
 // ---------------------------------------------------------------------------
 static const int kBand = 32;
+// Back-transform of more than 16 vectors: four panels per pass from this order
+// on, panel by panel below it, where there is one group or two and forming its
+// T is what is left (n = 144, 144 vectors: 0.24 ms by panels, 0.35 grouped;
+// n = 300: 0.69 and 0.47; n = 2600, 24 vectors: 7.8 and 2.1, 2600: 16.6 and 5.6).
+static const int kGroupedMinN = 256;
 
 // Automatic choice (two_stage == 0) when at most 20 vectors are wanted: the
 // two-stage reduction for FP64 storage from order 256 up and for FP32
@@ -1344,7 +1349,7 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
         HCK(hipStreamWaitEvent(st, ctx->join_ev, 0));
     } else if (nstore > 0 && nstore <= 16 && bse_apply_q_thin_workspace(n) <= sk_el) {
         HCK(bse_apply_q_thin(st, n, nb, Vst, Tall, nstore, Z, n, 0, skw));
-    } else if (nstore >= 2048 && nb == 32 && !getenv("BSE_BT_STRIPS")) {
+    } else if (nstore > 16 && n >= kGroupedMinN && nb == 32 && !getenv("BSE_BT_STRIPS")) {
         // many vectors: four panels per pass on FP64 matrix cores
         int64_t* voff_d = BUF(int64_t, S_BTVOFF, npan);
         HCK(hipMemcpyAsync(voff_d, voff.data(), sizeof(int64_t) * npan, hipMemcpyHostToDevice, st));

@@ -16,7 +16,7 @@
 // The strip is read twice and written once per panel, V once per phase from
 // L2.  Work per panel 16 m nbp ncols real flops (m = n - j0).  Every sum runs
 // in a fixed order, so the result is bitwise reproducible.
-#include "bse_common.hpp"
+#include "mma64.hpp"
 #include <algorithm>
 
 #define BT_CS 32       // columns per strip
@@ -204,53 +204,11 @@ extern "C" hipError_t bse_apply_q_strips(hipStream_t st, int n, int nb, int npan
 // Column k of a group is reflector l = k mod 32 of panel q = k / 32; it is
 // zero above group row 32 q and, for a short last panel, beyond its count.
 // ---------------------------------------------------------------------------
-typedef double btg_d4 __attribute__((ext_vector_type(4)));
 #define BTG_P 4                   // panels per group
 #define BTG_K (BTG_P * BT_NB)     // reflectors per group
-#ifndef BTG_KB
-#define BTG_KB 4                  // K steps per prefetched block
-#endif
 #ifndef BTG_WG
 #define BTG_WG 4096               // target workgroups of a full-height V^H Z launch
 #endif
-
-__device__ __forceinline__ btg_d4 btg_mfma(double a, double b, btg_d4 c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
-// c += a b for MT x NT complex 16 x 16 tiles (one K step of 4); a[i] is the
-// lane's A element of row tile i, b[j] its B element of column tile j.
-template <int MT, int NT>
-__device__ __forceinline__ void btg_cmma(btg_d4 (&cr)[MT][NT], btg_d4 (&ci)[MT][NT], const double2 (&a)[MT],
-                                         const double2 (&b)[NT]) {
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) cr[i][j] = btg_mfma(a[i].x, b[j].x, cr[i][j]);
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) ci[i][j] = btg_mfma(a[i].x, b[j].y, ci[i][j]);
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) cr[i][j] = btg_mfma(-a[i].y, b[j].y, cr[i][j]);
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) ci[i][j] = btg_mfma(a[i].y, b[j].x, ci[i][j]);
-}
-
-template <int MT, int NT>
-__device__ __forceinline__ void btg_zero(btg_d4 (&cr)[MT][NT], btg_d4 (&ci)[MT][NT]) {
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            cr[i][j] = btg_d4{0.0, 0.0, 0.0, 0.0};
-            ci[i][j] = btg_d4{0.0, 0.0, 0.0, 0.0};
-        }
-}
 
 // Panel p starts at row rb + 32 p and holds min(32, n - co - (rb + 32 p))
 // reflectors: rb = 0, co = 1 for the one-stage reduction (reflector j acts
@@ -268,46 +226,6 @@ struct BtgGroup {
     // reflectors of panel q of the group
     __device__ int nbp(int n, int q) const { return min(BT_NB, n - co - j0 - BT_NB * q); }
 };
-
-// Reduction over group rows r in [rlo, rhi) of conj(Va[r][a]) Vb[r][b] or
-// conj(Va[r][a]) Z[r][b] for one wave's 32 x 32 output (2 x 2 tiles).  The
-// lane's operand pointers pa[i], pb[j] address row 0 of its column (valid
-// flags va, vb).  Inside a block of 4 BTG_KB rows, K step t of lane quad lq
-// reads row rb + lq BTG_KB + t, so a lane reads BTG_KB consecutive rows.
-__device__ __forceinline__ void btg_rows(btg_d4 (&cr)[2][2], btg_d4 (&ci)[2][2], const double2* const (&pa)[2],
-                                         const bool (&va)[2], const double2* const (&pb)[2], const bool (&vb)[2],
-                                         int rlo, int rhi, int lq) {
-    double2 a[BTG_KB][2], b[BTG_KB][2];
-    auto load = [&](int rb, double2 (&A)[BTG_KB][2], double2 (&B)[BTG_KB][2]) {
-#pragma unroll
-        for (int t = 0; t < BTG_KB; ++t) {
-            const int r = rb + lq * BTG_KB + t;
-            const bool in = r < rhi;
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const double2 v = (in && va[i]) ? pa[i][r] : cmk(0, 0);
-                A[t][i] = cmk(v.x, -v.y);
-            }
-#pragma unroll
-            for (int j = 0; j < 2; ++j) B[t][j] = (in && vb[j]) ? pb[j][r] : cmk(0, 0);
-        }
-    };
-    if (rlo >= rhi) return;
-    load(rlo, a, b);
-    for (int rb = rlo; rb < rhi; rb += 4 * BTG_KB) {
-        double2 an[BTG_KB][2], bn[BTG_KB][2];
-        const bool more = rb + 4 * BTG_KB < rhi;
-        if (more) load(rb + 4 * BTG_KB, an, bn);
-#pragma unroll
-        for (int t = 0; t < BTG_KB; ++t) btg_cmma<2, 2>(cr, ci, a[t], b[t]);
-        if (more) {
-#pragma unroll
-            for (int t = 0; t < BTG_KB; ++t)
-#pragma unroll
-                for (int i = 0; i < 2; ++i) { a[t][i] = an[t][i]; b[t][i] = bn[t][i]; }
-        }
-    }
-}
 
 // Gram blocks V_i^H V_q (32 x 32, column-major) of every group: grid
 // (6 pairs, groups); the four waves split the rows, summed in wave order.
@@ -450,42 +368,52 @@ __global__ __launch_bounds__(256) void k_btg_w1(int n, int npan, int rb, int co,
             }
 }
 
-// W2[k][c] = -sum_k' T[k][k'] sum_s W1p[s][k'][c]: grid column tiles of 32;
-// the partials are summed into LDS, wave w forms rows 32 w .. of W2.
+// W2[k][c] = -sum_k' T[k][k'] sum_s W1p[s][k'][c]: grid column tiles of 16;
+// the partials are summed into LDS (in chunk order; eight loads of one sum are
+// in flight together, since nothing else hides their latency in a grid this
+// small), wave w forms rows 32 w .. of W2.  3600 columns, 32 partials: 158 us
+// with column tiles of 32 and one load at a time, 51 us this way.
 __global__ __launch_bounds__(256) void k_btg_w2(int nsplit, const double2* __restrict__ T,
                                                 const double2* __restrict__ W1p, int ncols, double2* __restrict__ W2)
 {
-    __shared__ double2 sW[BTG_K][32];
-    const int tid = threadIdx.x, c0 = blockIdx.x * 32;
-    for (int e = tid; e < BTG_K * 32; e += 256) {
-        const int k = e / 32, c = c0 + e % 32;
+    __shared__ double2 sW[BTG_K][16];
+    const int tid = threadIdx.x, c0 = blockIdx.x * 16;
+    const int64_t ps = (int64_t)BTG_K * ncols;
+    for (int e = tid; e < BTG_K * 16; e += 256) {
+        const int k = e / 16, c = c0 + e % 16;
         double2 v = cmk(0, 0);
-        if (c < ncols)
-            for (int s = 0; s < nsplit; ++s) v = cadd(v, W1p[((int64_t)s * BTG_K + k) * ncols + c]);
-        sW[k][e % 32] = v;
+        if (c < ncols) {
+            const double2* p = W1p + (int64_t)k * ncols + c;
+            int s = 0;
+            for (; s + 8 <= nsplit; s += 8) {
+                double2 x[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) x[u] = p[(s + u) * ps];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v = cadd(v, x[u]);
+            }
+            for (; s < nsplit; ++s) v = cadd(v, p[s * ps]);
+        }
+        sW[k][e % 16] = v;
     }
     __syncthreads();
     const int w = tid >> 6, lane = tid & 63, li = lane & 15, lq = lane >> 4;
-    btg_d4 cr[2][2], ci[2][2];
-    btg_zero<2, 2>(cr, ci);
+    btg_d4 cr[2][1], ci[2][1];
+    btg_zero<2, 1>(cr, ci);
     for (int k0 = BT_NB * w; k0 < BTG_K; k0 += 4) {
-        double2 a[2], b[2];
+        double2 a[2], b[1];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            a[t] = T[(BT_NB * w + 16 * t + li) + (int64_t)BTG_K * (k0 + lq)];
-            b[t] = sW[k0 + lq][16 * t + li];
-        }
-        btg_cmma<2, 2>(cr, ci, a, b);
+        for (int t = 0; t < 2; ++t) a[t] = T[(BT_NB * w + 16 * t + li) + (int64_t)BTG_K * (k0 + lq)];
+        b[0] = sW[k0 + lq][li];
+        btg_cmma<2, 1>(cr, ci, a, b);
     }
 #pragma unroll
     for (int ti = 0; ti < 2; ++ti)
 #pragma unroll
-        for (int tj = 0; tj < 2; ++tj)
-#pragma unroll
-            for (int reg = 0; reg < 4; ++reg) {
-                const int k = BT_NB * w + 16 * ti + mfma16_row_f64(lane, reg), c = c0 + 16 * tj + li;
-                if (c < ncols) W2[(int64_t)k * ncols + c] = cmk(-cr[ti][tj][reg], -ci[ti][tj][reg]);
-            }
+        for (int reg = 0; reg < 4; ++reg) {
+            const int k = BT_NB * w + 16 * ti + mfma16_row_f64(lane, reg), c = c0 + li;
+            if (c < ncols) W2[(int64_t)k * ncols + c] = cmk(-cr[ti][0][reg], -ci[ti][0][reg]);
+        }
 }
 
 // Z[j0 + r][c] += sum_k V[r][k] W2[k][c], computed as the transposed product
@@ -560,10 +488,11 @@ __global__ __launch_bounds__(256) void k_btg_upd(int n, int npan, int rb, int co
             }
 }
 
-static int btg_nsplit(int ncols) {
+static int btg_nsplit(int n, int ncols) {
     // about BTG_WG workgroups for the V^H Z partials of a full-height group,
-    // at most 32 partials for the reduction to sum
-    return (int)std::min<int64_t>(32, std::max<int64_t>(1, ceil_div64(BTG_WG, ceil_div64(ncols, 32))));
+    // at most 32 partials for the reduction to sum, of at least 64 rows each
+    const int64_t cap = std::min<int64_t>(32, ceil_div64(n, 64));
+    return (int)std::min<int64_t>(cap, std::max<int64_t>(1, ceil_div64(BTG_WG, ceil_div64(ncols, 32))));
 }
 
 // Workspace (complex elements) of the grouped back-transform: the Gram blocks
@@ -571,7 +500,7 @@ static int btg_nsplit(int ncols) {
 extern "C" int64_t bse_apply_q_grouped_workspace(int n, int npan, int ncols)
 {
     const int64_t ng = ceil_div64(npan, BTG_P);
-    return ng * 6 * BT_NB * BT_NB + ng * BTG_K * BTG_K + (int64_t)(btg_nsplit(ncols) + 1) * BTG_K * ncols;
+    return ng * 6 * BT_NB * BT_NB + ng * BTG_K * BTG_K + (int64_t)(btg_nsplit(n, ncols) + 1) * BTG_K * ncols;
 }
 
 // T of every group of four panels into the workspace (independent of Z).
@@ -602,7 +531,7 @@ extern "C" hipError_t bse_apply_q_grouped_run(hipStream_t st, int n, int npan, i
     double2* tbig = ws + (int64_t)ng * 6 * BT_NB * BT_NB;
     double2* w2 = tbig + (int64_t)ng * BTG_K * BTG_K;
     double2* w1p = w2 + (int64_t)BTG_K * ncols;
-    const int ns = btg_nsplit(ncols);
+    const int ns = btg_nsplit(n, ncols);
     const unsigned c32 = (unsigned)ceil_div64(ncols, 32), c64 = (unsigned)ceil_div64(ncols, 64);
     for (int g = ng - 1; g >= 0; --g) {
         const int m = n - rb - g * BTG_K;
@@ -611,7 +540,7 @@ extern "C" hipError_t bse_apply_q_grouped_run(hipStream_t st, int n, int npan, i
         const int nsg = (int)ceil_div64(m, rchunk);
         hipLaunchKernelGGL(k_btg_w1, dim3(c32, nsg), dim3(256), 0, st, n, npan, rb, co, g, Vst, voff_d, Z, ldz,
                            ncols, rchunk, w1p);
-        hipLaunchKernelGGL(k_btg_w2, dim3(c32), dim3(256), 0, st, nsg, tbig + (int64_t)g * BTG_K * BTG_K, w1p, ncols,
+        hipLaunchKernelGGL(k_btg_w2, dim3((unsigned)ceil_div64(ncols, 16)), dim3(256), 0, st, nsg, tbig + (int64_t)g * BTG_K * BTG_K, w1p, ncols,
                            w2);
         hipLaunchKernelGGL(k_btg_upd, dim3(c64, (unsigned)ceil_div64(m, 64)), dim3(256), 0, st, n, npan, rb, co, g,
                            Vst, voff_d, w2, Z, ldz, ncols);
