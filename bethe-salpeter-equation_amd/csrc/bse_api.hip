@@ -1851,24 +1851,10 @@ extern "C" int bse_eigh_full(bse_ctx* ctx, int n_vectors) {
     double2* Linv = BUF(double2, S_LINV, (size_t)nt2 * 64 * 64);
     int* ferr = BUF(int, S_FERR, 4);
     HCK(bse_launch_zero_words(st, 2, ferr));
-    const int64_t pm = std::max<int64_t>(n2 - 64, 1);
-    double2* P = BUF(double2, S_FPAN, (size_t)pm * 64);
-    double2* Ph = BUF(double2, S_FPANH, (size_t)pm * 64);
-    double2* zeros = BUF(double2, S_BZERO, 64);
-    HCK(bse_launch_zero_words(st, 128, zeros));
-    const int kind = ctx->her2k_valu[0] >= 0 ? ctx->her2k_valu[0] : 1;
     HCK(hipEventRecord(ctx->tev[0], st));
     for (int J = 0; J < nt2; ++J) {
         HCK(bse_launch_potrf_tile(st, n2, J, M, Linv, ferr));
-        HCK(bse_launch_trsm_panel(st, n2, J, M, Linv, P, Ph));
-        const int s0 = (J + 1) * 64;
-        if (s0 < n2) {
-            const int m = n2 - s0;
-            // A22 -= P P^H as two rank-64 halves of P Ph^H + Ph P^H, Ph = P / 2
-            HCK(bse_launch_her2k(st, 0, kind, n2, s0, M, P, Ph, m, s0, 32, zeros));
-            HCK(bse_launch_her2k(st, 0, kind, n2, s0, M, P + (int64_t)32 * m, Ph + (int64_t)32 * m, m, s0, 32,
-                                 zeros));
-        }
+        HCK(bse_launch_chol_panel(st, n2, J, M, Linv));
     }
     int herr = 0;
     HCK(hipMemcpyAsync(&herr, ferr, sizeof(int), hipMemcpyDeviceToHost, st));

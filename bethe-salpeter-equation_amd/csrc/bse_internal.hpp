@@ -96,9 +96,9 @@ hipError_t bse_launch_expand_sym(hipStream_t, int64_t, int, int, const double2*,
                                  const int*);
 hipError_t bse_launch_compose_full(hipStream_t, int64_t, const double2*, const double2*, double2*);
 hipError_t bse_launch_potrf_tile(hipStream_t, int, int, double2*, double2*, int*);
-hipError_t bse_launch_trsm_panel(hipStream_t, int, int, double2*, const double2*, double2*, double2*);
+hipError_t bse_launch_chol_panel(hipStream_t, int, int, double2*, const double2*);
 hipError_t bse_launch_lsl(hipStream_t, int64_t, const double2*, double2*);
-hipError_t bse_launch_lower_solve(hipStream_t, int, const double2*, const double2*, const double2*, double2*);
+hipError_t bse_launch_lower_solve(hipStream_t, int, const double2*, const double2*, double2*, double2*);
 hipError_t bse_launch_upper_solve(hipStream_t, int, int, const double2*, const double2*, const double2*,
                                   int64_t, double2*, int64_t, const double*);
 hipError_t bse_launch_full_rho(hipStream_t, int64_t, const double2*, double2*, int64_t);
@@ -302,7 +302,7 @@ enum Slot {
     S_BTVOFF, S_BTWS,
     // full BSE: coupling block, M / its Cholesky factor, W = L^H s3 L, tile
     // inverses, panel, rho~, L^-1 rho~, eigenvectors, error flag, scales
-    S_BCPL, S_MFULL, S_WFULL, S_LINV, S_FPAN, S_FPANH, S_RHOT, S_ZT, S_XFULL, S_FERR, S_FSCALE, S_EVNEG,
+    S_BCPL, S_MFULL, S_WFULL, S_LINV, S_RHOT, S_ZT, S_XFULL, S_FERR, S_FSCALE, S_EVNEG,
     // RPA screening: window states at the grid points, Pi(Q)
     S_RPAEPS, S_RPACOEF, S_RPAPI,
     // Wannier position table (R, D_ij(R), Dq_ij(k)) and the real-space
