@@ -9,18 +9,24 @@
 // textbook/Hermitian form):
 //   H_rs = delta_rs dE_r + alpha sum_j Apair_{(k,k'),c,c',j} Vl_{k,v,j} conj(Vr_{k',v',j})
 //        + beta sum_j PVr_{r,j} conj(Pc_{s,j})
-// in the k-major order r = k*B + c*nv + v.  A workgroup owns TK k-points of
-// rows (TR = TK*B rows) and sweeps over all column tiles; each thread owns one
-// row and a residue class of columns and accumulates its share of Y in
-// registers, so the only LDS traffic is the tile's pair intermediates and the
-// X rows of the current column tile.
+// in the k-major order r = k*B + c*nv + v.  Workgroup (ti, g) owns TK k-points
+// of rows (TR = TK*B rows) and sweeps over the column tiles g, g + ncg, ...;
+// each thread owns one row and a residue class of columns and accumulates its
+// share of Y in registers, so the only LDS traffic is the tile's pair
+// intermediates and the X rows of the current column tile.  The row blocks
+// alone leave most of the chip idle (N = 1600 with one band pair: 50 of them),
+// so the columns are split until there are about AP_WG workgroups; the shares
+// go to Yp[g] and k_apply_add adds them to Y in the order of g.
+// 1600 rows, 16 vectors: 300 us unsplit, 55 us split.
 //
 // Trace mode (Bm != null, no vectors): instead of H X the kernel accumulates
 // tr(H Bm) = sum_rs H_rs Bm_sr over the same recomputed tiles and adds each
-// workgroup's share to tr_part[blockIdx.x] (fixed order, deterministic).
+// workgroup's share to tr_part[ti + nt g] (fixed order, deterministic).
 #include "bse_common.hpp"
+#include <algorithm>
 
 #define APPLY_KMAX 32   // vectors per pass
+#define AP_WG 512       // workgroups that the column split aims at
 
 struct ApplyArgs {
     int nk, n1, n2, n3, nv, nc, norb, TK, k;
@@ -36,6 +42,7 @@ struct ApplyArgs {
     double alpha, beta;
     const double2* X;
     double2* Y;
+    double2* Yp;         // column shares: [ncg][k][N]
     const double2* Bm;   // trace mode: N x N, ld ldb
     int64_t ldb;
     double2* tr_part;
@@ -83,7 +90,7 @@ __global__ __launch_bounds__(256) void k_apply(ApplyArgs a)
     for (int v = 0; v < APPLY_KMAX / 2; ++v) acc[v] = cmk(0, 0);
 
     const int nt = (int)ceil_div64(a.nk, TK);
-    for (int tj = 0; tj < nt; ++tj) {
+    for (int tj = blockIdx.y; tj < nt; tj += gridDim.y) {
         const int kp0 = tj * TK;
         __syncthreads();
         for (int e = tid; e < TK * a.nc * no; e += blockDim.x) {
@@ -172,7 +179,8 @@ __global__ __launch_bounds__(256) void k_apply(ApplyArgs a)
     if (a.Bm != nullptr) {
         __shared__ double sh[32];
         tacc = block_sum2(tacc, sh);
-        if (tid == 0) a.tr_part[blockIdx.x] = cadd(a.tr_part[blockIdx.x], tacc);
+        double2* tp = a.tr_part + blockIdx.x + (int64_t)gridDim.x * blockIdx.y;
+        if (tid == 0) *tp = cadd(*tp, tacc);
         return;
     }
     if (grp < ngrp && grow < a.N) {
@@ -180,10 +188,23 @@ __global__ __launch_bounds__(256) void k_apply(ApplyArgs a)
         for (int vi = 0; vi < APPLY_KMAX / 2; ++vi) {
             const int v = grp + vi * ngrp;
             if (v >= a.k) break;
-            double2* y = a.Y + grow + (int64_t)v * a.ldy;
-            *y = cadd(*y, acc[vi]);
+            a.Yp[((int64_t)blockIdx.y * a.k + v) * a.N + grow] = acc[vi];
         }
     }
+}
+
+// Y(:, v) += sum_g Yp[g](:, v): grid (row blocks, vectors).
+__global__ __launch_bounds__(256) void k_apply_add(int64_t N, int k, int ncg, const double2* __restrict__ Yp,
+                                                   double2* __restrict__ Y, int64_t ldy)
+{
+    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int v = blockIdx.y;
+    if (r >= N) return;
+    double2 s = cmk(0, 0);
+#pragma unroll 4
+    for (int g = 0; g < ncg; ++g) s = cadd(s, Yp[((int64_t)g * k + v) * N + r]);
+    double2* y = Y + r + (int64_t)v * ldy;
+    *y = cadd(*y, s);
 }
 
 static size_t apply_lds_elems(int TK, int nv, int nc, int norb, int k) {
@@ -204,29 +225,43 @@ extern "C" int bse_apply_pick_tk(int nv, int nc, int norb) {
     return tk;
 }
 
+// Column groups of the product, the workspace (complex elements) of a product
+// with k vectors and the partial sums of a trace.
+static int apply_groups(int nk, int TK) {
+    const int64_t nt = ceil_div64(nk, TK);
+    return (int)std::max<int64_t>(1, std::min<int64_t>(nt, ceil_div64(AP_WG, nt)));
+}
+extern "C" int64_t bse_apply_workspace(int nk, int nv, int nc, int TK, int k) {
+    return (int64_t)apply_groups(nk, TK) * nk * nv * nc * std::min(k, APPLY_KMAX);
+}
+extern "C" int bse_apply_trace_parts(int nk, int TK) { return (int)ceil_div64(nk, TK) * apply_groups(nk, TK); }
+
+// Y += H X (ws: bse_apply_workspace elements), or with Bm the shares of the
+// trace (tr_part: bse_apply_trace_parts entries, added to).
 extern "C" hipError_t bse_launch_apply(hipStream_t st, int nk, int n1, int n2, int n3, int nv, int nc,
                                        int norb, int TK, const double2* Cl, const double2* Cr,
                                        const double2* Vl, const double2* Vr, const double2* wtab,
                                        const double2* PVr, const double2* Pc, const double* dE,
                                        double alpha, double beta, int k, const double2* X,
                                        int64_t ldx, double2* Y, int64_t ldy, const double2* Bm,
-                                       int64_t ldb, double2* tr_part)
+                                       int64_t ldb, double2* tr_part, double2* ws)
 {
     ApplyArgs a;
     a.nk = nk; a.n1 = n1; a.n2 = n2; a.n3 = n3; a.nv = nv; a.nc = nc; a.norb = norb; a.TK = TK;
     a.N = (int64_t)nk * nv * nc;
     a.Cl = Cl; a.Cr = Cr; a.Vl = Vl; a.Vr = Vr; a.wtab = wtab; a.PVr = PVr; a.Pc = Pc; a.dE = dE;
     a.alpha = alpha; a.beta = beta;
-    const int TR = TK * nv * nc;
+    const int TR = TK * nv * nc, ncg = apply_groups(nk, TK);
+    const dim3 grid((unsigned)ceil_div64(nk, TK), (unsigned)ncg);
     // each of the 256/TR vector groups holds at most APPLY_KMAX/2 accumulators
     if (TR > 256 || (int64_t)APPLY_KMAX > (int64_t)(256 / TR) * (APPLY_KMAX / 2))
         return hipErrorInvalidValue;
-    a.Bm = Bm; a.ldb = ldb; a.tr_part = tr_part;
+    a.Bm = Bm; a.ldb = ldb; a.tr_part = tr_part; a.Yp = ws;
     if (Bm != nullptr) {
         if (tr_part == nullptr) return hipErrorInvalidValue;
         a.k = 0; a.X = nullptr; a.ldx = 0; a.Y = nullptr; a.ldy = 0;
         const size_t lds = apply_lds_elems(TK, nv, nc, norb, 0) * sizeof(double2);
-        hipLaunchKernelGGL(k_apply, dim3((unsigned)ceil_div64(nk, TK)), dim3(256), lds, st, a);
+        hipLaunchKernelGGL(k_apply, grid, dim3(256), lds, st, a);
         return hipGetLastError();
     }
     for (int v0 = 0; v0 < k; v0 += APPLY_KMAX) {
@@ -234,7 +269,9 @@ extern "C" hipError_t bse_launch_apply(hipStream_t st, int nk, int n1, int n2, i
         a.X = X + (int64_t)v0 * ldx; a.ldx = ldx;
         a.Y = Y + (int64_t)v0 * ldy; a.ldy = ldy;
         const size_t lds = apply_lds_elems(TK, nv, nc, norb, a.k) * sizeof(double2);
-        hipLaunchKernelGGL(k_apply, dim3((unsigned)ceil_div64(nk, TK)), dim3(256), lds, st, a);
+        hipLaunchKernelGGL(k_apply, grid, dim3(256), lds, st, a);
+        hipLaunchKernelGGL(k_apply_add, dim3((unsigned)ceil_div64(a.N, 256), (unsigned)a.k), dim3(256), 0, st, a.N,
+                           a.k, ncg, (const double2*)ws, a.Y, ldy);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

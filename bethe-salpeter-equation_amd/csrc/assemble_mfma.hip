@@ -108,6 +108,11 @@ struct MfArgs {
     const double2* P;
     const double* dE;
     double alpha, beta;
+    const double2* dcoef;      // derivative product: d coef / d theta
+    const double2* PV2;        // trace mode: second exchange factor pair
+    const double2* P2;
+    const double2* Bm;         // trace mode: N x N, ld ldb
+    int64_t ldb;
 };
 
 template <int PREC>
@@ -247,9 +252,20 @@ extern "C" int bse_assemble_mfma_supported(int nv, int nc, int norb);
 // the tile loop: k_apply_px / k_apply_pxsum form Z = P^H X (norb x k, fixed
 // summation order), and k_apply_sum adds, in a fixed order, the partials,
 // beta PV Z and the diagonal dE X.  Requires TR <= 64 (bse_assemble_mfma_tk).
+//
+// DER: the product with dH/dtheta for derivatives of the coefficients.  Both
+// contractions are linear in the pair products c c'^* and v v'^*, so the four
+// product-rule terms are one tile: with A' and N' the derivatives of the pair
+// products, (A' W) N + (A W) N', six contractions instead of the twelve of
+// four separate products, and the tile meets X once.
+// KG = 0: the trace tr(H Bm) of the same tiles (no X).  The tile's elements,
+// with the exchange factors and the diagonal added, are multiplied by Bm^T and
+// summed per workgroup into Yp[ti + nt g] (fixed order).
+// N = 2304 (4 + 4 bands): 4.9 ms per derivative (six products on the vector
+// units, one workgroup per 64 rows), 0.1 ms (product), 0.35 ms (trace) this way.
 // ---------------------------------------------------------------------------
 #define AM_K 32      // vectors per launch: KG groups of 16, one MFMA column block each
-template <int KG>
+template <int KG, bool DER>
 __global__ __launch_bounds__(256) void k_apply_mfma(MfArgs a, const double2* __restrict__ X, int64_t ldx, int k,
                                                     int ncg, double2* __restrict__ Yp)
 {
@@ -267,19 +283,24 @@ __global__ __launch_bounds__(256) void k_apply_mfma(MfArgs a, const double2* __r
     double* sHi = sHr + 64 * 65;
     double* sXr = sHi + 64 * 65;               // [64][KX]
     double* sXi = sXr + 64 * KX;
+    double2* sDr = (double2*)(sXi + 64 * KX);  // DER: [TK][ns][8] each
+    double2* sDc = sDr + TK * ns * 8;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     for (int e = tid; e < TK * ns * 8; e += 256) {
         const int i = e & 7, sl = (e >> 3) % ns, kk = e / (8 * ns);
         const int kq = k0 + kk;
         sCr[e] = (kq < a.nk && i < no) ? a.coef[((size_t)kq * ns + sl) * no + i] : cmk(0, 0);
+        if constexpr (DER) sDr[e] = (kq < a.nk && i < no) ? a.dcoef[((size_t)kq * ns + sl) * no + i] : cmk(0, 0);
     }
+    double2 tacc = cmk(0, 0);
     // rows and columns of the 64 x 64 LDS tile beyond TR stay zero
     for (int e = tid; e < 64 * 65; e += 256) { sHr[e] = 0.0; sHi[e] = 0.0; }
     double* tw = sT + wv * 272;
     const int li = lane & 15, lq = lane >> 4;
-    mf_d4 yr[KG], yi[KG];
+    constexpr int KA = KG > 0 ? KG : 1;
+    mf_d4 yr[KA], yi[KA];
 #pragma unroll
-    for (int q = 0; q < KG; ++q) { yr[q] = mf_d4{0, 0, 0, 0}; yi[q] = mf_d4{0, 0, 0, 0}; }
+    for (int q = 0; q < KA; ++q) { yr[q] = mf_d4{0, 0, 0, 0}; yi[q] = mf_d4{0, 0, 0, 0}; }
     for (int tj = g; tj < nt; tj += ncg) {
         const int kp0 = tj * TK;
         __syncthreads();   // previous tile fully consumed
@@ -287,9 +308,10 @@ __global__ __launch_bounds__(256) void k_apply_mfma(MfArgs a, const double2* __r
             const int i = e & 7, sl = (e >> 3) % ns, kk = e / (8 * ns);
             const int kp = kp0 + kk;
             sCc[e] = (kp < a.nk && i < no) ? a.coef[((size_t)kp * ns + sl) * no + i] : cmk(0, 0);
+            if constexpr (DER) sDc[e] = (kp < a.nk && i < no) ? a.dcoef[((size_t)kp * ns + sl) * no + i] : cmk(0, 0);
         }
         for (int e = tid; e < 64 * KX; e += 256) {
-            const int rr = e / KX, j = e % KX;
+            const int rr = e / (16 * KA), j = e % (16 * KA);
             const int64_t col = (int64_t)kp0 * B + rr;
             double2 x = cmk(0, 0);
             if (rr < TR && col < a.N && j < k) x = X[col + (int64_t)j * ldx];
@@ -302,17 +324,21 @@ __global__ __launch_bounds__(256) void k_apply_mfma(MfArgs a, const double2* __r
             const int kx = k0 + kk, kp = kp0 + kq;
             const bool pok = kx < a.nk && kp < a.nk;
             const double2* wq = a.wtab + (pok ? (size_t)ktable_index(kx, kp, a.n1, a.n2, a.n3) * no * no : 0);
-            double a1[4], b1[4];
+            double a1[4], b1[4], a1d[4];
             const int rho = li, c = rho / a.nc, cp = rho % a.nc;
             const bool rok = rho < a.nc * a.nc;
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
                 const int kap = 4 * ks + lq;
                 const int i = kap & 7;
-                double2 x = cmk(0, 0);
-                if (pok && rok && i < no)
-                    x = cmulc(sCr[(kk * ns + a.nv + c) * 8 + i], sCc[(kq * ns + a.nv + cp) * 8 + i]);
+                double2 x = cmk(0, 0), xd = cmk(0, 0);
+                if (pok && rok && i < no) {
+                    const int er = (kk * ns + a.nv + c) * 8 + i, ec = (kq * ns + a.nv + cp) * 8 + i;
+                    x = cmulc(sCr[er], sCc[ec]);
+                    if constexpr (DER) xd = cadd(cmulc(sDr[er], sCc[ec]), cmulc(sCr[er], sDc[ec]));
+                }
                 a1[ks] = kap < 8 ? x.x : x.y;
+                if constexpr (DER) a1d[ks] = kap < 8 ? xd.x : xd.y;
                 const int jp = li;
                 const int jj = jp & 7, ii = kap & 7;
                 double wv2 = 0.0;
@@ -334,20 +360,49 @@ __global__ __launch_bounds__(256) void k_apply_mfma(MfArgs a, const double2* __r
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) a2[ks] = tw[li * 17 + 4 * ks + lq];
             __builtin_amdgcn_wave_barrier();
+            double a2d[4], b3r[4], b3i[4];
+            if constexpr (DER) {
+                const mf_d4 d1d = mm16(a1d, b1, mf_d4{0, 0, 0, 0});
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+                for (int reg = 0; reg < 4; ++reg) tw[mfma16_row_f64(lane, reg) * 17 + li] = d1d[reg];
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks) a2d[ks] = tw[li * 17 + 4 * ks + lq];
+                __builtin_amdgcn_wave_barrier();
+            }
             const int sg = li, v = sg / a.nv, vp = sg % a.nv;
             const bool sok = sg < a.nv * a.nv;
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
                 const int kap = 4 * ks + lq;
                 const int j = kap & 7;
-                double2 y = cmk(0, 0);
-                if (pok && sok && j < no)
-                    y = cmul(sCr[(kk * ns + v) * 8 + j], cconj(sCc[(kq * ns + vp) * 8 + j]));
+                double2 y = cmk(0, 0), yd = cmk(0, 0);
+                if (pok && sok && j < no) {
+                    const int er = (kk * ns + v) * 8 + j, ec = (kq * ns + vp) * 8 + j;
+                    y = cmul(sCr[er], cconj(sCc[ec]));
+                    if constexpr (DER) yd = cadd(cmul(sDr[er], cconj(sCc[ec])), cmul(sCr[er], cconj(sDc[ec])));
+                }
                 b2r[ks] = kap < 8 ? y.x : -y.y;
                 b2i[ks] = kap < 8 ? y.y : y.x;
+                if constexpr (DER) {
+                    b3r[ks] = kap < 8 ? yd.x : -yd.y;
+                    b3i[ks] = kap < 8 ? yd.y : yd.x;
+                }
             }
-            const mf_d4 dr = mm16(a2, b2r, mf_d4{0, 0, 0, 0});
-            const mf_d4 di = mm16(a2, b2i, mf_d4{0, 0, 0, 0});
+            mf_d4 dr = mf_d4{0, 0, 0, 0}, di = mf_d4{0, 0, 0, 0};
+            if constexpr (DER) {
+                dr = mm16(a2, b3r, dr);
+                di = mm16(a2, b3i, di);
+                dr = mm16(a2d, b2r, dr);
+                di = mm16(a2d, b2i, di);
+            } else {
+                dr = mm16(a2, b2r, dr);
+                di = mm16(a2, b2i, di);
+            }
 #pragma unroll
             for (int reg = 0; reg < 4; ++reg) {
                 const int rh = mfma16_row_f64(lane, reg);
@@ -365,11 +420,29 @@ __global__ __launch_bounds__(256) void k_apply_mfma(MfArgs a, const double2* __r
             }
         }
         __syncthreads();
+        if constexpr (KG == 0) {
+            for (int e = tid; e < TR * TR; e += 256) {
+                const int cl = e % TR, rl = e / TR;
+                const int64_t gr = (int64_t)k0 * B + rl, gc = (int64_t)kp0 * B + cl;
+                if (gr >= a.N || gc >= a.N) continue;
+                double2 h = cmk(sHr[rl * 65 + cl], sHi[rl * 65 + cl]);
+                if (a.PV != nullptr) {
+                    double2 x = cmk(0, 0);
+                    for (int j = 0; j < no; ++j) {
+                        cfma(x, a.PV[gr * no + j], cconj(a.P[gc * no + j]));
+                        cfma(x, a.PV2[gr * no + j], cconj(a.P2[gc * no + j]));
+                    }
+                    h = cadd(h, cscale(x, a.beta));
+                }
+                if (gr == gc && a.dE != nullptr) h.x += a.dE[gr];
+                cfma(tacc, h, a.Bm[gc + gr * a.ldb]);
+            }
+        }
         // Y rows 16 wv .. 16 wv + 15 += H(rows, 0:64) X(0:64, 0:KX), one H
         // tile formed for all KX vectors
         const int hr0 = (16 * wv + li) * 65;
 #pragma unroll 4
-        for (int kc = 0; kc < 64; kc += 4) {
+        for (int kc = 0; kc < (KG > 0 ? 64 : 0); kc += 4) {
             const double hr = sHr[hr0 + kc + lq], hi = sHi[hr0 + kc + lq];
 #pragma unroll
             for (int q = 0; q < KG; ++q) {
@@ -380,6 +453,11 @@ __global__ __launch_bounds__(256) void k_apply_mfma(MfArgs a, const double2* __r
                 yi[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(hi, xr, yi[q], 0, 0, 0);
             }
         }
+    }
+    if constexpr (KG == 0) {
+        tacc = block_sum2(tacc, sT);
+        if (tid == 0) Yp[ti + (int64_t)nt * g] = tacc;
+        return;
     }
     // lane holds Y[row 16 wv + mfma16_row_f64(lane, reg)][vector 16 q + li]
 #pragma unroll
@@ -417,11 +495,15 @@ __global__ __launch_bounds__(256) void k_apply_pxsum(int G, const double2* __res
     Z[threadIdx.x] = z;
 }
 
-// Y(r, j) = sum_g Yp[g](r, j) + beta sum_i PV(r, i) Z(i, j) + dE(r) X(r, j).
+// Y(r, j) = sum_g Yp[g](r, j) + beta sum_i PV(r, i) Z(i, j) + dE(r) X(r, j),
+// with a second pair PV2, Z2 of the exchange when PV2 is given; no exchange
+// when PV is null, no diagonal when dE is null.
 __global__ __launch_bounds__(256) void k_apply_sum(int64_t N, int k, int ncg, int no,
                                                    const double2* __restrict__ Yp,
                                                    const double2* __restrict__ PV,
-                                                   const double2* __restrict__ Z, const double* __restrict__ dE,
+                                                   const double2* __restrict__ Z,
+                                                   const double2* __restrict__ PV2,
+                                                   const double2* __restrict__ Z2, const double* __restrict__ dE,
                                                    double beta, const double2* __restrict__ X, int64_t ldx,
                                                    double2* __restrict__ Y, int64_t ldy)
 {
@@ -433,17 +515,19 @@ __global__ __launch_bounds__(256) void k_apply_sum(int64_t N, int k, int ncg, in
     double2 s = cmk(0, 0);
     for (int gg = 0; gg < ncg; ++gg) s = cadd(s, Yp[(int64_t)gg * N * AM_K + e]);
     double2 x = cmk(0, 0);
-    for (int i = 0; i < no; ++i) cfma(x, PV[r * no + i], Z[i + 8 * j]);
+    if (PV != nullptr)
+        for (int i = 0; i < no; ++i) cfma(x, PV[r * no + i], Z[i + 8 * j]);
+    if (PV2 != nullptr)
+        for (int i = 0; i < no; ++i) cfma(x, PV2[r * no + i], Z2[i + 8 * j]);
     const double2 xr = X[r + (int64_t)j * ldx];
     s = cadd(s, cscale(x, beta));
-    s = cadd(s, cscale(xr, dE[r]));
+    if (dE != nullptr) s = cadd(s, cscale(xr, dE[r]));
     Y[r + (int64_t)j * ldy] = s;
 }
 
-static size_t apply_mfma_lds_bytes(int TK, int nv, int nc, int kg) {
-    const int ns = nv + nc, B = nv * nc;
-    (void)B;
-    return ((size_t)2 * TK * ns * 8) * sizeof(double2) +
+static size_t apply_mfma_lds_bytes(int TK, int nv, int nc, int kg, bool der) {
+    const int ns = nv + nc;
+    return ((size_t)(der ? 4 : 2) * TK * ns * 8) * sizeof(double2) +
            ((size_t)4 * 272 + 2 * 64 * 65 + 2 * 64 * 16 * kg) * sizeof(double);
 }
 
@@ -454,49 +538,95 @@ extern "C" int bse_apply_mfma_groups(int nk, int nv, int nc) {
     return (int)std::max<int64_t>(1, std::min<int64_t>(nt, ceil_div64(1024, nt)));
 }
 extern "C" int64_t bse_apply_mfma_workspace(int nk, int nv, int nc) {
-    return (int64_t)bse_apply_mfma_groups(nk, nv, nc) * nk * nv * nc * AM_K + (APX_BLOCKS + 1) * 256;
+    return (int64_t)bse_apply_mfma_groups(nk, nv, nc) * nk * nv * nc * AM_K + (APX_BLOCKS + 2) * 256;
+}
+// Partial sums of the trace.
+extern "C" int bse_trace_mfma_parts(int nk, int nv, int nc) {
+    return (int)ceil_div64(nk, bse_assemble_mfma_tk(nv, nc)) * bse_apply_mfma_groups(nk, nv, nc);
 }
 
-extern "C" hipError_t bse_launch_apply_mfma(hipStream_t st, int nk, int n1, int n2, int n3, int nv, int nc,
-                                            int norb, const double2* coef, const double2* wtab,
-                                            const double2* PV, const double2* P, const double* dE,
-                                            double alpha, double beta, int k, const double2* X,
-                                            int64_t ldx, double2* Y, int64_t ldy, double2* ws)
+template <int KG, bool DER>
+static hipError_t apply_mfma_tiles(hipStream_t st, const MfArgs& a, int k, const double2* X, int64_t ldx,
+                                   double2* out)
 {
-    if (!bse_assemble_mfma_supported(nv, nc, norb) || k <= 0 || k > AM_K) return hipErrorInvalidValue;
-    MfArgs a;
+    // the LDS beyond 64 KB is asked for explicitly (once per process)
+    static const hipError_t attr = hipFuncSetAttribute((const void*)k_apply_mfma<KG, DER>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 1024);
+    if (attr != hipSuccess) return attr;
+    const int nt = (int)ceil_div64(a.nk, a.TK), ncg = bse_apply_mfma_groups(a.nk, a.nv, a.nc);
+    hipLaunchKernelGGL((k_apply_mfma<KG, DER>), dim3((unsigned)nt, (unsigned)ncg), dim3(256),
+                       apply_mfma_lds_bytes(a.TK, a.nv, a.nc, KG, DER), st, a, X, ldx, k, ncg, out);
+    return hipGetLastError();
+}
+
+static hipError_t apply_mfma_args(MfArgs& a, int nk, int n1, int n2, int n3, int nv, int nc, int norb,
+                                  const double2* coef, const double2* dcoef, const double2* wtab, double alpha,
+                                  double beta)
+{
+    if (!bse_assemble_mfma_supported(nv, nc, norb)) return hipErrorInvalidValue;
+    a = MfArgs{};
     a.nk = nk; a.n1 = n1; a.n2 = n2; a.n3 = n3; a.nv = nv; a.nc = nc; a.norb = norb;
     a.TK = bse_assemble_mfma_tk(nv, nc);
     if (a.TK * nv * nc > 64) return hipErrorInvalidValue;
     a.N = (int64_t)nk * nv * nc;
     a.nt = tile_count(a.N);
-    a.coef = coef; a.wtab = wtab; a.PV = PV; a.P = P; a.dE = dE; a.alpha = alpha; a.beta = beta;
-    const int nt = (int)ceil_div64(nk, a.TK);
+    a.coef = coef; a.dcoef = dcoef; a.wtab = wtab; a.alpha = alpha; a.beta = beta;
+    return hipSuccess;
+}
+
+// Y = H X for k <= 32 vectors.  With dcoef the direct term is its derivative
+// along dcoef; PV P^H and PV2 P2^H are the exchange (either may be null), dE
+// the diagonal (may be null).
+extern "C" hipError_t bse_launch_apply_mfma(hipStream_t st, int nk, int n1, int n2, int n3, int nv, int nc,
+                                            int norb, const double2* coef, const double2* dcoef,
+                                            const double2* wtab, const double2* PV, const double2* P,
+                                            const double2* PV2, const double2* P2, const double* dE,
+                                            double alpha, double beta, int k, const double2* X,
+                                            int64_t ldx, double2* Y, int64_t ldy, double2* ws)
+{
+    if (k <= 0 || k > AM_K) return hipErrorInvalidValue;
+    MfArgs a;
+    hipError_t e = apply_mfma_args(a, nk, n1, n2, n3, nv, nc, norb, coef, dcoef, wtab, alpha, beta);
+    if (e != hipSuccess) return e;
     const int ncg = bse_apply_mfma_groups(nk, nv, nc);
-    const int kg = k > 16 ? 2 : 1;
-    const size_t lds = apply_mfma_lds_bytes(a.TK, nv, nc, kg);
     double2* Zp = ws + (int64_t)ncg * a.N * AM_K;   // exchange: Z = P^H X
     double2* Z = Zp + (int64_t)APX_BLOCKS * 256;
-    hipLaunchKernelGGL(k_apply_px, dim3(APX_BLOCKS), dim3(256), 0, st, a.N, norb, k, P, X, ldx, Zp);
-    hipLaunchKernelGGL(k_apply_pxsum, dim3(1), dim3(256), 0, st, APX_BLOCKS, (const double2*)Zp, Z);
-    // the LDS beyond 64 KB is asked for explicitly (once per process)
-    static const hipError_t attr = [] {
-        const int big = 160 * 1024 - 1024;
-        hipError_t e = hipFuncSetAttribute((const void*)k_apply_mfma<1>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void*)k_apply_mfma<2>, hipFuncAttributeMaxDynamicSharedMemorySize, big);
-        return e;
-    }();
-    if (attr != hipSuccess) return attr;
-    if (kg == 2)
-        hipLaunchKernelGGL(k_apply_mfma<2>, dim3((unsigned)nt, (unsigned)ncg), dim3(256), lds, st, a, X, ldx, k,
-                           ncg, ws);
+    double2* Z2 = Z + 256;
+    if (PV != nullptr) {
+        hipLaunchKernelGGL(k_apply_px, dim3(APX_BLOCKS), dim3(256), 0, st, a.N, norb, k, P, X, ldx, Zp);
+        hipLaunchKernelGGL(k_apply_pxsum, dim3(1), dim3(256), 0, st, APX_BLOCKS, (const double2*)Zp, Z);
+    }
+    if (PV2 != nullptr) {
+        hipLaunchKernelGGL(k_apply_px, dim3(APX_BLOCKS), dim3(256), 0, st, a.N, norb, k, P2, X, ldx, Zp);
+        hipLaunchKernelGGL(k_apply_pxsum, dim3(1), dim3(256), 0, st, APX_BLOCKS, (const double2*)Zp, Z2);
+    }
+    if (k > 16)
+        e = dcoef ? apply_mfma_tiles<2, true>(st, a, k, X, ldx, ws) : apply_mfma_tiles<2, false>(st, a, k, X, ldx, ws);
     else
-        hipLaunchKernelGGL(k_apply_mfma<1>, dim3((unsigned)nt, (unsigned)ncg), dim3(256), lds, st, a, X, ldx, k,
-                           ncg, ws);
+        e = dcoef ? apply_mfma_tiles<1, true>(st, a, k, X, ldx, ws) : apply_mfma_tiles<1, false>(st, a, k, X, ldx, ws);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_apply_sum, dim3((unsigned)ceil_div64(a.N * AM_K, 256)), dim3(256), 0, st, a.N, k,
-                       ncg, norb, (const double2*)ws, PV, (const double2*)Z, dE, beta, X, ldx, Y, ldy);
+                       ncg, norb, (const double2*)ws, PV, (const double2*)Z, PV2, (const double2*)Z2, dE, beta, X,
+                       ldx, Y, ldy);
     return hipGetLastError();
+}
+
+// tr(H Bm) into bse_trace_mfma_parts partial sums; arguments as above (PV and
+// PV2 both given or both null).
+extern "C" hipError_t bse_launch_trace_mfma(hipStream_t st, int nk, int n1, int n2, int n3, int nv, int nc,
+                                            int norb, const double2* coef, const double2* dcoef,
+                                            const double2* wtab, const double2* PV, const double2* P,
+                                            const double2* PV2, const double2* P2, const double* dE,
+                                            double alpha, double beta, const double2* Bm, int64_t ldb,
+                                            double2* part)
+{
+    MfArgs a;
+    hipError_t e = apply_mfma_args(a, nk, n1, n2, n3, nv, nc, norb, coef, dcoef, wtab, alpha, beta);
+    if (e != hipSuccess) return e;
+    if ((PV == nullptr) != (PV2 == nullptr) || Bm == nullptr) return hipErrorInvalidValue;
+    a.PV = PV; a.P = P; a.PV2 = PV2; a.P2 = P2; a.dE = dE; a.Bm = Bm; a.ldb = ldb;
+    return dcoef ? apply_mfma_tiles<0, true>(st, a, 0, nullptr, 0, part)
+                 : apply_mfma_tiles<0, false>(st, a, 0, nullptr, 0, part);
 }
 
 extern "C" int bse_assemble_mfma_supported(int nv, int nc, int norb) {

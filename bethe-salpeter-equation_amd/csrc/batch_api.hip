@@ -43,7 +43,7 @@ struct SysDev {
     int2* clusters;
     double *iiscr, *iix;
     double2 *y, *f, *Z;
-    double2 *RS, *RHS, *RX, *RG, *RHG, *RC, *skw;
+    double2 *RS, *RHS, *RX, *RG, *RHG, *RC, *skw, *apw;
     double* small;
     int64_t sk_el;
     double* eps_out;     // re (n_omega) | im (n_omega)
@@ -167,6 +167,8 @@ void carve(Bump& bp, const SysHost& h, int fp32, int nlow, int n_omega, SysDev& 
     d.small = bp.take<double>(4 * (size_t)nlow + 8);
     d.sk_el = (int64_t)64 * m * m;
     d.skw = bp.take<double2>(d.sk_el);
+    d.apw = bp.take<double2>(bse_apply_workspace(g.nk, g.sys.nv, g.sys.nc,
+                                                 bse_apply_pick_tk(g.sys.nv, g.sys.nc, no), nlow));
     d.eps_out = bp.take<double>(2 * (size_t)std::max(n_omega, 1));
     d.evals_out = bp.take<double>(nlow);
 }
@@ -224,7 +226,7 @@ static hipError_t record_apply(BatchState* b, int s, hipStream_t st, int k, cons
     if ((e = bse_launch_zero_words(st, 2 * g.N * k, Y))) return e;
     return bse_launch_apply(st, g.nk, sy.n1, sy.n2, g.n3, sy.nv, sy.nc, g.norb,
                             bse_apply_pick_tk(sy.nv, sy.nc, g.norb), d.coef, d.coef, d.coef, d.coef,
-                            d.wtab, d.PV, d.P, d.dE, alpha, beta, k, X, g.N, Y, g.N, nullptr, 0, nullptr);
+                            d.wtab, d.PV, d.P, d.dE, alpha, beta, k, X, g.N, Y, g.N, nullptr, 0, nullptr, d.apw);
 }
 
 // Per-system work after the reduction: tridiagonal eigenpairs, oscillator

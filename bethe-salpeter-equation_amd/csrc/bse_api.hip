@@ -1400,20 +1400,23 @@ static int apply_H(bse_ctx* ctx, int k, const double2* X, int64_t ldx, double2* 
         double2* ws = BUF(double2, S_APPLYP, bse_apply_mfma_workspace(ctx->nk, s.nv, s.nc));
         for (int c0 = 0; c0 < k; c0 += 32) {
             const int kc = std::min(32, k - c0);
-            HCK(bse_launch_apply_mfma(ctx->st, ctx->nk, s.n1, s.n2, ctx->n3, s.nv, s.nc, ctx->norb, coef,
+            HCK(bse_launch_apply_mfma(ctx->st, ctx->nk, s.n1, s.n2, ctx->n3, s.nv, s.nc, ctx->norb, coef, nullptr,
                                       (const double2*)ctx->bufs[S_WTAB].p, (const double2*)ctx->bufs[S_PV].p,
-                                      (const double2*)ctx->bufs[S_P].p, (const double*)ctx->bufs[S_DE].p,
+                                      (const double2*)ctx->bufs[S_P].p, nullptr, nullptr,
+                                      (const double*)ctx->bufs[S_DE].p,
                                       alpha, beta, kc, X + (int64_t)c0 * ldx, ldx, Y + (int64_t)c0 * ldy,
                                       ldy, ws));
         }
         return BSE_OK;
     }
+    const int tk = bse_apply_pick_tk(s.nv, s.nc, ctx->norb);
+    double2* ws = BUF(double2, S_APPLYP, bse_apply_workspace(ctx->nk, s.nv, s.nc, tk, k));
     HCK(hipMemsetAsync(Y, 0, sizeof(double2) * ldy * k, ctx->st));
     HCK(bse_launch_apply(ctx->st, ctx->nk, s.n1, s.n2, ctx->n3, s.nv, s.nc, ctx->norb,
-                         bse_apply_pick_tk(s.nv, s.nc, ctx->norb), coef, coef, coef, coef,
+                         tk, coef, coef, coef, coef,
                          (const double2*)ctx->bufs[S_WTAB].p, (const double2*)ctx->bufs[S_PV].p,
                          (const double2*)ctx->bufs[S_P].p, (const double*)ctx->bufs[S_DE].p, alpha,
-                         beta, k, X, ldx, Y, ldy, nullptr, 0, nullptr));
+                         beta, k, X, ldx, Y, ldy, nullptr, 0, nullptr, ws));
     return BSE_OK;
 }
 
@@ -1537,6 +1540,41 @@ extern "C" int bse_apply(bse_ctx* ctx, int k, const double* x, int64_t ldx, doub
 // energies and coefficients (parallel-transport gauge); the gauge part of dc
 // drops out of A^H dH A.
 // ---------------------------------------------------------------------------
+// The product Y = dH A (k vectors) or the trace tr(dH Bm) of one derivative on
+// matrix cores: arguments as for bse_launch_apply_mfma.
+static int grad_apply_mfma(bse_ctx* ctx, const double2* dcoef, const double2* wtab, const double2* PV,
+                           const double2* P, const double2* PV2, const double2* P2, const double* dE, int k,
+                           const double2* A, double2* Y, const double2* Bm, double2* trp) {
+    const bse_system& s = ctx->sys;
+    const int64_t N = ctx->N;
+    const double2* coef = (const double2*)ctx->bufs[S_COEF].p;
+    const double alpha = -s.direct_scale / (ctx->cell * ctx->nk);
+    const double beta = s.f_s * s.exchange_scale / (ctx->cell * ctx->nk);
+    if (Bm) {
+        HCK(bse_launch_trace_mfma(ctx->st, ctx->nk, s.n1, s.n2, ctx->n3, s.nv, s.nc, ctx->norb, coef, dcoef, wtab,
+                                  PV, P, PV2, P2, dE, alpha, beta, Bm, N, trp));
+        return BSE_OK;
+    }
+    double2* ws = BUF(double2, S_APPLYP, bse_apply_mfma_workspace(ctx->nk, s.nv, s.nc));
+    for (int c0 = 0; c0 < k; c0 += 32)
+        HCK(bse_launch_apply_mfma(ctx->st, ctx->nk, s.n1, s.n2, ctx->n3, s.nv, s.nc, ctx->norb, coef, dcoef, wtab,
+                                  PV, P, PV2, P2, dE, alpha, beta, std::min(32, k - c0), A + c0 * N, N, Y + c0 * N,
+                                  N, ws));
+    return BSE_OK;
+}
+
+// The matrix-core product covers a system's shape (else the general one).
+static bool grad_on_mfma(const bse_ctx* ctx) {
+    return !ctx->force_valu_assembly && bse_assemble_mfma_supported(ctx->sys.nv, ctx->sys.nc, ctx->norb);
+}
+
+// Partial sums that a derivative's trace leaves.
+static int grad_trace_parts(const bse_ctx* ctx) {
+    const bse_system& s = ctx->sys;
+    if (grad_on_mfma(ctx)) return bse_trace_mfma_parts(ctx->nk, s.nv, s.nc);
+    return bse_apply_trace_parts(ctx->nk, bse_apply_pick_tk(s.nv, s.nc, ctx->norb));
+}
+
 static int grad_tb_apply(bse_ctx* ctx, int which, int k, const double2* A, double2* Y,
                          const double2* Bm = nullptr, double2* trp = nullptr) {
     const bse_system& s = ctx->sys;
@@ -1577,22 +1615,26 @@ static int grad_tb_apply(bse_ctx* ctx, int which, int k, const double2* A, doubl
                                ctx->dip_nr > 0 ? (const double2*)ctx->bufs[S_DIPQ].p : nullptr));
     const double2* coef = (const double2*)ctx->bufs[S_COEF].p;
     const double2* wt = (const double2*)ctx->bufs[S_WTAB].p;
+    if (grad_on_mfma(ctx))
+        return grad_apply_mfma(ctx, dcoef, wt, dPV, (const double2*)ctx->bufs[S_P].p,
+                               (const double2*)ctx->bufs[S_PV].p, dP, ddE, k, A, Y, Bm, trp);
     const double alpha = -s.direct_scale / (ctx->cell * ctx->nk);
     const double beta = s.f_s * s.exchange_scale / (ctx->cell * ctx->nk);
     const int tk = bse_apply_pick_tk(s.nv, s.nc, no);
+    double2* ws = Bm ? nullptr : BUF(double2, S_APPLYP, bse_apply_workspace(ctx->nk, s.nv, s.nc, tk, k));
     if (!Bm) HCK(hipMemsetAsync(Y, 0, sizeof(double2) * ctx->N * k, ctx->st));
     const double2* fac[4][4] = {{dcoef, coef, coef, coef}, {coef, dcoef, coef, coef},
                                 {coef, coef, dcoef, coef}, {coef, coef, coef, dcoef}};
     for (int t = 0; t < 4; ++t)
         HCK(bse_launch_apply(ctx->st, ctx->nk, s.n1, s.n2, ctx->n3, s.nv, s.nc, no, tk, fac[t][0], fac[t][1],
                              fac[t][2], fac[t][3], wt, nullptr, nullptr, nullptr, alpha, 0.0, k, A,
-                             ctx->N, Y, ctx->N, Bm, ctx->N, trp));
+                             ctx->N, Y, ctx->N, Bm, ctx->N, trp, ws));
     // exchange: beta (dP V P^H + P V dP^H); diagonal d(eps_c - eps_v)
     HCK(bse_launch_apply(ctx->st, ctx->nk, s.n1, s.n2, ctx->n3, s.nv, s.nc, no, tk, coef, coef, coef, coef, wt,
-                         dPV, (const double2*)ctx->bufs[S_P].p, ddE, 0.0, beta, k, A, ctx->N, Y, ctx->N, Bm, ctx->N, trp));
+                         dPV, (const double2*)ctx->bufs[S_P].p, ddE, 0.0, beta, k, A, ctx->N, Y, ctx->N, Bm, ctx->N, trp, ws));
     HCK(bse_launch_apply(ctx->st, ctx->nk, s.n1, s.n2, ctx->n3, s.nv, s.nc, no, tk, coef, coef, coef, coef, wt,
                          (const double2*)ctx->bufs[S_PV].p, dP, nullptr, 0.0, beta, k, A, ctx->N, Y,
-                         ctx->N, Bm, ctx->N, trp));
+                         ctx->N, Bm, ctx->N, trp, ws));
     return BSE_OK;
 }
 
@@ -1619,12 +1661,16 @@ static int grad_w_apply(bse_ctx* ctx, int which, int k, const double2* A, double
                            (const double*)ctx->bufs[S_GVEC].p, ctx->recip,
                            (const double*)ctx->bufs[S_TAU].p, s.r0, s.eps_env, s.radius, kC, dwbar,
                            which == 2 ? 1 : 2, dW));
+    if (grad_on_mfma(ctx))
+        return grad_apply_mfma(ctx, nullptr, dW, nullptr, nullptr, nullptr, nullptr, nullptr, k, A, Y, Bm, trp);
     const double2* coef = (const double2*)ctx->bufs[S_COEF].p;
     const double alpha = -s.direct_scale / (ctx->cell * ctx->nk);
+    const int tk = bse_apply_pick_tk(s.nv, s.nc, no);
+    double2* ws = Bm ? nullptr : BUF(double2, S_APPLYP, bse_apply_workspace(ctx->nk, s.nv, s.nc, tk, k));
     if (!Bm) HCK(hipMemsetAsync(Y, 0, sizeof(double2) * ctx->N * k, ctx->st));
     HCK(bse_launch_apply(ctx->st, ctx->nk, s.n1, s.n2, ctx->n3, s.nv, s.nc, no,
-                         bse_apply_pick_tk(s.nv, s.nc, no), coef, coef, coef, coef, dW, nullptr,
-                         nullptr, nullptr, alpha, 0.0, k, A, ctx->N, Y, ctx->N, Bm, ctx->N, trp));
+                         tk, coef, coef, coef, coef, dW, nullptr,
+                         nullptr, nullptr, alpha, 0.0, k, A, ctx->N, Y, ctx->N, Bm, ctx->N, trp, ws));
     return BSE_OK;
 }
 
@@ -1714,8 +1760,7 @@ extern "C" int bse_grad_spectrum(bse_ctx* ctx, const double* omega, int n_omega,
     HCK(bse_zgemm(st, 0, 0, (int)N, nw, (int)N, 1, 0, A, N, Fac, N, 0, 0, U, N, nullptr, 0));
     HCK(bse_zgemm(st, 0, 1, (int)N, (int)N, nw, 1, 0, Xr, N, U, N, 0, 0, Bm, N, nullptr, 0));
     HCK(bse_zgemm(st, 0, 0, (int)N, 1, (int)N, 1, 0, A, N, sb, N, 0, 0, p1, N, nullptr, 0));
-    const int tk = bse_apply_pick_tk(ctx->sys.nv, ctx->sys.nc, ctx->norb);
-    const int nblk = (int)ceil_div64(ctx->nk, tk);
+    const int nblk = grad_trace_parts(ctx);
     double2* part = BUF(double2, S_SGPART, std::max(nblk, 1));
     std::vector<double2> hpart(std::max(nblk, 1));
     std::vector<double2> hv(3 * (size_t)N);

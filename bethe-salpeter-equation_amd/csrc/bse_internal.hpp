@@ -166,8 +166,13 @@ int bse_assemble_mfma_supported(int, int, int);
 int bse_apply_mfma_groups(int, int, int);
 int64_t bse_apply_mfma_workspace(int, int, int);
 hipError_t bse_launch_apply_mfma(hipStream_t, int, int, int, int, int, int, int, const double2*, const double2*,
-                                 const double2*, const double2*, const double*, double, double, int,
-                                 const double2*, int64_t, double2*, int64_t, double2*);
+                                 const double2*, const double2*, const double2*, const double2*, const double2*,
+                                 const double*, double, double, int, const double2*, int64_t, double2*, int64_t,
+                                 double2*);
+int bse_trace_mfma_parts(int, int, int);
+hipError_t bse_launch_trace_mfma(hipStream_t, int, int, int, int, int, int, int, const double2*, const double2*,
+                                 const double2*, const double2*, const double2*, const double2*, const double2*,
+                                 const double*, double, double, const double2*, int64_t, double2*);
 hipError_t bse_launch_assemble_mfma(hipStream_t, int, int, int, int, int, int, int, int, int64_t,
                                     const double2*, const double2*, const double2*, const double2*,
                                     const double*, double, double, void*);
@@ -175,7 +180,9 @@ hipError_t bse_launch_apply(hipStream_t, int, int, int, int, int, int, int, int,
                             const double2*, const double2*, const double2*, const double2*,
                             const double2*, const double2*, const double*, double, double, int,
                             const double2*, int64_t, double2*, int64_t, const double2*, int64_t,
-                            double2*);
+                            double2*, double2*);
+int64_t bse_apply_workspace(int, int, int, int, int);
+int bse_apply_trace_parts(int, int);
 hipError_t bse_launch_small_rr(hipStream_t, int, int, const double2*, const double2*, double,
                                double*, double2*, int*);
 hipError_t bse_launch_residual(hipStream_t, int64_t, int, const double2*, const double2*, int64_t,
