@@ -695,7 +695,26 @@ static bool use_two_stage(const bse_ctx* ctx, int n, int n_vectors, int max_vect
     return ctx->two_stage > 0 || n >= (fp32 ? 4096 : 256);
 }
 
-static int twostage_tridiag(bse_ctx* ctx, int n, void* H, int fp32, const double2* rho) {
+// Many vectors by two stages: the chase's reflectors are kept (n^2 / 2 complex
+// numbers) and applied to the tridiagonal vectors.  FP64 storage, from order
+// kQ2MinN, where the one-stage reduction's time a column outgrows the second
+// back-transform (reduction and vectors, all of them, one stage and two: n =
+// 2600 43.3 and 49.8 ms, 3200 65.1 and 66.2, 3500 79.6 and 77.4, 4000 105.6 and
+// 95.7, 8096 580 and 410; 64 of them: 3200 58.8 and 59.5, 3500 70.9 and 68.8).
+static const int kQ2MinN = 3400;
+static bool use_q2(const bse_ctx* ctx, int n, int n_vectors, int vec_first, int max_vectors, int fp32) {
+    const int want = (n_vectors < 0) ? n : std::max(n_vectors, max_vectors);
+    if (fp32 || ctx->two_stage < 0 || n < 2 || want == 0 || (want <= 20 && vec_first == 0)) return false;
+    const char* che = getenv("BSE_CHASE");
+    if (che && !strcmp(che, "tasks")) return false;
+    return (ctx->two_stage > 0 || n >= kQ2MinN) &&
+           bse_chase_resident_workspace(n, kBand, 2 * kBand + 1, ctx->device) > 0;
+}
+
+// V2 (may be null): the chase's reflectors are wanted.  Returns kNotResident,
+// with H as it was, when they could not be had (the resident chase did not run).
+static const int kNotResident = 1;
+static int twostage_tridiag(bse_ctx* ctx, int n, void* H, int fp32, const double2* rho, double2* V2 = nullptr) {
     hipStream_t st = ctx->st;
     const int b = kBand, ldab = 2 * b + 1;
     double* d = BUF(double, S_D, n);
@@ -862,10 +881,16 @@ static int twostage_tridiag(bse_ctx* ctx, int n, void* H, int fp32, const double
     const int64_t mel = (che && !strcmp(che, "tasks")) ? 0 : bse_chase_resident_workspace(n, b, ldab, ctx->device);
     if (mel > 0) {
         double2* msg = BUF(double2, S_BMSG, mel);
-        HCK(bse_launch_chase_resident(st, ctx->device, n, b, AB, ldab, y, d, e, msg, prog + ncnt));
+        HCK(bse_launch_chase_resident(st, ctx->device, n, b, AB, ldab, y, d, e, msg, prog + ncnt, V2));
         HCK(hipEventRecord(tv[2], st));
         HCK(hipMemcpyAsync(&err, prog + ncnt, sizeof(int), hipMemcpyDeviceToHost, st));
         HCK(hipStreamSynchronize(st));
+        if (err == 2 && V2) {
+            if (npan > 0)
+                HCK(hipMemcpyAsync(H, ctx->bufs[S_BH0].p, (size_t)tiled_elems(n) * (fp32 ? sizeof(float2) : sizeof(double2)),
+                                   hipMemcpyDeviceToDevice, st));
+            return kNotResident;
+        }
         if (err == 2) HCK(bse_launch_zero_words(st, (ncnt + 4) / 2, prog));
     }
     if (mel <= 0 || err == 2) {
@@ -983,8 +1008,15 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     const int nb = kPanel;
     hipStream_t st = ctx->st;
     if (vec_first < 0 || vec_first > n) return fail(ctx, BSE_ERR_ARG, "first vector index out of range");
-    const bool two = vec_first == 0 && use_two_stage(ctx, n, n_vectors, max_vectors, fp32);
-    ctx->last_two_stage = two;
+    bool two = vec_first == 0 && use_two_stage(ctx, n, n_vectors, max_vectors, fp32);
+    // many vectors by two stages, if there is memory for the chase's reflectors
+    double2* V2 = nullptr;
+    if (!two && use_q2(ctx, n, n_vectors, vec_first, max_vectors, fp32)) {
+        int no = BSE_OK;
+        V2 = bufT<double2>(ctx, S_Q2V, (size_t)bse_q2_workspace(n), &no);
+        if (!V2) (void)hipGetLastError();
+        two = V2 != nullptr;
+    }
     ctx->stage_ms[ST_BAND] = ctx->stage_ms[ST_CHASE] = 0.0;
     if (ctx->prof) ctx->prof_two_stage = false;
     // ---------------- K5: tridiagonalisation
@@ -999,15 +1031,21 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     double* e = nullptr;
     if (two) {
         stage_begin(ctx, ST_TRD);
-        int rc2 = twostage_tridiag(ctx, n, H, fp32, rho);
-        if (rc2) return rc2;
+        int rc2 = twostage_tridiag(ctx, n, H, fp32, rho, V2);
+        if (rc2 == kNotResident) two = false;
+        else if (rc2) return rc2;
+    }
+    const bool q2 = two && V2 != nullptr;
+    ctx->last_two_stage = two;
+    if (two) {
         d = (double*)ctx->bufs[S_D].p;
         e = (double*)ctx->bufs[S_E].p;
         sk_el = (int64_t)64 * 1024 * 1024 / sizeof(double2);
         skw = BUF(double2, S_SPLITK, std::min<int64_t>(sk_el, std::max<int64_t>((int64_t)64 * nb * 64, (int64_t)nb * nb * 512)));
         sk_el = (int64_t)(ctx->bufs[S_SPLITK].cap / sizeof(double2));
         stage_end(ctx, ST_TRD);
-    } else {
+    }
+    if (!two) {
     bse_hetrd_workspace(n, nb, &vs_el, &yr_el, &yc_el, &part_d);
     bse_hetrd_workspace(n, nb, &vs_el, &yr_el, &yc_el, &part_d);
     {
@@ -1164,7 +1202,11 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     bstart.push_back(0);
     for (int i = 0; i < n - 1; ++i) {
         const double ee = he[i] * he[i];
-        if (fabs(hd[i] * hd[i + 1]) * DBL_EPSILON * DBL_EPSILON + DBL_MIN >= ee) {
+        // the chase grades what rounding leaves of a rank-deficient matrix down to
+        // nothing; its vectors are told apart only when entries below the
+        // rounding error of the norm split the matrix
+        if (fabs(hd[i] * hd[i + 1]) * DBL_EPSILON * DBL_EPSILON + DBL_MIN >= ee ||
+            (q2 && fabs(he[i]) <= 0.5 * DBL_EPSILON * tnorm)) {
             he[i] = 0.0;
             bstart.push_back(i + 1);
         } else {
@@ -1268,7 +1310,7 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     // two-stage: the band inverse iteration and Z = Q1 X need only the
     // eigenvalues, so they run on the side stream beside the tridiagonal
     // vectors of the oscillator contraction; st joins before the refinement
-    const bool vec_side = two && nstore > 0;
+    const bool vec_side = two && !q2 && nstore > 0;
     std::vector<int64_t> bvoff;
     if (vec_side) {
         HCK(hipEventRecord(ctx->fork_ev, st));
@@ -1304,7 +1346,7 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     int m0 = 0;
     // the two-stage path forms its vectors from the band matrix: the
     // tridiagonal vectors are needed only for the oscillator contraction
-    if (two && !rho) m0 = n;
+    if (two && !q2 && !rho) m0 = n;
     size_t ci = 0;   // clusters are visited in order of their first member
     std::vector<int2> clall_sorted = clall;
     std::sort(clall_sorted.begin(), clall_sorted.end(),
@@ -1331,7 +1373,7 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
         }
         // commit the batch's members of [vec_first, vec_first + nstore)
         const int lo = std::max(m0, vec_first), hi = std::min(m1, vec_first + nstore);
-        if (!two && hi > lo)
+        if ((!two || q2) && hi > lo)
             HCK(bse_launch_commit(st, n, bsz, cnt - (lo - m0), hi - lo, lo, d_bsv, d_nbv, xb + (lo - m0), Z, n,
                                   lo - vec_first));
         HCK(hipStreamSynchronize(st));   // keeps d_cl and the host vectors alive
@@ -1347,6 +1389,21 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
             if (rc3) return rc3;
         }
         HCK(hipStreamWaitEvent(st, ctx->join_ev, 0));
+    } else if (q2 && nstore > 0) {
+        // Z <- Q1 Q2 Z
+        HCK(bse_apply_q2(st, n, V2, Z, n, nstore));
+        const int npb = (int)ctx->band_panels.size();
+        if (npb > 0) {
+            bvoff.resize(npb);
+            for (int p = 0; p < npb; ++p) bvoff[p] = ctx->band_panels[p].voff;
+            int64_t* voff_d = BUF(int64_t, S_BTVOFF, npb);
+            HCK(hipMemcpyAsync(voff_d, bvoff.data(), sizeof(int64_t) * npb, hipMemcpyHostToDevice, st));
+            const int64_t wel = bse_apply_q_grouped_workspace(n, npb, nstore);
+            double2* bws = BUF(double2, S_BTWS, wel);
+            const double2* V1 = (const double2*)ctx->bufs[S_VSTORE].p;
+            HCK(bse_apply_q_grouped_prepare(st, n, npb, kBand, 0, V1, voff_d, (const double2*)ctx->bufs[S_TALL].p, bws));
+            HCK(bse_apply_q_grouped_run(st, n, npb, kBand, 0, V1, voff_d, Z, n, nstore, bws, wel));
+        }
     } else if (nstore > 0 && nstore <= 16 && bse_apply_q_thin_workspace(n) <= sk_el) {
         HCK(bse_apply_q_thin(st, n, nb, Vst, Tall, nstore, Z, n, 0, skw));
     } else if (nstore > 16 && n >= kGroupedMinN && nb == 32 && !getenv("BSE_BT_STRIPS")) {

@@ -239,6 +239,13 @@ __device__ inline double rcp_nr(double x) {
     return fma(r, fma(-x, r, 1.0), r);
 }
 
+// The bulge chase's reflectors, 32 entries each: those of row block k (rows s + 1
+// + 32 k .. of sweep s) start at reflector 32 (k C - k (k - 1) / 2), C = ceil((n -
+// 1) / 32), in the order of s; element offset of the S-th group of 32 there.
+__host__ __device__ inline int64_t bse_q2_block(int C, int S, int k) {
+    return ((int64_t)k * C - (int64_t)k * (k - 1) / 2 + S) * 32 * 32;
+}
+
 // c ? a : b on the components (a conditional on the vectors themselves selects
 // between their addresses and puts both in scratch memory).
 __device__ inline double2 csel(bool c, double2 a, double2 b) { return cmk(c ? a.x : b.x, c ? a.y : b.y); }

@@ -124,7 +124,9 @@ hipError_t bse_launch_her2k_part(hipStream_t, int, int, int, int, int, void*, co
                                  int64_t, int, int, const double2*);
 int64_t bse_chase_resident_workspace(int, int, int, int);
 hipError_t bse_launch_chase_resident(hipStream_t, int, int, int, const double2*, int, double2*, double*, double*,
-                                     double2*, int*);
+                                     double2*, int*, double2*);
+int64_t bse_q2_workspace(int);
+hipError_t bse_apply_q2(hipStream_t, int, const double2*, double2*, int64_t, int);
 int64_t bse_chase_counters(int);
 hipError_t bse_launch_chase(hipStream_t, int, int, double2*, int, double2*, double*, double*, int*, int*, int);
 int64_t bse_band_ii_workspace(int, int, int);
@@ -304,7 +306,7 @@ enum Slot {
     S_RS, S_RHS, S_RX, S_RG, S_RHG, S_RC, S_RSMALL,
     S_GDHR, S_GDEPS, S_GDCOEF, S_GDP, S_GDPV, S_GDRHO, S_GDDE, S_GDW, S_GY, S_GOUT,
     S_SGFB, S_SGFA, S_SGX, S_SGU, S_SGB, S_SGV, S_SGPART, S_APPLYP, S_MEMB, S_KMAP, S_KINV, S_TBK, S_TBH, S_TBR, S_TBE, S_TBC,
-    S_BAB, S_BAB0, S_BPAN, S_BTSQR, S_BUPD, S_BPROG, S_BMSG, S_PNMSG, S_PNERR, S_BII, S_BZERO, S_BH0, S_BFAIL,
+    S_BAB, S_BAB0, S_BPAN, S_BTSQR, S_BUPD, S_BPROG, S_BMSG, S_PNMSG, S_Q2V, S_PNERR, S_BII, S_BZERO, S_BH0, S_BFAIL,
     // grouped back-transform: panel offsets, workspace
     S_BTVOFF, S_BTWS,
     // full BSE: coupling block, M / its Cholesky factor, W = L^H s3 L, tile

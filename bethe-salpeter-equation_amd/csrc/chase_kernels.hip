@@ -58,14 +58,17 @@ __device__ inline void wave_lds_sync() {
 
 // Reflector (LAPACK zlarfg): from alpha (lane 0's x) and ss = sum |x_i|^2
 // over i >= 1, H = I - tau v v^H with v_0 = 1, v_i = x_i scal, H^H x = beta e_1.
+// H = I where |x|^2 <= tiny: with tiny > 0 (1e-290: |x|^2 has all its digits) H
+// is unitary to rounding whatever x, which only who keeps H needs.
 struct Refl { double2 tau, scal; double beta; };
-__device__ inline Refl make_refl(double2 alpha, double ss) {
+__device__ inline Refl make_refl(double2 alpha, double ss, double tiny = 0.0) {
     Refl r;
     r.tau = cmk(0, 0);
     r.scal = cmk(0, 0);
     r.beta = alpha.x;
-    if (!(ss == 0.0 && alpha.y == 0.0)) {
-        const double nrm = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + ss);
+    const double nrm2 = alpha.x * alpha.x + alpha.y * alpha.y + ss;
+    if (!(ss == 0.0 && alpha.y == 0.0) && !(nrm2 <= tiny && tiny > 0.0)) {
+        const double nrm = sqrt(nrm2);
         r.beta = (alpha.x >= 0.0) ? -nrm : nrm;
         r.tau = cmk((r.beta - alpha.x) / r.beta, -alpha.y / r.beta);
         r.scal = crecip_safe(cmk(alpha.x - r.beta, alpha.y), nrm);
@@ -432,6 +435,7 @@ struct ChaseSysArgs {
     bse_i4v* msg;        // npos x CHS_SLOT words, zeroed
     unsigned* meet;      // arrivals (zeroed)
     int* err;            // 0; 1: a wait was given up; 2: not every workgroup became resident
+    double2* V2;         // may be null; the reflectors, entry 0 holding tau (q2_kernels.hip)
 };
 // words (16 bytes) of one workgroup's inbox
 #define CHS_V 0                               // 64: v_{k-1} (its unit first entry replaced by tau)
@@ -567,7 +571,7 @@ __global__ __launch_bounds__(128, 2) void k_chase_resident(ChaseSysArgs a)
                                                        __builtin_amdgcn_readlane(__double2loint(x.x), 0)),
                                       __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x.y), 0),
                                                        __builtin_amdgcn_readlane(__double2loint(x.y), 0)));
-            const Refl r = make_refl(alpha, ss);
+            const Refl r = make_refl(alpha, ss, a.V2 ? 1e-290 : 0.0);
             const double2 v = (i == 0) ? cmk(1.0, 0.0) : cmul(x, r.scal);
             const double2 out = (i == 0) ? r.tau : v;
             if (right)
@@ -640,6 +644,8 @@ __global__ __launch_bounds__(128, 2) void k_chase_resident(ChaseSysArgs a)
             if (lane < 3) reinterpret_cast<double*>(sW)[lane == 0 ? 0 : lane + 1] = dw;   // sW = (D(0,0), -), y
             wave_lds_sync();
             const double2 v = sV[par][i], tau = sTau[par];
+            if (a.V2 && h == 0)
+                a.V2[bse_q2_block(a.npos, 0, k) + (int64_t)s * CH_B + i] = cmk(i == 0 ? tau.x : v.x, i == 0 ? tau.y : v.y);
             // row i of D_k: the lower triangle as stored, the upper one from it;
             // row and column 31 are the entering ones (all of them in LDS in sweep 0)
             double2 t[16];
@@ -750,7 +756,8 @@ hipError_t resident_launch(int device, hipStream_t st, const std::function<hipEr
 // err receives 0, 1 (a wait was given up) or 2 (the workgroups did not become
 // resident together: AB, y, d and e are as they were).
 extern "C" hipError_t bse_launch_chase_resident(hipStream_t st, int device, int n, int b, const double2* AB,
-                                                int ldab, double2* y, double* d, double* e, double2* ws, int* err)
+                                                int ldab, double2* y, double* d, double* e, double2* ws, int* err,
+                                                double2* V2)
 {
     const int grid = chase_resident_grid(n, b, ldab, device);
     if (grid == 0) return hipErrorInvalidValue;
@@ -759,7 +766,7 @@ extern "C" hipError_t bse_launch_chase_resident(hipStream_t st, int device, int 
     hipError_t rc = bse_launch_zero_words(st, 2 * (words + 1), ws);
     if (rc != hipSuccess) return rc;
     const ChaseSysArgs args{n, ldab, npos, AB, y, d, e, reinterpret_cast<bse_i4v*>(ws),
-                            reinterpret_cast<unsigned*>(ws + words), err};
+                            reinterpret_cast<unsigned*>(ws + words), err, V2};
     return resident_launch(device, st, [&]() -> hipError_t {
         hipLaunchKernelGGL(k_chase_resident, dim3((unsigned)grid), dim3(128), 0, st, args);
         return hipGetLastError();

@@ -1,0 +1,112 @@
+"""Many eigenvectors through the two-stage reduction: the bulge chase's
+reflectors applied to the tridiagonal vectors, at the edges of their 32-sweep
+blocks, of the 128 sweeps of a pass and of the column strips (16 columns, and 32
+where the columns fill the chip).
+
+Vectors of a unitary similarity transform in FP64: residual and orthogonality
+to 1e-12 sqrt(n) of the norm, as for the other back-transforms.
+"""
+import numpy as np
+import pytest
+
+import bse_amd
+from bse_amd import _abi
+from bse_amd.lattice import KGrid
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx2():
+    mp = pytest.MonkeyPatch()
+    mp.setenv("BSE_TWO_STAGE", "1")
+    c = _abi.Context(0)
+    mp.undo()
+    yield c
+    c.close()
+
+
+def _herm(n):
+    rng = np.random.default_rng(n)
+    a = rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n))
+    return 0.5 * (a + a.conj().T)
+
+
+@pytest.mark.parametrize("n", [21, 31, 32, 33, 34, 35, 63, 64, 65, 66, 97, 98, 128, 129, 130, 161, 258, 290, 545])
+@pytest.mark.parametrize("nvec", [21, -1])
+def test_orders(ctx2, n, nvec):
+    print(f"many vectors n={n} nvec={nvec}", flush=True)
+    a = _herm(n)
+    ev, z = ctx2.eigh_dense(a, "fp64", nvec)
+    ref = np.linalg.eigvalsh(a)
+    k, tol = z.shape[1], 1e-12 * n ** 0.5
+    assert np.abs(ev - ref).max() < tol * np.abs(ref).max()
+    assert np.abs(a @ z - z * ev[None, :k]).max() < tol * np.abs(ref).max()
+    assert np.abs(z.conj().T @ z - np.eye(k)).max() < tol
+
+
+@pytest.mark.parametrize("n", [2, 3, 5])
+def test_smallest(ctx2, n):
+    print(f"many vectors n={n}", flush=True)
+    a = _herm(n)
+    ev, z = ctx2.eigh_dense(a, "fp64", -1)
+    assert np.abs(a @ z - z * ev[None, :]).max() < 1e-13 * n * max(np.abs(ev).max(), 1.0)
+
+
+def test_wide_strips(ctx2):
+    n = 4130
+    print(f"many vectors n={n}", flush=True)
+    a = _herm(n)
+    ev, z = ctx2.eigh_dense(a, "fp64", -1)
+    pick = np.unique(np.r_[np.arange(0, n, 41), n - 33:n])
+    zp = z[:, pick]
+    tol = 1e-12 * n ** 0.5
+    assert np.abs(a @ zp - zp * ev[None, pick]).max() < tol * np.abs(ev).max()
+    g = z.conj().T @ zp
+    g[pick, np.arange(pick.size)] -= 1.0
+    assert np.abs(g).max() < tol
+
+
+@pytest.mark.parametrize("make", [lambda: np.diag(np.arange(1.0, 71.0)), lambda: np.zeros((70, 70)),
+                                  lambda: np.kron(np.eye(7), _herm(10)), lambda: np.ones((66, 66))],
+                         ids=["diagonal", "zero", "blocks", "rank1"])
+def test_vanishing_reflectors(ctx2, make):
+    a = make().astype(complex)
+    n = a.shape[0]
+    ev, z = ctx2.eigh_dense(a, "fp64", -1)
+    scale = max(np.abs(ev).max(), 1.0)
+    assert np.abs(a @ z - z * ev[None, :]).max() < 1e-11 * scale
+    assert np.abs(z.conj().T @ z - np.eye(n)).max() < 1e-10
+
+
+def test_without_the_resident_chase(ctx2, monkeypatch):
+    """The general chase keeps no reflectors: the one-stage reduction serves."""
+    a = _herm(200)
+    monkeypatch.setenv("BSE_CHASE", "tasks")
+    ev, z = ctx2.eigh_dense(a, "fp64", -1)
+    assert np.abs(a @ z - z * ev[None, :]).max() < 1e-11 * np.abs(ev).max()
+
+
+@pytest.mark.parametrize("grid", [(5, 7), (8, 13), (11, 12)])
+def test_problem_and_full_form(ctx2, grid):
+    """With a dipole vector and an offset first vector (the full BSE's positive
+    branch), against the one-stage reduction."""
+    s = bse_amd.honeycomb_plain(6, gap=2.2).with_params(grid=KGrid(*grid))
+    om = s.omegas()
+    print(f"many vectors grid {grid}", flush=True)
+    mp = pytest.MonkeyPatch()
+    mp.setenv("BSE_TWO_STAGE", "0")
+    c1 = _abi.Context(0)
+    mp.undo()
+    res = []
+    for c in (c1, ctx2):
+        c.set_system(s).build("fp64").eigh(-1)
+        tda = (c.eigenvalues(), c.spectrum(om, s.eta))
+        c.build_full().eigh_full(-1)
+        x, E = c.eigenvectors(s.n_bse), c.eigenvalues()
+        res.append(tda + (E, c.spectrum(om, s.eta)))
+        s3 = np.concatenate([np.ones(s.n_bse), -np.ones(s.n_bse)])
+        assert np.abs(x.conj().T @ (s3[:, None] * x) - np.eye(s.n_bse)).max() < 1e-8
+    c1.close()
+    for a, b in zip(*res):
+        assert np.linalg.norm(a - b) < 1e-10 * np.linalg.norm(a)
