@@ -38,8 +38,10 @@
 // ---------------------------------------------------------------------------
 // Gather of panel p from the tiled lower storage: P (m x b, ld m, FP64) and
 // the lower triangle of the diagonal block A[c0 : c0+b, c0 : c0+b] into the
-// band store.  One thread per row of the panel (b columns each); the threads
-// of the first block also copy the diagonal block.
+// band store.  A workgroup takes 64 rows, each wave eight columns of them, all
+// eight loads in flight (one thread per row and one load at a time was 13 us a
+// panel at n = 4624, 4.4 now); the threads of the first block also copy the
+// diagonal block.
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(256) void k_band_gather(int n, int c0, int b, const T* __restrict__ A,
@@ -48,9 +50,14 @@ __global__ __launch_bounds__(256) void k_band_gather(int n, int c0, int b, const
 {
     const int nt = tile_count(n);
     const int s = c0 + b, m = n - s;
-    const int r = blockIdx.x * 256 + threadIdx.x;
+    const int r = blockIdx.x * 64 + (threadIdx.x & 63), j0 = 8 * (threadIdx.x >> 6);
     if (r < m) {
-        for (int j = 0; j < b; ++j) P[r + (int64_t)j * m] = cplx<T>::load(A + tix(s + r, c0 + j, nt));
+        double2 x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = cplx<T>::load(A + tix(s + r, c0 + min(j0 + u, b - 1), nt));
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (j0 + u < b) P[r + (int64_t)(j0 + u) * m] = x[u];
     }
     if (blockIdx.x == 0) {
         // diagonal block, lower triangle (rows and columns below n)
@@ -534,7 +541,9 @@ __global__ __launch_bounds__(256) void k_rows_small(int m, int k0, int kx, int n
 // to rounding level), when a column is zero, or when G2 is not within 0.1 of
 // the identity.
 // ---------------------------------------------------------------------------
-#define CQ_G 64           // workgroups of the row-parallel passes
+// Partial Gram matrices (one workgroup per 64 rows up to this many; with 63 of
+// them a panel of 4624 rows took a second round: 13 us, 8 now) and their sum.
+#define CQ_G 257
 
 // Partial Gram matrices G = P^H P over each workgroup's 64-row chunks
 // (chunks g, g + grid, ...), partial g (b x b, column-major) -> Gp + g b b.
@@ -576,23 +585,36 @@ __global__ __launch_bounds__(256) void k_cq_gram(int m, const double2* __restric
     for (int u = 0; u < 4; ++u) Gp[(int64_t)blockIdx.x * BR_B * BR_B + tid + 256 * u] = g[u];
 }
 
-// G = sum of the ng partial Gram matrices (fixed order), one element per
-// thread over 4 workgroups, 16 loads in flight per batch.  Runs when flag[f]
-// is set (f < 0: always).
+// G = sum of the ng partial Gram matrices: a workgroup takes 32 elements, thread
+// (part, element) the partials part, part + 8, ... with 16 loads in flight, and
+// the eight part sums are added in order.  Runs when flag[f] is set (f < 0:
+// always).
 __global__ __launch_bounds__(256) void k_cq_reduce(int ng, const double2* __restrict__ Gp,
                                                    double2* __restrict__ G, const int* __restrict__ flag, int f)
 {
+    __shared__ double2 sp[8][32];
     if (f >= 0 && flag[f] == 0) return;
-    const int e = blockIdx.x * 256 + threadIdx.x;        // < BR_B * BR_B
+    const int l = threadIdx.x & 31, part = threadIdx.x >> 5;
+    const int e = blockIdx.x * 32 + l;                   // < BR_B * BR_B
     double2 acc = cmk(0, 0);
-    for (int g0 = 0; g0 < ng; g0 += 16) {
+    for (int g0 = part; g0 < ng; g0 += 128) {
         double2 t[16];
 #pragma unroll
-        for (int q = 0; q < 16; ++q) t[q] = (g0 + q < ng) ? Gp[(int64_t)(g0 + q) * BR_B * BR_B + e] : cmk(0, 0);
+        for (int q = 0; q < 16; ++q) {
+            const int g = g0 + 8 * q;
+            const double2 x = Gp[(int64_t)min(g, ng - 1) * BR_B * BR_B + e];
+            t[q] = cmk(g < ng ? x.x : 0.0, g < ng ? x.y : 0.0);
+        }
 #pragma unroll
         for (int q = 0; q < 16; ++q) acc = cadd(acc, t[q]);
     }
-    G[e] = acc;
+    sp[part][l] = acc;
+    __syncthreads();
+    if (part == 0) {
+#pragma unroll
+        for (int u = 1; u < 8; ++u) acc = cadd(acc, sp[u][l]);
+        G[e] = acc;
+    }
 }
 
 // The 32 x 32 factorisations below keep the matrix in registers, thread
@@ -1128,18 +1150,33 @@ __global__ __launch_bounds__(256) void k_band_xt(int n, int s, int k, int b, con
         const int i = e % BR_B, j = e / BR_B;
         sT[i][j] = (i < k && j < k) ? Tp[i + j * b] : cmk(0, 0);
     }
-    for (int e = threadIdx.x; e < 64 * BR_B; e += 256) {
-        const int rr = e & 63, c = e >> 6;
-        const int r = r0 + rr;
-        double2 x = cmk(0, 0), v = cmk(0, 0);
-        if (r < m && c < k) {
-            const int64_t t = (int64_t)(s + r) - (int64_t)tcs * 64;
-            for (int qq = 0; qq < HEMM_KSPLIT; ++qq)
-                x = cadd(x, Xp[(int64_t)qq * nT * 64 * BR_B + t + (int64_t)c * nT * 64]);
-            v = V[r + (int64_t)c * m];
+    // two of a thread's eight elements at a time: the loads of their partials are
+    // in flight together (one after the other: 26 us a panel at n = 4624, 19 now)
+    {
+        const int rr = threadIdx.x & 63, r = r0 + rr;
+        const int64_t t = (int64_t)(s + min(r, m - 1)) - (int64_t)tcs * 64;
+#pragma unroll 1
+        for (int u = 0; u < 8; u += 2) {
+            double2 x[2][HEMM_KSPLIT], v[2];
+#pragma unroll
+            for (int w = 0; w < 2; ++w) {
+                const int c = min((int)(threadIdx.x >> 6) + 4 * (u + w), k - 1);
+                v[w] = V[min(r, m - 1) + (int64_t)c * m];
+#pragma unroll
+                for (int qq = 0; qq < HEMM_KSPLIT; ++qq)
+                    x[w][qq] = Xp[(int64_t)qq * nT * 64 * BR_B + t + (int64_t)c * nT * 64];
+            }
+#pragma unroll
+            for (int w = 0; w < 2; ++w) {
+                const int c = (threadIdx.x >> 6) + 4 * (u + w);
+                double2 a = cmk(0, 0);
+#pragma unroll
+                for (int qq = 0; qq < HEMM_KSPLIT; ++qq) a = cadd(a, x[w][qq]);
+                const bool in = r < m && c < k;
+                sX[rr][c] = cmk(in ? a.x : 0.0, in ? a.y : 0.0);
+                sV[rr][c] = cmk(in ? v[w].x : 0.0, in ? v[w].y : 0.0);
+            }
         }
-        sX[rr][c] = x;
-        sV[rr][c] = v;
     }
     __syncthreads();
     // XT rows: every thread forms its 8 entries from the X rows, then they
@@ -1151,7 +1188,8 @@ __global__ __launch_bounds__(256) void k_band_xt(int n, int s, int k, int b, con
         const int e = threadIdx.x + 256 * u, rr = e & 63, c = e >> 6;
         const int r = r0 + rr;
         double2 acc = cmk(0, 0);
-        for (int l = 0; l < k; ++l) cfma(acc, sX[rr][l], sT[l][c]);
+#pragma unroll 8
+        for (int l = 0; l < BR_B; ++l) cfma(acc, sX[rr][l], sT[l][c]);
         if (r < m && c < k) Z[r + (int64_t)c * m] = acc;
         xt[u] = (r < m && c < k) ? acc : cmk(0, 0);
     }
@@ -1166,6 +1204,7 @@ __global__ __launch_bounds__(256) void k_band_xt(int n, int s, int k, int b, con
     for (int e = threadIdx.x; e < BR_B * BR_B; e += 256) {
         const int i = e % BR_B, j = e / BR_B;
         double2 acc = cmk(0, 0);
+#pragma unroll 8
         for (int rr = 0; rr < 64; ++rr) cfmac(acc, sV[rr][i], sX[rr][j]);
         Gp[(int64_t)blockIdx.x * BR_B * BR_B + e] = acc;
     }
@@ -1206,7 +1245,8 @@ extern "C" hipError_t bse_band_gather(hipStream_t st, int fp32, int n, int c0, i
                                       double2* P, double2* AB, int ldab)
 {
     const int m = n - c0 - b;
-    const unsigned g = (unsigned)std::max<int64_t>(1, ceil_div64(std::max(m, 1), 256));
+    const unsigned g = (unsigned)std::max<int64_t>(1, ceil_div64(std::max(m, 1), 64));
+    if (b > BR_B) return hipErrorInvalidValue;
     if (fp32)
         hipLaunchKernelGGL(k_band_gather<float2>, dim3(g), dim3(256), 0, st, n, c0, b, (const float2*)A, P, AB, ldab);
     else
@@ -1307,13 +1347,13 @@ extern "C" hipError_t bse_band_panel_qr(hipStream_t st, int m, int b, double2* P
         const int g = (int)std::min<int64_t>(CQ_G - 1, ceil_div64(m, 64));
         double2* Gs = Gp + (int64_t)(CQ_G - 1) * BR_B * BR_B;    // the summed G (last partial slot is spare)
         hipLaunchKernelGGL(k_cq_gram<0>, dim3((unsigned)g), dim3(256), 0, st, m, (const double2*)P, Gp, flags);
-        hipLaunchKernelGGL(k_cq_reduce, dim3(BR_B * BR_B / 256), dim3(256), 0, st, g, (const double2*)Gp, Gs,
+        hipLaunchKernelGGL(k_cq_reduce, dim3(BR_B * BR_B / 32), dim3(256), 0, st, g, (const double2*)Gp, Gs,
                            (const int*)flags, -1);
         hipLaunchKernelGGL(k_cq_chol1, dim3(1), dim3(256), 0, st, (const double2*)Gs, R1, R1i, flags, fail);
         hipLaunchKernelGGL(k_rows_small, dim3((unsigned)ceil_div64(m, 64)), dim3(256), 0, st, m, 0, BR_B, BR_B, BR_B,
                            (const double2*)P, (const double2*)R1i, Q, 0, (const int*)(flags + 1));
         hipLaunchKernelGGL(k_cq_gram<1>, dim3((unsigned)g), dim3(256), 0, st, m, (const double2*)Q, Gp, flags);
-        hipLaunchKernelGGL(k_cq_reduce, dim3(BR_B * BR_B / 256), dim3(256), 0, st, g, (const double2*)Gp, Gs,
+        hipLaunchKernelGGL(k_cq_reduce, dim3(BR_B * BR_B / 32), dim3(256), 0, st, g, (const double2*)Gp, Gs,
                            (const int*)flags, 1);
         hipLaunchKernelGGL(k_cq_chol2, dim3(1), dim3(256), 0, st, m, b, (const double2*)Gs, (const double2*)Q,
                            (const double2*)R1, Vout, Tp, Mp, AB, ldab, c0, flags, fail);
