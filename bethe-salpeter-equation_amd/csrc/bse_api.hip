@@ -996,6 +996,20 @@ static int twostage_vectors_rest(bse_ctx* ctx, hipStream_t st, int n, int nstore
     return BSE_OK;
 }
 
+// Whether `extra` bytes beside what a solve with nvec vectors will still allocate
+// (its vectors, reflectors and inverse-iteration scratch) are there: a faster path
+// must not take the memory that the solve needs.  Orders up to 16384 need at most
+// a tenth of the device's memory and are not asked about.
+static bool memory_to_spare(const bse_ctx* ctx, int n, int nvec, double extra) {
+    if (n <= 16384) return true;
+    size_t free_b = 0, total = 0;
+    if (hipMemGetInfo(&free_b, &total) != hipSuccess) return true;
+    const double dn = n, batch = std::min(dn, std::max(4096.0, 24e9 / (48.0 * dn)));
+    double have = (double)free_b;
+    for (int slot : {S_Z, S_VSTORE, S_IISCR, S_IIX, S_BH0, S_Q2V}) have += (double)ctx->bufs[slot].cap;
+    return extra + 16.0 * dn * nvec + 8.0 * dn * dn + 48.0 * dn * batch + 4e9 <= have;
+}
+
 // guard_tol > 0: eigenvalues within guard_tol above the last requested one
 // are formed as well, up to max_vectors in total (ctx->nvec reports the count).
 // vec_first > 0: the vectors formed are those of the sorted eigenvalues
@@ -1011,7 +1025,9 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     bool two = vec_first == 0 && use_two_stage(ctx, n, n_vectors, max_vectors, fp32);
     // many vectors by two stages, if there is memory for the chase's reflectors
     double2* V2 = nullptr;
-    if (!two && use_q2(ctx, n, n_vectors, vec_first, max_vectors, fp32)) {
+    const int nvec_max = (n_vectors < 0) ? n : std::min(n, std::max(n_vectors, max_vectors));
+    if (!two && use_q2(ctx, n, n_vectors, vec_first, max_vectors, fp32) &&
+        memory_to_spare(ctx, n, nvec_max, 16.0 * (double)n * n)) {
         int no = BSE_OK;
         V2 = bufT<double2>(ctx, S_Q2V, (size_t)bse_q2_workspace(n), &no);
         if (!V2) (void)hipGetLastError();
@@ -1090,7 +1106,7 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     void* H0 = nullptr;
     if (prun.ws_el > 0) {
         int no = BSE_OK;
-        H0 = buf(ctx, S_BH0, hbytes, &no);
+        if (memory_to_spare(ctx, n, nvec_max, (double)hbytes)) H0 = buf(ctx, S_BH0, hbytes, &no);
         if (!H0) {
             (void)hipGetLastError();
             prun.ws_el = 0;                 // no room for the copy: per-column launches

@@ -70,7 +70,7 @@ __global__ __launch_bounds__(256) void k_compose_full(int64_t N, const double2* 
 // before it; the pivot column passes through LDS, one barrier a step (the
 // columns, published unscaled, stay as L D^1/2), the inverse's part of the
 // pivot row is lane j of every wave.  200 us with three barriers a step on an LDS tile and a serial
-// substitution per column for the inverse, 47 us this way.
+// substitution per column for the inverse, 65 us this way.
 // ---------------------------------------------------------------------------
 __device__ inline double lane_value(double x, int lane) {
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), lane),
