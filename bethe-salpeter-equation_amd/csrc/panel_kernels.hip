@@ -32,6 +32,20 @@
 // later.  So it polls the former first and forms the reflector and the panel
 // corrections from them while the latter are on their way.
 //
+// Reuse of the message areas.  Each has two copies by the column's parity, so a
+// workgroup's words for column c + 2 replace those for column c, which every
+// reader must have read by then.  A workgroup posts words for column c + 2
+// only once it holds a word of x(c + 2), and the owner that posted this word had
+// finished column c + 1, in which it waited for the sums over x(c + 1) of every
+// owner, posted by each behind its last read of column c; and it waited for
+// x^H A x of column c + 1 from every workgroup, posted behind their last read of
+// x(c).  So every workgroup has to wait for some row of x in every column, row
+// s0 included (pn_awaits): the last row of an order 64 k + 1 is s0 itself in the
+// last column, and all there is to wait for in tile (k, k).  An owner needs no
+// such row: it has finished column c + 1 itself.  Tile row 0 can be behind s0,
+// but its tile (0, 0) is workgroup 0's, an owner; every other one reaches s0 or
+// beyond (bse_panel_unawaited counts what does not, on the host).
+//
 // Every sum runs in a fixed order.  FP64 throughout; T is the storage type.
 //
 // Measured (FP64 storage), us per column: 6.7 with 3 tile rows, 7.9 with 22 (one
@@ -87,6 +101,10 @@ __host__ __device__ inline PanelMsg panel_msg(int nbk, int grid) {
     L.total = (int64_t)L.p + 2 * (int64_t)L.ps;
     return L;
 }
+
+// Whether a tile waits for row g of x in the column with x below row s0: its rows
+// below s0 and, for the reuse rule above, s0 itself (which takes no part).
+__host__ __device__ inline bool pn_awaits(int g, int s0, int n) { return g >= s0 && g < n; }
 
 // R complex values, value u at word off[u] (off < 0: not wanted, zero), all
 // polled together.  False when the wait was given up.
@@ -246,11 +264,12 @@ __global__ __launch_bounds__(PN_THREADS) void k_trd_panel(PanelArgs a)
 #pragma unroll
             for (int k = 0; k < NT; ++k) tb = (r == k) ? ((w & 1) ? J[k] : I[k]) : tb;
             const int g = R0 + 64 * tb + lane;
-            const int off[1] = {(tb >= 0 && g > s0 && g < n) ? L.x + par * L.xs + (tb * 64 + lane) * 2 : -1};
+            const int off[1] = {(tb >= 0 && pn_awaits(g, s0, n)) ? L.x + par * L.xs + (tb * 64 + lane) * 2 : -1};
             double2 v[1];
             if (!pn_poll<1>(rm, off, tag, v, a.err)) return;
-            if (w & 1) sXc[r][lane] = v[0];
-            else sXr[r][lane] = v[0];
+            const double2 x = pn_sel(g == s0, cmk(0, 0), v[0]);
+            if (w & 1) sXc[r][lane] = x;
+            else sXr[r][lane] = x;
         }
         __syncthreads();
         double ql = 0.0;
@@ -580,6 +599,29 @@ extern "C" int bse_panel_first(int n, int nwg)
     for (int j0 = 0; j0 < n - 1; j0 += PN_B)
         if (panel_plan(n, j0, nwg).ok) return j0;
     return n;
+}
+
+// Workgroups without tile rows of their own (no owners) that would wait for no
+// row of x in some column, over all panels: none, or the reuse rule is broken.
+extern "C" int64_t bse_panel_unawaited(int n, int nwg)
+{
+    int64_t bad = 0;
+    for (int j0 = bse_panel_first(n, nwg); j0 < n - 1; j0 += PN_B) {
+        const PanelPlan p = panel_plan(n, j0, nwg);
+        if (!p.ok) return -1;
+        for (int wg = p.nbk; wg < p.grid; ++wg)
+            for (int s0 = j0 + 1; s0 <= std::min(j0 + PN_B, n - 1); ++s0) {
+                bool waits = false;
+                for (int t = wg; t < p.ntl && !waits; t += p.grid) {
+                    int I, J;
+                    tri_tile(t, I, J);
+                    for (int r = 0; r < 64 && !waits; ++r)
+                        waits = pn_awaits(64 * (p.tc0 + I) + r, s0, n) || pn_awaits(64 * (p.tc0 + J) + r, s0, n);
+                }
+                bad += waits ? 0 : 1;
+            }
+    }
+    return bad;
 }
 
 // 16-byte elements of the messages and of the panels' meeting counters.
