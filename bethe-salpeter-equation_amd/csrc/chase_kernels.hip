@@ -58,21 +58,46 @@ __device__ inline void wave_lds_sync() {
 
 // Reflector (LAPACK zlarfg): from alpha (lane 0's x) and ss = sum |x_i|^2
 // over i >= 1, H = I - tau v v^H with v_0 = 1, v_i = x_i scal, H^H x = beta e_1.
-// H = I where |x|^2 <= tiny: with tiny > 0 (1e-290: |x|^2 has all its digits) H
-// is unitary to rounding whatever x, which only who keeps H needs.
 struct Refl { double2 tau, scal; double beta; };
-__device__ inline Refl make_refl(double2 alpha, double ss, double tiny = 0.0) {
+__device__ inline Refl make_refl(double2 alpha, double ss) {
     Refl r;
     r.tau = cmk(0, 0);
     r.scal = cmk(0, 0);
     r.beta = alpha.x;
-    const double nrm2 = alpha.x * alpha.x + alpha.y * alpha.y + ss;
-    if (!(ss == 0.0 && alpha.y == 0.0) && !(nrm2 <= tiny && tiny > 0.0)) {
-        const double nrm = sqrt(nrm2);
+    if (!(ss == 0.0 && alpha.y == 0.0)) {
+        const double nrm = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + ss);
         r.beta = (alpha.x >= 0.0) ? -nrm : nrm;
         r.tau = cmk((r.beta - alpha.x) / r.beta, -alpha.y / r.beta);
         r.scal = crecip_safe(cmk(alpha.x - r.beta, alpha.y), nrm);
     }
+    return r;
+}
+
+// The reflector of a wave's column x (alpha in lane 0, its other entries in the
+// lanes with tail set); v_i = x_i scal with the x left here.  A column whose
+// squares would lose digits (|x|^2 below 1e-290: what a rank-deficient matrix
+// leaves, or a matrix of that size) is scaled up first, by 2^480 once or twice, so
+// that H is unitary to rounding, and nothing is dropped, whatever the size of x.
+__device__ inline Refl column_refl(double2& x, bool tail) {
+    double ss;
+    double2 alpha;
+    auto sums = [&]() {
+        ss = wave_sum_dpp(tail ? cabs2(x) : 0.0);
+        alpha = cmk(__hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x.x), 0),
+                                     __builtin_amdgcn_readlane(__double2loint(x.x), 0)),
+                    __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x.y), 0),
+                                     __builtin_amdgcn_readlane(__double2loint(x.y), 0)));
+    };
+    sums();
+    int up = 0;
+    // (the sums are the wave's, so every lane takes the same turn)
+    while (up < 960 && __any(cabs2(alpha) + ss < 1e-290) && __any(x.x != 0.0 || x.y != 0.0)) {
+        x = cmk(ldexp(x.x, 480), ldexp(x.y, 480));
+        up += 480;
+        sums();
+    }
+    Refl r = make_refl(alpha, ss);
+    if (up) r.beta = ldexp(r.beta, -up);
     return r;
 }
 
@@ -236,11 +261,9 @@ __global__ __launch_bounds__(64 * CH_W) void k_chase(ChaseArgs a)
                     tmp[c] = mem.ld(dbase + c * (ldab - 1) + lane, c < L && lane >= c && row);
                 double2 yy = cmk(0, 0);
                 if (k == 0) {
-                    const double2 x = mem.ld(s * ldab + 1 + lane, row);
+                    double2 x = mem.ld(s * ldab + 1 + lane, row);
                     if (a.y) yy = mem.ldy(lo + lane, row);
-                    const double ss = wave_sum_dpp((lane >= 1 && row) ? cabs2(x) : 0.0);
-                    const double2 alpha = cmk(__shfl(x.x, 0, 64), __shfl(x.y, 0, 64));
-                    const Refl r = make_refl(alpha, ss);
+                    const Refl r = column_refl(x, lane >= 1 && row);
                     tau = r.tau;
                     const double2 v0 = (lane == 0) ? cmk(1.0, 0.0) : cmul(x, r.scal);
                     if (row) sv[lane] = v0;
@@ -330,10 +353,8 @@ __global__ __launch_bounds__(64 * CH_W) void k_chase(ChaseArgs a)
                 }
                 wave_lds_sync();     // every lane is done with H_{k-1}'s vector
                 // (2) reflector from column 0
-                const double2 x = row ? xr[0] : cmk(0, 0);
-                const double ss = wave_sum_dpp((lane >= 1 && row) ? cabs2(x) : 0.0);
-                const double2 alpha = cmk(__shfl(x.x, 0, 64), __shfl(x.y, 0, 64));
-                const Refl r = make_refl(alpha, ss);
+                double2 x = row ? xr[0] : cmk(0, 0);
+                const Refl r = column_refl(x, lane >= 1 && row);
                 const double2 v = (lane == 0) ? cmk(1.0, 0.0) : (row ? cmul(x, r.scal) : cmk(0, 0));
                 if (lane < CH_B) {
                     sv[lane] = v;
@@ -566,12 +587,7 @@ __global__ __launch_bounds__(128, 2) void k_chase_resident(ChaseSysArgs a)
             } else {
                 x = ent;
             }
-            const double ss = wave_sum_dpp((i >= 1 && h == 0) ? cabs2(x) : 0.0);
-            const double2 alpha = cmk(__hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x.x), 0),
-                                                       __builtin_amdgcn_readlane(__double2loint(x.x), 0)),
-                                      __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x.y), 0),
-                                                       __builtin_amdgcn_readlane(__double2loint(x.y), 0)));
-            const Refl r = make_refl(alpha, ss, a.V2 ? 1e-290 : 0.0);
+            const Refl r = column_refl(x, i >= 1 && h == 0);
             const double2 v = (i == 0) ? cmk(1.0, 0.0) : cmul(x, r.scal);
             const double2 out = (i == 0) ? r.tau : v;
             if (right)

@@ -79,6 +79,43 @@ def test_vanishing_reflectors(ctx2, make):
     assert np.abs(z.conj().T @ z - np.eye(n)).max() < 1e-10
 
 
+@pytest.mark.parametrize("scale", [1e-129, 1e-140, 1e-147])
+@pytest.mark.parametrize("n", [70, 200])
+def test_small_scale(ctx2, n, scale):
+    """The same matrix in small units, plain and graded over ten decades: columns
+    of the chase whose squares leave the range of normal numbers count in full.
+    Errors relative to the norm as in test_orders.  (Below 1e-135 the inverse
+    iteration's own squares overflow, and at 1e-147 squares of the graded
+    matrix's small entries underflow in the tridiagonal's split.)"""
+    print(f"many vectors n={n} scale={scale}", flush=True)
+    g = np.logspace(0, -5, n)
+    for a in [_herm(n)] + ([_herm(n) * g[:, None] * g[None, :]] if scale > 1e-145 else []):
+        ref = np.linalg.eigvalsh(a)
+        ev, z = ctx2.eigh_dense(a * scale, "fp64", -1)
+        ev = ev / scale
+        tol = 1e-12 * n ** 0.5 * np.abs(ref).max()
+        assert np.abs(ev - ref).max() < tol
+        if scale > 1e-135:
+            assert np.abs(a @ z - z * ev[None, :]).max() < tol
+            assert np.abs(z.conj().T @ z - np.eye(n)).max() < 1e-12 * n ** 0.5
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-129])
+@pytest.mark.parametrize("nvec", [16, -1])
+def test_numerically_rank_one(ctx2, nvec, scale):
+    """What rounding leaves of a rank-one matrix is graded down to nothing."""
+    n = 300
+    print(f"rank one n={n} nvec={nvec} scale={scale}", flush=True)
+    v = np.random.default_rng(5).uniform(0.5, 1.5, n)
+    a = np.outer(v, v).astype(complex)
+    ev, z = ctx2.eigh_dense(a * scale, "fp64", nvec)
+    ev, k = ev / scale, z.shape[1]
+    tol = 1e-12 * n ** 0.5
+    assert np.abs(ev[:-1]).max() < tol * (v @ v) and abs(ev[-1] - v @ v) < tol * (v @ v)
+    assert np.abs(a @ z - z * ev[None, :k]).max() < tol * (v @ v)
+    assert np.abs(z.conj().T @ z - np.eye(k)).max() < tol
+
+
 def test_without_the_resident_chase(ctx2, monkeypatch):
     """The general chase keeps no reflectors: the one-stage reduction serves."""
     a = _herm(200)
