@@ -1101,7 +1101,8 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     // their workgroups at once
     const char* pne = getenv("BSE_TRD_PANEL");
     const int pnwg = ((pne && pne[0] == '0') || getenv("BSE_HEMV_CODE")) ? 0 : bse_panel_workgroups(ctx->device, fp32);
-    PanelRun prun{ctx->device, n, pnwg, nullptr, pnwg > 0 ? bse_panel_workspace(n, pnwg) : 0, nullptr};
+    PanelRun prun{ctx->device, n, pnwg, nullptr, pnwg > 0 ? bse_panel_workspace(n, pnwg) : 0, nullptr,
+                  nullptr};
     const size_t hbytes = (size_t)tiled_elems(n) * (fp32 ? sizeof(float2) : sizeof(double2));
     void* H0 = nullptr;
     if (prun.ws_el > 0) {
@@ -1117,8 +1118,9 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
         prun.ws = BUF(double2, S_PNMSG, prun.ws_el);
         prun.err = BUF(int, S_PNERR, 4);
         HCK(bse_launch_zero_words(st, 2 * prun.ws_el, prun.ws));
+        prun.big = reinterpret_cast<double*>(prun.err + 2);
         HCK(bse_launch_zero_words(st, 2, prun.err));
-        HCK(hipMemcpyAsync(H0, H, hbytes, hipMemcpyDeviceToDevice, st));
+        HCK(bse_launch_copy_max(st, fp32, n, H, H0, prun.big));
     }
     const int panel_first = prun.ws_el > 0 ? prun.first : n;
     {

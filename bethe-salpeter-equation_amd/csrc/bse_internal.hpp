@@ -13,12 +13,13 @@
 
 // Panels of the one-stage reduction that run in one launch each: from column
 // first on, nwg workgroups at most, messages and counters in ws (zeroed), err
-// (zeroed) as in resident.hpp.
+// (zeroed) as in resident.hpp, big the matrix's largest component.
 struct PanelRun {
     int device, first, nwg;
     double2* ws;
     int64_t ws_el;
     int* err;
+    double* big;
 };
 
 // ---- kernel launchers implemented in the other translation units ----------
@@ -60,7 +61,8 @@ int bse_panel_workgroups(int, int);
 int bse_panel_first(int, int);
 int64_t bse_panel_workspace(int, int);
 hipError_t bse_launch_panel(hipStream_t, int, int, int, int, int, const void*, double2*, double2*, double2*, double2*,
-                            double*, double*, double2*, double2*, int64_t, int*);
+                            double*, double*, double2*, double2*, int64_t, int*, const double*);
+hipError_t bse_launch_copy_max(hipStream_t, int, int, const void*, void*, double*);
 hipError_t bse_launch_hemv(hipStream_t, int, int, int, int, const void*, const double2*, double2*,
                            double2*);
 hipError_t bse_launch_last_diag(hipStream_t, int, int, const void*, double*);

@@ -20,6 +20,10 @@
 //   - the next column is s0 itself, and its update needs row s0 of V and W:
 //     published one step earlier up to the newest column, where V(s0) = 1 and
 //     every owner sums W(s0) itself from the partials of that one row.
+// x^H A x is of third order in the matrix, so x is that column in units of the
+// matrix (times 2^-e, 2^e <= max |a| < 2^(e+1), an exact scaling): without them a matrix
+// of size 1e-129 had x^H A x = 0 and one of 1e120 an infinite one.  d and beta take
+// the 2^e back; everything else is formed from v = e_1 + sc x, which has none.
 //
 // Tiles: NT 64 x 64 tiles of the lower triangle per workgroup, 8 columns of each
 // per wave, kept in registers for the whole panel (the panel does not change
@@ -55,6 +59,7 @@
 // column is bound by the latency of two messages and of about 700 dependent
 // instructions of one wave.
 #include "resident.hpp"
+#include <cfloat>
 
 #define PN_WAVES 8
 #define PN_THREADS (64 * PN_WAVES)
@@ -76,6 +81,7 @@ struct PanelArgs {
     bse_i4v* msg;
     unsigned* meet;
     int* err;
+    const double* big;         // the matrix's largest |Re a|, |Im a| before the first panel
 };
 
 // Message areas, in 16-byte words (two copies each, by the column's parity).
@@ -192,6 +198,10 @@ __global__ __launch_bounds__(PN_THREADS) void k_trd_panel(PanelArgs a)
     const T* A = (const T*)a.A;
     const PanelMsg L = panel_msg(a.nbk, G);
     const __amdgpu_buffer_rsrc_t rm = bse_rsrc(a.msg, (int)(L.total * 16));
+    // units of x: 2^ex (1 for a zero matrix or one that is not finite)
+    const double big = *a.big;
+    const int ex = (big > 0.0 && big <= DBL_MAX) ? max(-1000, min(1000, ilogb(big))) : 0;
+    const double up = ldexp(1.0, -ex), down = ldexp(1.0, ex);
     const bool owner = wg < a.nbk;
     const int grow = R0 + 64 * wg + lane;              // an owner's row of this lane
     int I[NT], J[NT];                                  // tiles wg, wg + G, ..; I < 0: none
@@ -239,7 +249,7 @@ __global__ __launch_bounds__(PN_THREADS) void k_trd_panel(PanelArgs a)
     double2 xown = cmk(0, 0), as0 = cmk(0, 0), as1 = cmk(0, 0);
     double a11 = 0.0, a11n = 0.0;
     if (owner && w < 2) {
-        xown = acol(j0);
+        xown = cscale(acol(j0), up);
         as0 = acol(j0 + 1);
         if (w == 0) {
             a11 = diag(j0 + 1);
@@ -493,6 +503,7 @@ __global__ __launch_bounds__(PN_THREADS) void k_trd_panel(PanelArgs a)
             if (more) {
                 double2 x = csub(csub(as0, xs), cadd(cmul(v, cconj(ws0)), wv));
                 if (grow == s0) x.y = 0.0;
+                x = cscale(x, up);
                 xown = x;
                 if (in) pn_post(rm, L.x + (par ^ 1) * L.xs + (wg * 64 + lane) * 2, x, tag + 1);
                 sX[lane] = pn_sel(in && grow > s0 + 1, x, cmk(0, 0));
@@ -505,8 +516,8 @@ __global__ __launch_bounds__(PN_THREADS) void k_trd_panel(PanelArgs a)
             }
             if (wg == 0) {
                 if (lane == 0) {
-                    a.d[c] = sC[4];
-                    a.e[c] = beta;
+                    a.d[c] = sC[4] * down;
+                    a.e[c] = beta * down;
                     a.tau[c] = tau;
                 }
                 if (lane < i) a.G[lane + (int64_t)i * 64] = cadd(cconj(sRow[1][lane]), cmul(sc, sDot[1][lane]));
@@ -543,6 +554,44 @@ __global__ __launch_bounds__(PN_THREADS) void k_trd_panel(PanelArgs a)
         as0 = as1;
         a11 = a11n;
     }
+}
+
+// dst = src (vec 16-byte vectors of the tiled storage, whose padding is zero) and
+// the largest component's size into *big (zeroed before), NaNs left out.
+template <typename V>
+__global__ __launch_bounds__(256) void k_copy_max(int64_t vec, const V* __restrict__ src, V* __restrict__ dst,
+                                                  unsigned long long* __restrict__ big)
+{
+    __shared__ double sm[4];
+    double m = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < vec; i += (int64_t)gridDim.x * 256) {
+        const V x = src[i];
+        dst[i] = x;
+        m = fmax(m, fmax(fabs((double)x.x), fabs((double)x.y)));
+        if constexpr (sizeof(x.x) == 4) m = fmax(m, fmax(fabs((double)x.z), fabs((double)x.w)));
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) m = fmax(m, __shfl_xor(m, o, 64));
+    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        m = fmax(fmax(sm[0], sm[1]), fmax(sm[2], sm[3]));
+        // sizes of doubles order as their bits do
+        if (m > 0.0) atomicMax(big, (unsigned long long)__double_as_longlong(m));
+    }
+}
+
+extern "C" hipError_t bse_launch_copy_max(hipStream_t st, int fp32, int n, const void* src, void* dst, double* big)
+{
+    const int64_t vec = tiled_elems(n) / (fp32 ? 2 : 1);
+    const dim3 g((unsigned)std::min<int64_t>(ceil_div64(vec, 256), 2048));
+    if (fp32)
+        hipLaunchKernelGGL(k_copy_max<float4>, g, dim3(256), 0, st, vec, (const float4*)src, (float4*)dst,
+                           (unsigned long long*)big);
+    else
+        hipLaunchKernelGGL(k_copy_max<double2>, g, dim3(256), 0, st, vec, (const double2*)src, (double2*)dst,
+                           (unsigned long long*)big);
+    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -634,17 +683,18 @@ extern "C" int64_t bse_panel_workspace(int n, int nwg)
 }
 
 // The panel at j0 (a multiple of 32, >= bse_panel_first).  ws: zeroed before
-// the first panel of a reduction; err: zeroed, set as in resident.hpp.
+// the first panel of a reduction; err: zeroed, set as in resident.hpp; big: from
+// bse_launch_copy_max.
 extern "C" hipError_t bse_launch_panel(hipStream_t st, int device, int fp32, int n, int j0, int nwg, const void* A,
                                        double2* Vp, double2* Wp, double2* alpha2, double2* G, double* d, double* e,
-                                       double2* tau, double2* ws, int64_t ws_el, int* err)
+                                       double2* tau, double2* ws, int64_t ws_el, int* err, const double* big)
 {
     const PanelPlan p = panel_plan(n, j0, nwg);
     const int64_t cnt = ceil_div64(n, PN_B) / 4 + 2;
     if (!p.ok || p.words + cnt > ws_el) return hipErrorInvalidValue;
     unsigned* meet = reinterpret_cast<unsigned*>(ws + (ws_el - cnt)) + j0 / PN_B;
     const PanelArgs args{n, j0, std::min(PN_B, n - 1 - j0), p.tc0, p.nbk, p.ntl, A, Vp, Wp, alpha2, G,
-                         d, e, tau, reinterpret_cast<bse_i4v*>(ws), meet, err};
+                         d, e, tau, reinterpret_cast<bse_i4v*>(ws), meet, err, big};
     return resident_launch(device, st, [&]() -> hipError_t {
         const dim3 g((unsigned)p.grid), t(PN_THREADS);
 #define PN_GO(TT, NT) hipLaunchKernelGGL((k_trd_panel<TT, NT>), g, t, 0, st, args)

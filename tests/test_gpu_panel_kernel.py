@@ -83,6 +83,22 @@ def test_vanishing_reflectors(ctx, prec):
     _check(b, ev, z, np.linalg.eigvalsh(b), tol)
 
 
+@pytest.mark.parametrize("scale", [1e-140, 1e-129, 1e-105, 1e-60, 1e60, 1e101, 1e120, 1e140])
+@pytest.mark.parametrize("n", [70, 200, 1500])
+def test_scale(ctx, n, scale):
+    """The same matrix in other units: x^H A x is of third order in them.  (Below
+    1e-135 the inverse iteration's own squares overflow.)"""
+    print(f"panel kernel n={n} scale={scale}", flush=True)
+    a = _herm(n, n)
+    ref = np.linalg.eigvalsh(a)
+    ev, z = ctx.eigh_dense(a * scale, "fp64", 16)
+    ev = ev / scale
+    assert np.abs(ev - ref).max() < 1e-13 * np.abs(ref).max() * n ** 0.5
+    if scale > 1e-135:
+        assert np.abs(a @ z - z * ev[None, :16]).max() < 1e-12 * np.abs(ref).max() * n ** 0.5
+        assert np.abs(z.conj().T @ z - np.eye(16)).max() < 1e-10
+
+
 def test_two_contexts_at_once():
     import threading
     mats = [_herm(500, 11), _herm(460, 12)]
