@@ -126,7 +126,9 @@ __global__ __launch_bounds__(512) void k_potrf_tile(int n2, int J, double2* __re
                 if (!bad) bad = r0 + j + 1;
                 d = 1.0;
             }
-            const double2 m = cscale(col, rcp_nr(d));
+            // (1 / d of a subnormal pivot would overflow: both sides scaled up)
+            const double us = d < 1e-290 ? 0x1p600 : 1.0;
+            const double2 m = cscale(cscale(col, us), rcp_nr(d * us));
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
                 const int c = 8 * g + q;

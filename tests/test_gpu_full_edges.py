@@ -42,3 +42,16 @@ def test_orders(ctx, grid, k):
     assert np.abs(x.conj().T @ (s3[:, None] * x) - np.eye(k)).max() < 1e-9
     eps = ctx.spectrum(p.omegas, p.eta)
     assert np.linalg.norm(eps - sol["eps"]) < 1e-9 * np.linalg.norm(sol["eps"] - 1.0)
+
+
+@pytest.mark.parametrize("gap", [1e-100, 1e-300, 1e-309, 1e-315])
+def test_tiny_pivots(ctx, gap):
+    """Flat bands without interaction, whose M is the gap times the identity: a
+    positive pivot factors whatever its size, subnormal ones included."""
+    from dataclasses import replace
+    s = bse_amd.honeycomb_plain(6)
+    s = s.with_params(model=replace(s.model, h_r=np.zeros_like(s.model.h_r)), grid=KGrid(5, 7), scissor=gap,
+                      direct_scale=0.0, exchange_scale=0.0)
+    ctx.set_system(s).build_full().eigh_full(-1)
+    # (a few units of the last place of a subnormal number)
+    assert np.abs(ctx.eigenvalues() - gap).max() <= 1e-12 * gap + 2e-323
