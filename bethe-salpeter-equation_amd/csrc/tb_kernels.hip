@@ -195,13 +195,15 @@ __global__ __launch_bounds__(64 * TB_WAVES) void k_tb_states(
             tb_sync();
         }
     }
-    // ascending order (stable); the padding row is not an eigenvalue
+    // ascending order (stable, NaN last, so that ord is a permutation whatever the
+    // values); the padding row is not an eigenvalue
     for (int i = l; i < n; i += S::L) {
         const double x = A[at(i, i)].x;
         int rank = 0;
         for (int j = 0; j < n; ++j) {
             const double y = A[at(j, j)].x;
-            if (y < x || (y == x && j < i)) ++rank;
+            const bool xn = x != x, yn = y != y;
+            if (y < x || (xn && !yn) || ((y == x || (xn && yn)) && j < i)) ++rank;
         }
         ev[i] = x;
         ord[rank] = i;

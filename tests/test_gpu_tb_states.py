@@ -73,3 +73,17 @@ def test_degenerate(ctx, norb):
     flat = replace(two, h_r=np.zeros_like(h))
     e, u = ctx.tb_states_at(k, model=flat)
     assert np.all(e == 0.0)
+
+
+@pytest.mark.parametrize("norb", [2, 3, 5, 16])
+def test_phase_that_is_no_number(ctx, norb):
+    """A k point so far out that its phase overflows: its own energies are NaN (no
+    others in their place), those of the other points in its wave are right."""
+    print(f"states of {norb} orbitals, one k point out of range", flush=True)
+    model = tb.random_square(norb, seed=norb)
+    k = np.random.default_rng(norb).uniform(-2, 2, size=(3, 9))
+    k[:, 4] = [1.5e308, 1.5e308, 0.0]
+    e, u = ctx.tb_states_at(k, model=model)
+    assert np.all(np.isnan(e[4]))
+    ok = np.delete(np.arange(9), 4)
+    _check(model, k[:, ok], e[ok], u[ok])
