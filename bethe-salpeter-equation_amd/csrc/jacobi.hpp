@@ -21,7 +21,7 @@ __device__ inline JacobiRot jacobi_rot(double app, double aqq, double2 a) {
     JacobiRot t;
     const double h0 = 0.5 * (aqq - app);
     const double big = fmax(fabs(h0), fmax(fabs(a.x), fabs(a.y)));
-    const bool act = (a.x != 0.0 || a.y != 0.0) && big > 0.0;
+    const bool act = a.x != 0.0 || a.y != 0.0;          // (a NaN goes on into c and s)
     int ex;
     (void)frexp(act ? big : 1.0, &ex);
     const double h = ldexp(h0, -ex);

@@ -84,6 +84,6 @@ def test_phase_that_is_no_number(ctx, norb):
     k = np.random.default_rng(norb).uniform(-2, 2, size=(3, 9))
     k[:, 4] = [1.5e308, 1.5e308, 0.0]
     e, u = ctx.tb_states_at(k, model=model)
-    assert np.all(np.isnan(e[4]))
+    assert np.all(np.isnan(e[4])) and np.all(np.isnan(u[4]).any(axis=-1))
     ok = np.delete(np.arange(9), 4)
     _check(model, k[:, ok], e[ok], u[ok])
