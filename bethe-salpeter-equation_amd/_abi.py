@@ -28,7 +28,7 @@ ABI_SYMBOLS = (
     "bse_batch_prepare", "bse_batch_run", "bse_batch_results", "bse_batch_info",
     "bse_grad_spectrum", "bse_refine_info", "bse_set_problem_klist", "bse_tb_states_at",
     "bse_eigh_dense_noalloc", "bse_noalloc_info", "bse_build_full", "bse_eigh_full", "bse_get_coupling",
-    "bse_wannier_integrals", "bse_probe_rate",
+    "bse_wannier_integrals", "bse_probe_rate", "bse_reduction_info",
 )
 
 
@@ -165,6 +165,7 @@ def load_library(path: pathlib.Path | str | None = None):
         "bse_wannier_integrals": (i32, [vp, C.POINTER(WannierGridC), i32, C.POINTER(C.c_int32), i32, dp,
                                         dp, dp, dp]),
         "bse_probe_rate": (i32, [i32, dp]),
+        "bse_reduction_info": (i32, [vp, C.POINTER(C.c_int)]),
     }
     for name, (res, args) in sig.items():
         fn = getattr(lib, name)
@@ -497,6 +498,17 @@ class Context:
         return dict(kind="bytes", kernel="kb_hemv (every variant the tuner picks)", ms=out[0],
                     bytes=out[1], launches=int(out[2]), hemv_ms=out[0], hemv_bytes=out[1],
                     hemv_launches=int(out[2]))
+
+    def reduction_info(self):
+        """How the last eigensolve reduced its matrix: the reduction, whether its
+        panels ran in one launch each, the form of the bulge chase, and what a
+        resident kernel that was given up reported (0: none)."""
+        out = (C.c_int * 4)()
+        self._check(self.lib.bse_reduction_info(self.h, out), "bse_reduction_info")
+        return dict(reduction=("one stage", "two stages", "two stages, reflectors kept")[out[0]],
+                    panels=("none", "ran", "repeated")[out[1]],
+                    chase=("none", "resident", "tasks", "tasks after refusal", "one stage after refusal")[out[2]],
+                    reason=out[3])
 
     def stage_times(self):
         out = np.zeros(len(STAGES))

@@ -107,6 +107,12 @@ extern "C" int bse_profile(bse_ctx* ctx, int enable, double* out) {
     return BSE_OK;
 }
 
+extern "C" int bse_reduction_info(const bse_ctx* ctx, int out[4]) {
+    if (!ctx || !out) return BSE_ERR_ARG;
+    for (int i = 0; i < 4; ++i) out[i] = ctx->red_info[i];
+    return BSE_OK;
+}
+
 extern "C" int bse_problem_sizes(const bse_ctx* ctx, int64_t out[4]) {
     if (!ctx || !out) return BSE_ERR_ARG;
     out[0] = ctx->nk; out[1] = ctx->N; out[2] = ctx->norb; out[3] = ctx->ng;
@@ -711,6 +717,13 @@ static bool use_q2(const bse_ctx* ctx, int n, int n_vectors, int vec_first, int 
            bse_chase_resident_workspace(n, kBand, 2 * kBand + 1, ctx->device) > 0;
 }
 
+// BSE_RESIDENT_REFUSE=panel or chase: that resident kernel leaves as if its
+// workgroups had not met (tests of the paths that serve then).
+static bool resident_refused(const char* kernel) {
+    const char* r = getenv("BSE_RESIDENT_REFUSE");
+    return r && !strcmp(r, kernel);
+}
+
 // V2 (may be null): the chase's reflectors are wanted.  Returns kNotResident,
 // with H as it was, when they could not be had (the resident chase did not run).
 static const int kNotResident = 1;
@@ -878,13 +891,16 @@ static int twostage_tridiag(bse_ctx* ctx, int n, void* H, int fp32, const double
     // band with more workgroups than the device holds, or a device that did
     // not hold them together) takes one wave per sweep instead
     const char* che = getenv("BSE_CHASE");
+    const bool refuse = resident_refused("chase");
     const int64_t mel = (che && !strcmp(che, "tasks")) ? 0 : bse_chase_resident_workspace(n, b, ldab, ctx->device);
     if (mel > 0) {
         double2* msg = BUF(double2, S_BMSG, mel);
-        HCK(bse_launch_chase_resident(st, ctx->device, n, b, AB, ldab, y, d, e, msg, prog + ncnt, V2));
+        HCK(bse_launch_chase_resident(st, ctx->device, n, b, AB, ldab, y, d, e, msg, prog + ncnt, V2, refuse));
         HCK(hipEventRecord(tv[2], st));
         HCK(hipMemcpyAsync(&err, prog + ncnt, sizeof(int), hipMemcpyDeviceToHost, st));
         HCK(hipStreamSynchronize(st));
+        ctx->red_info[2] = err == 2 ? (V2 ? 4 : 3) : 1;
+        ctx->red_info[3] = err;
         if (err == 2 && V2) {
             if (npan > 0)
                 HCK(hipMemcpyAsync(H, ctx->bufs[S_BH0].p, (size_t)tiled_elems(n) * (fp32 ? sizeof(float2) : sizeof(double2)),
@@ -900,6 +916,7 @@ static int twostage_tridiag(bse_ctx* ctx, int n, void* H, int fp32, const double
         // predecessor runs); BSE_CHASE_GRID sets the count for measurements
         int cgrid = std::max(1, ncu - 16);
         if (const char* g = getenv("BSE_CHASE_GRID")) cgrid = std::max(1, std::min(atoi(g), ncu));
+        if (mel <= 0) ctx->red_info[2] = 2;
         HCK(bse_launch_chase(st, n, b, AB, ldab, y, d, e, prog, prog + ncnt, cgrid));
         HCK(hipEventRecord(tv[2], st));
         HCK(hipMemcpyAsync(&err, prog + ncnt, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -1034,6 +1051,7 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
         two = V2 != nullptr;
     }
     ctx->stage_ms[ST_BAND] = ctx->stage_ms[ST_CHASE] = 0.0;
+    for (int& r : ctx->red_info) r = 0;
     if (ctx->prof) ctx->prof_two_stage = false;
     // ---------------- K5: tridiagonalisation
     int64_t vs_el = 1, yr_el = 1, yc_el = 1, part_d = 1;
@@ -1053,6 +1071,7 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     }
     const bool q2 = two && V2 != nullptr;
     ctx->last_two_stage = two;
+    ctx->red_info[0] = q2 ? 2 : (two ? 1 : 0);
     if (two) {
         d = (double*)ctx->bufs[S_D].p;
         e = (double*)ctx->bufs[S_E].p;
@@ -1102,7 +1121,7 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     const char* pne = getenv("BSE_TRD_PANEL");
     const int pnwg = ((pne && pne[0] == '0') || getenv("BSE_HEMV_CODE")) ? 0 : bse_panel_workgroups(ctx->device, fp32);
     PanelRun prun{ctx->device, n, pnwg, nullptr, pnwg > 0 ? bse_panel_workspace(n, pnwg) : 0, nullptr,
-                  nullptr};
+                  nullptr, resident_refused("panel")};
     const size_t hbytes = (size_t)tiled_elems(n) * (fp32 ? sizeof(float2) : sizeof(double2));
     void* H0 = nullptr;
     if (prun.ws_el > 0) {
@@ -1138,7 +1157,9 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
         int perr = 0;
         HCK(hipMemcpyAsync(&perr, prun.err, sizeof(int), hipMemcpyDeviceToHost, st));
         HCK(hipStreamSynchronize(st));
+        ctx->red_info[1] = perr ? 2 : 1;
         if (perr) {
+            ctx->red_info[3] = perr;
             HCK(hipMemcpyAsync(H, H0, hbytes, hipMemcpyDeviceToDevice, st));
             int rc = autotune_hemv(ctx, fp32, n, H, acol, Yr, Yc);
             if (rc) return rc;

@@ -20,6 +20,7 @@ struct PanelRun {
     int64_t ws_el;
     int* err;
     double* big;
+    int refuse;                // tests: the last panel leaves as if not resident
 };
 
 // ---- kernel launchers implemented in the other translation units ----------
@@ -61,7 +62,7 @@ int bse_panel_workgroups(int, int);
 int bse_panel_first(int, int);
 int64_t bse_panel_workspace(int, int);
 hipError_t bse_launch_panel(hipStream_t, int, int, int, int, int, const void*, double2*, double2*, double2*, double2*,
-                            double*, double*, double2*, double2*, int64_t, int*, const double*);
+                            double*, double*, double2*, double2*, int64_t, int*, const double*, int);
 hipError_t bse_launch_copy_max(hipStream_t, int, int, const void*, void*, double*);
 hipError_t bse_launch_hemv(hipStream_t, int, int, int, int, const void*, const double2*, double2*,
                            double2*);
@@ -126,7 +127,7 @@ hipError_t bse_launch_her2k_part(hipStream_t, int, int, int, int, int, void*, co
                                  int64_t, int, int, const double2*);
 int64_t bse_chase_resident_workspace(int, int, int, int);
 hipError_t bse_launch_chase_resident(hipStream_t, int, int, int, const double2*, int, double2*, double*, double*,
-                                     double2*, int*, double2*);
+                                     double2*, int*, double2*, int);
 int64_t bse_q2_workspace(int);
 hipError_t bse_apply_q2(hipStream_t, int, const double2*, double2*, int64_t, int);
 int64_t bse_chase_counters(int);
@@ -275,6 +276,7 @@ struct bse_ctx {
     // (row start, rows, reflectors, offset into the reflector store)
     int two_stage = 0;
     bool last_two_stage = false;
+    int red_info[4] = {0, 0, 0, 0};     // bse_reduction_info
     // full (non-Tamm-Dancoff) BSE state: M composed; last eig was of it
     bool full_built = false, full_eig = false, have_coupling = false;
     int64_t full_ldx = 0;

@@ -770,10 +770,10 @@ hipError_t resident_launch(int device, hipStream_t st, const std::function<hipEr
 }
 
 // err receives 0, 1 (a wait was given up) or 2 (the workgroups did not become
-// resident together: AB, y, d and e are as they were).
+// resident together, or refuse: AB, y, d and e are as they were).
 extern "C" hipError_t bse_launch_chase_resident(hipStream_t st, int device, int n, int b, const double2* AB,
                                                 int ldab, double2* y, double* d, double* e, double2* ws, int* err,
-                                                double2* V2)
+                                                double2* V2, int refuse)
 {
     const int grid = chase_resident_grid(n, b, ldab, device);
     if (grid == 0) return hipErrorInvalidValue;
@@ -781,6 +781,7 @@ extern "C" hipError_t bse_launch_chase_resident(hipStream_t st, int device, int 
     const int64_t words = (int64_t)npos * CHS_SLOT;
     hipError_t rc = bse_launch_zero_words(st, 2 * (words + 1), ws);
     if (rc != hipSuccess) return rc;
+    if (refuse && (rc = rs_refuse(st, reinterpret_cast<unsigned*>(ws + words))) != hipSuccess) return rc;
     const ChaseSysArgs args{n, ldab, npos, AB, y, d, e, reinterpret_cast<bse_i4v*>(ws),
                             reinterpret_cast<unsigned*>(ws + words), err, V2};
     return resident_launch(device, st, [&]() -> hipError_t {

@@ -1458,7 +1458,7 @@ extern "C" hipError_t bse_hetrd(hipStream_t st, int fp32, int n, void* A, int nb
             double2* Vp = Vstore + panel_voff(n, nb, p);
             if ((err = bse_launch_panel(st, run->device, fp32, n, j0, run->nwg, A, Vp, Wp, alpha2,
                                         G + (int64_t)p * 64 * 64, d, e, tau, run->ws, run->ws_el, run->err,
-                                        run->big)) != hipSuccess)
+                                        run->big, run->refuse)) != hipSuccess)
                 return err;
             if ((err = bse_launch_her2k(st, fp32, her2k_kind, n, j0 + nbp, A, Vp, Wp, n - j0, j0, nbp, alpha2)) !=
                 hipSuccess)

@@ -684,15 +684,20 @@ extern "C" int64_t bse_panel_workspace(int n, int nwg)
 
 // The panel at j0 (a multiple of 32, >= bse_panel_first).  ws: zeroed before
 // the first panel of a reduction; err: zeroed, set as in resident.hpp; big: from
-// bse_launch_copy_max.
+// bse_launch_copy_max; refuse: the last panel is refused (rs_refuse).
 extern "C" hipError_t bse_launch_panel(hipStream_t st, int device, int fp32, int n, int j0, int nwg, const void* A,
                                        double2* Vp, double2* Wp, double2* alpha2, double2* G, double* d, double* e,
-                                       double2* tau, double2* ws, int64_t ws_el, int* err, const double* big)
+                                       double2* tau, double2* ws, int64_t ws_el, int* err, const double* big,
+                                       int refuse)
 {
     const PanelPlan p = panel_plan(n, j0, nwg);
     const int64_t cnt = ceil_div64(n, PN_B) / 4 + 2;
     if (!p.ok || p.words + cnt > ws_el) return hipErrorInvalidValue;
     unsigned* meet = reinterpret_cast<unsigned*>(ws + (ws_el - cnt)) + j0 / PN_B;
+    if (refuse && j0 + PN_B >= n - 1) {
+        const hipError_t rc = rs_refuse(st, meet);
+        if (rc != hipSuccess) return rc;
+    }
     const PanelArgs args{n, j0, std::min(PN_B, n - 1 - j0), p.tc0, p.nbk, p.ntl, A, Vp, Wp, alpha2, G,
                          d, e, tau, reinterpret_cast<bse_i4v*>(ws), meet, err, big};
     return resident_launch(device, st, [&]() -> hipError_t {

@@ -35,6 +35,13 @@ __device__ inline bse_i4v rs_word(double v, int tag) {
 __device__ inline bool rs_here(bse_i4v w, int tag) { return w[1] == tag && w[3] == tag; }
 __device__ inline double rs_value(bse_i4v w) { return __hiloint2double(w[2], w[0]); }
 
+// The host's refusal, for tests of what follows one: the counter starts with the
+// abort bit, so every workgroup leaves from rs_meet.
+inline hipError_t rs_refuse(hipStream_t st, unsigned* meet) {
+    static const unsigned abort_bit = RS_ABORT;
+    return hipMemcpyAsync(meet, &abort_bit, sizeof(abort_bit), hipMemcpyHostToDevice, st);
+}
+
 // All workgroups resident?  An arrival adds one; a workgroup that has waited
 // too long sets RS_ABORT, and only while the count is short (compare and
 // swap), so either every workgroup sees the full count or every one leaves.

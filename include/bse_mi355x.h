@@ -283,6 +283,16 @@ int  bse_eigh_dense(bse_ctx* ctx, int n, const double* a, int64_t lda, int a_on_
  * parts of [3] (0 after a one-stage reduction).  n <= 16. */
 int  bse_stage_times(const bse_ctx* ctx, double* ms, int n);
 
+/* How the last eigensolve reduced its matrix to tridiagonal form: out[0] 0 one
+ * stage, 1 two stages, 2 two stages with the bulge chase's reflectors kept;
+ * out[1] panels of the one-stage reduction in one launch each: 0 none, 1 they
+ * ran, 2 given up and the reduction repeated by columns; out[2] bulge chase: 0
+ * none, 1 resident in LDS, 2 one wave per sweep, 3 one wave per sweep and 4 the
+ * one-stage reduction after the resident form had been given up; out[3] why
+ * (0; 1 a wait inside the kernel was given up, 2 not all workgroups became
+ * resident at once). */
+int  bse_reduction_info(const bse_ctx* ctx, int out[4]);
+
 /* Kernel-level profile of the tridiagonalisation's dominant kernels (HIP
  * events around every launch on the context stream).  enable switches
  * recording on for later calls; out (may be NULL, else 9 doubles) receives,

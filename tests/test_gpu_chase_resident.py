@@ -26,6 +26,9 @@ def ctx2():
     c.close()
 
 
+RESIDENT = dict(reduction="two stages", panels="none", chase="resident", reason=0)
+
+
 @pytest.mark.parametrize("n", [2, 3, 31, 32, 33, 34, 35, 63, 64, 65, 66, 67, 97, 98, 129, 258, 290, 545])
 def test_same_eigenvalues(ctx2, monkeypatch, n):
     print(f"resident chase n={n}", flush=True)
@@ -33,8 +36,10 @@ def test_same_eigenvalues(ctx2, monkeypatch, n):
     a = rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n))
     a = 0.5 * (a + a.conj().T)
     ev, _ = ctx2.eigh_dense(a, "fp64", 0)
+    assert ctx2.reduction_info() == RESIDENT
     monkeypatch.setenv("BSE_CHASE", "tasks")
     ev2, _ = ctx2.eigh_dense(a, "fp64", 0)
+    assert ctx2.reduction_info() == dict(RESIDENT, chase="tasks")
     ref = np.linalg.eigvalsh(a)
     tol = 1e-13 * np.abs(ref).max() * n ** 0.5
     assert np.abs(ev - ev2).max() < tol
@@ -49,12 +54,33 @@ def test_same_oscillator_strengths(ctx2, monkeypatch, grid):
     om = s.omegas()
     print(f"resident chase y, grid {grid}", flush=True)
     ctx2.set_system(s).build("fp64").eigh(1)
+    assert ctx2.reduction_info() == RESIDENT
     e, eps = ctx2.eigenvalues(), ctx2.spectrum(om, s.eta)
     monkeypatch.setenv("BSE_CHASE", "tasks")
     ctx2.set_system(s).build("fp64").eigh(1)
     e2, eps2 = ctx2.eigenvalues(), ctx2.spectrum(om, s.eta)
     assert np.abs(e - e2).max() < 1e-12 * np.abs(e2).max()
     assert np.linalg.norm(eps - eps2) < 1e-11 * np.linalg.norm(eps2 - 1)
+
+
+@pytest.mark.parametrize("grid", [(1, 2), (5, 13), (14, 23)])
+def test_refused(ctx2, monkeypatch, grid):
+    """The resident chase leaves as if not resident, with the band and y untouched:
+    one wave per sweep serves, with its own results bit for bit."""
+    s = bse_amd.honeycomb_plain(6).with_params(grid=KGrid(*grid))
+    om = s.omegas()
+    print(f"resident chase refused, grid {grid}", flush=True)
+    res = []
+    for name, value, chase in (("BSE_RESIDENT_REFUSE", "chase", "tasks after refusal"),
+                               ("BSE_CHASE", "tasks", "tasks")):
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setenv(name, value)
+            ctx2.set_system(s).build("fp64").eigh(1)
+        info = ctx2.reduction_info()
+        assert info["chase"] == chase and info["reason"] == (2 if "after" in chase else 0)
+        res.append((ctx2.eigenvalues(), ctx2.spectrum(om, s.eta), ctx2.eigenvectors(1)))
+    for a, b in zip(*res):
+        assert np.array_equal(a, b)
 
 
 @pytest.mark.parametrize("two_stage", ["0", "1"])

@@ -1,7 +1,6 @@
 """Many eigenvectors through the two-stage reduction: the bulge chase's
 reflectors applied to the tridiagonal vectors, at the edges of their 32-sweep
-blocks, of the 128 sweeps of a pass and of the column strips (16 columns, and 32
-where the columns fill the chip).
+blocks, of the 128 sweeps of a pass and of the column strips (16 columns).
 
 Vectors of a unitary similarity transform in FP64: residual and orthogonality
 to 1e-12 sqrt(n) of the norm, as for the other back-transforms.
@@ -32,12 +31,16 @@ def _herm(n):
     return 0.5 * (a + a.conj().T)
 
 
+KEPT = dict(reduction="two stages, reflectors kept", panels="none", chase="resident", reason=0)
+
+
 @pytest.mark.parametrize("n", [21, 31, 32, 33, 34, 35, 63, 64, 65, 66, 97, 98, 128, 129, 130, 161, 258, 290, 545])
 @pytest.mark.parametrize("nvec", [21, -1])
 def test_orders(ctx2, n, nvec):
     print(f"many vectors n={n} nvec={nvec}", flush=True)
     a = _herm(n)
     ev, z = ctx2.eigh_dense(a, "fp64", nvec)
+    assert ctx2.reduction_info() == KEPT
     ref = np.linalg.eigvalsh(a)
     k, tol = z.shape[1], 1e-12 * n ** 0.5
     assert np.abs(ev - ref).max() < tol * np.abs(ref).max()
@@ -53,11 +56,15 @@ def test_smallest(ctx2, n):
     assert np.abs(a @ z - z * ev[None, :]).max() < 1e-13 * n * max(np.abs(ev).max(), 1.0)
 
 
-def test_wide_strips(ctx2):
+def test_chosen_by_order():
+    """An order beyond the line of the automatic choice, with 33 passes of 128
+    sweeps and a last strip of two columns."""
     n = 4130
     print(f"many vectors n={n}", flush=True)
     a = _herm(n)
-    ev, z = ctx2.eigh_dense(a, "fp64", -1)
+    with _abi.Context(0) as c:
+        ev, z = c.eigh_dense(a, "fp64", -1)
+        assert c.reduction_info() == KEPT
     pick = np.unique(np.r_[np.arange(0, n, 41), n - 33:n])
     zp = z[:, pick]
     tol = 1e-12 * n ** 0.5
@@ -121,7 +128,24 @@ def test_without_the_resident_chase(ctx2, monkeypatch):
     a = _herm(200)
     monkeypatch.setenv("BSE_CHASE", "tasks")
     ev, z = ctx2.eigh_dense(a, "fp64", -1)
+    assert ctx2.reduction_info()["reduction"] == "one stage"
     assert np.abs(a @ z - z * ev[None, :]).max() < 1e-11 * np.abs(ev).max()
+
+
+@pytest.mark.parametrize("n", [21, 40, 200, 545])
+def test_refused(ctx2, monkeypatch, n):
+    """The chase leaves as if not resident: the matrix, by then a band matrix, is
+    taken from its copy and reduced in one stage."""
+    print(f"many vectors refused n={n}", flush=True)
+    a = _herm(n)
+    monkeypatch.setenv("BSE_RESIDENT_REFUSE", "chase")
+    ev, z = ctx2.eigh_dense(a, "fp64", -1)
+    assert ctx2.reduction_info() == dict(reduction="one stage", panels="ran", chase="one stage after refusal", reason=2)
+    ref = np.linalg.eigvalsh(a)
+    tol = 1e-12 * n ** 0.5
+    assert np.abs(ev - ref).max() < tol * np.abs(ref).max()
+    assert np.abs(a @ z - z * ev[None, :]).max() < tol * np.abs(ref).max()
+    assert np.abs(z.conj().T @ z - np.eye(n)).max() < tol
 
 
 @pytest.mark.parametrize("grid", [(5, 7), (8, 13), (11, 12)])

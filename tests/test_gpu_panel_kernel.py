@@ -1,8 +1,8 @@
 """One-stage reduction with a panel per launch (resident workgroups) against
 LAPACK and against the per-column launches: orders around the 32-column panels
-and 64-row tiles, the change from one tile to 2 x 2 tiles per workgroup (22
-tile rows), several groups of tiles per workgroup, both storage types, and
-matrices whose reflectors vanish.
+and 64-row tiles, the change from one tile per workgroup (up to 22
+tile rows) to two, three and four, both storage types, matrices whose reflectors
+vanish, and a panel that is refused.
 
 Eigenvalues of a unitary similarity transform computed in FP64 are good to a
 modest multiple of eps ||A||: 1e-13 sqrt(n) of the norm, as for the per-column
@@ -32,6 +32,9 @@ def _herm(n, seed):
     return 0.5 * (a + a.conj().T)
 
 
+RAN = dict(reduction="one stage", panels="ran", chase="none", reason=0)
+
+
 def _check(a, ev, z, ref, tol):
     n = a.shape[0]
     scale = max(np.abs(ref).max(), 1e-300)
@@ -46,6 +49,7 @@ def test_orders(ctx, n, prec):
     print(f"panel kernel n={n} {prec}", flush=True)
     a = _herm(n, n)
     ev, z = ctx.eigh_dense(a, prec)
+    assert ctx.reduction_info() == RAN
     _check(a, ev, z, np.linalg.eigvalsh(a), 1e-13 if prec == "fp64" else 2e-6)
 
 
@@ -55,12 +59,30 @@ def test_against_column_launches(ctx, monkeypatch, n, prec):
     print(f"panel kernel n={n} {prec}", flush=True)
     a = _herm(n, n)
     ev, z = ctx.eigh_dense(a, prec, 8)
+    assert ctx.reduction_info() == RAN
     monkeypatch.setenv("BSE_TRD_PANEL", "0")
     ev2, _ = ctx.eigh_dense(a, prec, 8)
+    assert ctx.reduction_info()["panels"] == "none"
     scale = np.abs(ev2).max()
     assert np.abs(ev - ev2).max() < (1e-13 if prec == "fp64" else 2e-7) * scale * n ** 0.5
     tol = 1e-12 if prec == "fp64" else 1e-5
     assert np.abs(a @ z - z * ev[None, :8]).max() < tol * scale * n ** 0.5
+
+
+@pytest.mark.parametrize("n", [2, 70, 333, 1500, 2960])
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_refused(ctx, monkeypatch, n, prec):
+    """The last panel leaves as if not resident: the matrix, changed by the panels
+    before it, is taken from its copy and reduced by columns."""
+    print(f"panel kernel refused n={n} {prec}", flush=True)
+    a = _herm(n, n)
+    monkeypatch.setenv("BSE_RESIDENT_REFUSE", "panel")
+    ev, z = ctx.eigh_dense(a, prec, min(n, 8))
+    assert ctx.reduction_info() == dict(RAN, panels="repeated", reason=2)
+    monkeypatch.delenv("BSE_RESIDENT_REFUSE")
+    monkeypatch.setenv("BSE_TRD_PANEL", "0")
+    ev2, z2 = ctx.eigh_dense(a, prec, min(n, 8))
+    assert np.array_equal(ev, ev2) and np.array_equal(z, z2)      # the same launches
 
 
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
