@@ -726,8 +726,9 @@ static bool resident_refused(const char* kernel) {
 
 // V2 (may be null): the chase's reflectors are wanted.  Returns kNotResident,
 // with H as it was, when they could not be had (the resident chase did not run).
+// *saved is set once H, which is overwritten, is in S_BH0.
 static const int kNotResident = 1;
-static int twostage_tridiag(bse_ctx* ctx, int n, void* H, int fp32, const double2* rho, double2* V2 = nullptr) {
+static int twostage_tridiag(bse_ctx* ctx, int n, void* H, int fp32, const double2* rho, double2* V2, bool* saved) {
     hipStream_t st = ctx->st;
     const int b = kBand, ldab = 2 * b + 1;
     double* d = BUF(double, S_D, n);
@@ -805,6 +806,7 @@ static int twostage_tridiag(bse_ctx* ctx, int n, void* H, int fp32, const double
         const size_t hbytes = (size_t)tiled_elems(n) * (fp32 ? sizeof(float2) : sizeof(double2));
         void* H0 = BUF(char, S_BH0, hbytes);
         HCK(hipMemcpyAsync(H0, H, hbytes, hipMemcpyDeviceToDevice, st));
+        *saved = true;
         int tsqr = 0;
         // factor panel q on stream sq; apply its reflectors to y = Q^H rho
         auto factor = [&](hipStream_t sq, int q) -> int {
@@ -1013,27 +1015,47 @@ static int twostage_vectors_rest(bse_ctx* ctx, hipStream_t st, int n, int nstore
     return BSE_OK;
 }
 
-// Whether `extra` bytes beside what a solve with nvec vectors will still allocate
-// (its vectors, reflectors and inverse-iteration scratch) are there: a faster path
-// must not take the memory that the solve needs.  Orders up to 16384 need at most
-// a tenth of the device's memory and are not asked about.
-static bool memory_to_spare(const bse_ctx* ctx, int n, int nvec, double extra) {
-    if (n <= 16384) return true;
+// What one eigensolve keeps beyond what it needs: the chase's reflectors, the
+// copy of the matrix behind the one-launch panels.
+struct EigMemory {
+    bool lean = false;     // take no such path
+    bool taken = false;    // such a buffer is held
+    bool saved = false;    // the matrix, overwritten since, is in S_BH0
+};
+
+// Whether there is room for the buffers `want` of a faster path beside what a
+// solve with nvec vectors will still allocate (its vectors, reflectors,
+// inverse-iteration scratch, and a margin for the smaller ones): such a path must
+// not take the memory that the solve needs.  Buffers that are held already are
+// not asked about (eig_pipeline gives them back if the solve runs short).
+static bool memory_to_spare(const bse_ctx* ctx, int n, int nvec, const EigMemory& mem,
+                            std::initializer_list<std::pair<int, size_t>> want) {
+    if (mem.lean) return false;
+    if (ctx->arena_base) return true;                    // buf decides
+    double need = 0.0, have = 0.0;
+    bool held = true;
+    for (const auto& w : want) {
+        held = held && ctx->bufs[w.first].cap >= w.second;
+        need += (double)w.second;
+        have += (double)ctx->bufs[w.first].cap;
+    }
+    if (held) return true;
     size_t free_b = 0, total = 0;
     if (hipMemGetInfo(&free_b, &total) != hipSuccess) return true;
+    const size_t sum = held_bytes(ctx);
+    have += (double)std::min(free_b, ctx->mem_limit - std::min(sum, ctx->mem_limit));
+    for (int slot : {S_Z, S_VSTORE, S_IISCR, S_IIX}) have += (double)ctx->bufs[slot].cap;
     const double dn = n, batch = std::min(dn, std::max(4096.0, 24e9 / (48.0 * dn)));
-    double have = (double)free_b;
-    for (int slot : {S_Z, S_VSTORE, S_IISCR, S_IIX, S_BH0, S_Q2V}) have += (double)ctx->bufs[slot].cap;
-    return extra + 16.0 * dn * nvec + 8.0 * dn * dn + 48.0 * dn * batch + 4e9 <= have;
+    const double margin = std::min(4e9, 1e8 + 64.0 * dn * dn);
+    return need + 16.0 * dn * nvec + 8.0 * dn * dn + 48.0 * dn * batch + margin <= have;
 }
 
 // guard_tol > 0: eigenvalues within guard_tol above the last requested one
 // are formed as well, up to max_vectors in total (ctx->nvec reports the count).
 // vec_first > 0: the vectors formed are those of the sorted eigenvalues
 // vec_first .. vec_first + n_vectors - 1 (one-stage reduction, no guard).
-static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
-                        const double2* rho, int n_vectors, double guard_tol = 0.0,
-                        int max_vectors = 0, int vec_first = 0)
+static int eig_attempt(bse_ctx* ctx, int64_t n64, void* H, int fp32, const double2* rho, int n_vectors,
+                       double guard_tol, int max_vectors, int vec_first, EigMemory& mem)
 {
     const int n = (int)n64;
     const int nb = kPanel;
@@ -1044,11 +1066,11 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     double2* V2 = nullptr;
     const int nvec_max = (n_vectors < 0) ? n : std::min(n, std::max(n_vectors, max_vectors));
     if (!two && use_q2(ctx, n, n_vectors, vec_first, max_vectors, fp32) &&
-        memory_to_spare(ctx, n, nvec_max, 16.0 * (double)n * n)) {
+        memory_to_spare(ctx, n, nvec_max, mem, {{S_Q2V, sizeof(double2) * (size_t)bse_q2_workspace(n)},
+                                                {S_BH0, sizeof(double2) * (size_t)tiled_elems(n)}})) {
         int no = BSE_OK;
         V2 = bufT<double2>(ctx, S_Q2V, (size_t)bse_q2_workspace(n), &no);
-        if (!V2) (void)hipGetLastError();
-        two = V2 != nullptr;
+        two = mem.taken = V2 != nullptr;
     }
     ctx->stage_ms[ST_BAND] = ctx->stage_ms[ST_CHASE] = 0.0;
     for (int& r : ctx->red_info) r = 0;
@@ -1065,7 +1087,7 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     double* e = nullptr;
     if (two) {
         stage_begin(ctx, ST_TRD);
-        int rc2 = twostage_tridiag(ctx, n, H, fp32, rho, V2);
+        int rc2 = twostage_tridiag(ctx, n, H, fp32, rho, V2, &mem.saved);
         if (rc2 == kNotResident) two = false;
         else if (rc2) return rc2;
     }
@@ -1126,11 +1148,9 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     void* H0 = nullptr;
     if (prun.ws_el > 0) {
         int no = BSE_OK;
-        if (memory_to_spare(ctx, n, nvec_max, (double)hbytes)) H0 = buf(ctx, S_BH0, hbytes, &no);
-        if (!H0) {
-            (void)hipGetLastError();
-            prun.ws_el = 0;                 // no room for the copy: per-column launches
-        }
+        if (memory_to_spare(ctx, n, nvec_max, mem, {{S_BH0, hbytes}})) H0 = buf(ctx, S_BH0, hbytes, &no);
+        if (!H0) prun.ws_el = 0;            // no room for the copy: per-column launches
+        else mem.taken = true;
     }
     if (prun.ws_el > 0) {
         prun.first = bse_panel_first(n, pnwg);
@@ -1140,6 +1160,7 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
         prun.big = reinterpret_cast<double*>(prun.err + 2);
         HCK(bse_launch_zero_words(st, 2, prun.err));
         HCK(bse_launch_copy_max(st, fp32, n, H, H0, prun.big));
+        mem.saved = true;
     }
     const int panel_first = prun.ws_el > 0 ? prun.first : n;
     {
@@ -1445,7 +1466,8 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
         }
     } else if (nstore > 0 && nstore <= 16 && bse_apply_q_thin_workspace(n) <= sk_el) {
         HCK(bse_apply_q_thin(st, n, nb, Vst, Tall, nstore, Z, n, 0, skw));
-    } else if (nstore > 16 && n >= kGroupedMinN && nb == 32 && !getenv("BSE_BT_STRIPS")) {
+    } else if ((mem.lean ? nstore >= 2048 : nstore > 16 && n >= kGroupedMinN) && nb == 32 &&
+               !getenv("BSE_BT_STRIPS")) {
         // many vectors: four panels per pass on FP64 matrix cores
         int64_t* voff_d = BUF(int64_t, S_BTVOFF, npan);
         HCK(hipMemcpyAsync(voff_d, voff.data(), sizeof(int64_t) * npan, hipMemcpyHostToDevice, st));
@@ -1477,6 +1499,30 @@ static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32,
     ctx->have_eig = true;
     ctx->have_f = (rho != nullptr);
     return BSE_OK;
+}
+
+static int eig_pipeline(bse_ctx* ctx, int64_t n64, void* H, int fp32, const double2* rho, int n_vectors,
+                        double guard_tol = 0.0, int max_vectors = 0, int vec_first = 0)
+{
+    const char* ml = getenv("BSE_MEMORY_LIMIT");
+    ctx->mem_limit = (ml && ml[0]) ? (size_t)strtoull(ml, nullptr, 10) : SIZE_MAX;
+    EigMemory mem;
+    const int rc = eig_attempt(ctx, n64, H, fp32, rho, n_vectors, guard_tol, max_vectors, vec_first, mem);
+    if (rc != BSE_ERR_ALLOC || !mem.taken || ctx->arena_base) return rc;
+    // what the faster path keeps took the memory that the solve needs: give it
+    // back and solve without
+    HCK(hipStreamSynchronize(ctx->side));
+    if (mem.saved)
+        HCK(hipMemcpyAsync(H, ctx->bufs[S_BH0].p, (size_t)tiled_elems(n64) * (fp32 ? sizeof(float2) : sizeof(double2)),
+                           hipMemcpyDeviceToDevice, ctx->st));
+    HCK(hipStreamSynchronize(ctx->st));
+    for (int slot : {S_Q2V, S_BH0, S_PNMSG, S_BAB, S_BAB0, S_BPAN, S_BTSQR, S_BUPD, S_BPROG, S_BMSG, S_BTWS}) {
+        DevBuf& b = ctx->bufs[slot];
+        if (b.p) (void)hipFree(b.p);
+        b = DevBuf{};
+    }
+    mem.lean = true;
+    return eig_attempt(ctx, n64, H, fp32, rho, n_vectors, guard_tol, max_vectors, vec_first, mem);
 }
 
 // ---------------------------------------------------------------------------

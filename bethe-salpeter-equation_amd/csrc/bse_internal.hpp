@@ -218,6 +218,7 @@ struct bse_ctx {
     hipStream_t st = nullptr;
     std::string err;
     std::vector<DevBuf> bufs;   // indexed by slot id
+    size_t mem_limit = SIZE_MAX;    // bytes the buffers may hold together (BSE_MEMORY_LIMIT, read by every eigensolve)
     // problem
     bool have_problem = false;
     bse_system sys{};
@@ -336,6 +337,13 @@ int fail(bse_ctx* c, int code, const std::string& msg) {
             return fail(ctx, BSE_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(_e)); \
     } while (0)
 
+// Device memory in the context's buffers.
+size_t held_bytes(const bse_ctx* ctx) {
+    size_t sum = 0;
+    for (const DevBuf& b : ctx->bufs) sum += b.cap;
+    return sum;
+}
+
 void* buf(bse_ctx* ctx, int slot, size_t bytes, int* status) {
     DevBuf& b = ctx->bufs[slot];
     if (bytes == 0) bytes = 16;
@@ -355,7 +363,8 @@ void* buf(bse_ctx* ctx, int slot, size_t bytes, int* status) {
         return b.p;
     }
     if (b.p) { (void)hipFree(b.p); b.p = nullptr; b.cap = 0; }
-    if (hipMalloc(&b.p, bytes) != hipSuccess) {
+    if (held_bytes(ctx) + bytes > ctx->mem_limit || hipMalloc(&b.p, bytes) != hipSuccess) {
+        (void)hipGetLastError();            // the next launch is not to report it
         b.p = nullptr;
         *status = fail(ctx, BSE_ERR_ALLOC, "hipMalloc failed for " + std::to_string(bytes) + " bytes");
         return nullptr;
