@@ -354,6 +354,17 @@ def main():
         eps64 = ctx.spectrum(omegas, s.eta)
         log(f"fp64 all-vector path: {t_fp64:.3f} s (first call {cold['fp64_all_vectors_s']:.3f} s), "
             f"stages {stages_fp64}")
+        # both use the two-stage reduction: the one-stage reduction, in a context of
+        # its own and untimed, is the independent comparison
+        os.environ["BSE_TWO_STAGE"] = "0"
+        one = _abi.Context(0)
+        del os.environ["BSE_TWO_STAGE"]
+        one.set_system(s)
+        one.build("fp64")
+        one.eigh(0)
+        E64_one = one.eigenvalues()
+        assert one.reduction_info()["reduction"] == "one stage"
+        one.close()
         nchk = 256
         Z64 = ctx.eigenvectors(nchk)
         scale = float(np.abs(E64).max())
@@ -368,6 +379,8 @@ def main():
             speedup_vs_fp64_all_vectors=t_fp64 / t_mixed, speedup_vs_fp64_lowest16=t_fp64_16 / t_mixed,
             lowest16_err_meV_vs_fp64=err_mev,
             all_eigenvalues_max_err_meV_vs_fp64=float(np.abs(E_mixed - E64).max() * 1e3),
+            lowest16_two_stage_fp64_vs_one_stage_fp64_eV=float(np.abs(E64_16[:n_low] - E64_one[:n_low]).max()),
+            all_eigenvalues_two_stage_vs_one_stage_fp64_eV=float(np.abs(E64 - E64_one).max()),
             lowest16_fp64_16_vectors_vs_all_vectors_eV=float(np.abs(E64_16[:n_low] - E64[:n_low]).max()),
             eigenvector_overlap_per_cluster=overlaps,
             spectrum_rel_l2_vs_fp64=spec_l2,
