@@ -1053,7 +1053,8 @@ static bool memory_to_spare(const bse_ctx* ctx, int n, int nvec, const EigMemory
 // guard_tol > 0: eigenvalues within guard_tol above the last requested one
 // are formed as well, up to max_vectors in total (ctx->nvec reports the count).
 // vec_first > 0: the vectors formed are those of the sorted eigenvalues
-// vec_first .. vec_first + n_vectors - 1 (one-stage reduction, no guard).
+// vec_first .. vec_first + n_vectors - 1 (no guard; one stage, or two with the
+// chase's reflectors kept).
 static int eig_attempt(bse_ctx* ctx, int64_t n64, void* H, int fp32, const double2* rho, int n_vectors,
                        double guard_tol, int max_vectors, int vec_first, EigMemory& mem)
 {
@@ -1103,7 +1104,6 @@ static int eig_attempt(bse_ctx* ctx, int64_t n64, void* H, int fp32, const doubl
         stage_end(ctx, ST_TRD);
     }
     if (!two) {
-    bse_hetrd_workspace(n, nb, &vs_el, &yr_el, &yc_el, &part_d);
     bse_hetrd_workspace(n, nb, &vs_el, &yr_el, &yc_el, &part_d);
     {
         int64_t off = 0;

@@ -271,9 +271,9 @@ struct bse_ctx {
     // caller's k order (bse_set_problem_klist): list position of each grid
     // index and its inverse; empty for the plain grid
     std::vector<int> kmap_h, kinv_h;
-    // two-stage reduction: 0 auto (for at most 20 eigenvectors and n >= 256),
-    // 1 whenever the eigenvectors asked for are at most 20, -1 never
-    // (BSE_TWO_STAGE=1 / 0); band panels of the last two-stage reduction
+    // two-stage reduction: 0 auto by order, storage and vectors wanted, 1 at any
+    // order (FP32 storage: for at most 20 vectors), -1 never (BSE_TWO_STAGE=1 /
+    // 0; use_two_stage and use_q2 in bse_api.hip); band panels of the last two-stage reduction
     // (row start, rows, reflectors, offset into the reflector store)
     int two_stage = 0;
     bool last_two_stage = false;

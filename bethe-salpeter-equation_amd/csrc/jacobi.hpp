@@ -16,8 +16,10 @@ __device__ inline double jacobi_rsq(double x) {
 struct JacobiRot { double c, dl; double2 s; };
 __device__ inline JacobiRot jacobi_rot(double app, double aqq, double2 a) {
     // h = (a_qq - a_pp)/2, r = sqrt(h^2 + |a|^2), c^2 = (r + |h|)/(2 r),
-    // s = sign(h) a / (2 r c); the pair is scaled by its size so that no
-    // square leaves the range
+    // s = sign(h) a / (2 r c); the pair is scaled by its size, so c and s have
+    // all their digits however small a pair is (the sweeps' own convergence
+    // tests form squares of the entries as they are: matrices of a size between
+    // about 1e-140 and 1e150)
     JacobiRot t;
     const double h0 = 0.5 * (aqq - app);
     const double big = fmax(fabs(h0), fmax(fabs(a.x), fabs(a.y)));

@@ -18,7 +18,7 @@
 //
 // Mapping: MP x MP lanes per matrix, MP = 1, 2, 4 or 8 >= norb / 2 (the order
 // is padded with a zero row and column), 64 / MP^2 matrices per wave, A and V in
-// LDS (8 KB per wave whatever MP).  Lane (P, Q) applies a round's rotations to
+// LDS (12, 10, 9 and 8.5 KB per wave).  Lane (P, Q) applies a round's rotations to
 // the 2 x 2 block of A in the rows of pair P and the columns of pair Q, and
 // that of pair Q to rows P and P + MP of V.  A round is bound by its latency
 // (LDS reads, two reciprocal square roots, LDS writes), so the lanes share

@@ -278,9 +278,9 @@ int  bse_eigh_dense(bse_ctx* ctx, int n, const double* a, int64_t lda, int a_on_
 /* Stage timings of the last build/eigh (milliseconds, HIP events):
  * [0] tb, [1] tables, [2] assembly, [3] tridiagonalisation, [4] tridiagonal
  * eigenvalues, [5] tridiagonal vectors, [6] back-transform, [7] refinement,
- * [8] oscillator+spectrum; after a two-stage reduction (few vectors, large
- * N) [9] dense -> band with Q1^H rho and [10] band -> tridiagonal, the two
- * parts of [3] (0 after a one-stage reduction).  n <= 16. */
+ * [8] oscillator+spectrum; after a two-stage reduction [9] dense -> band with
+ * Q1^H rho and [10] band -> tridiagonal, the two parts of [3] (0 after a
+ * one-stage reduction).  n <= 16. */
 int  bse_stage_times(const bse_ctx* ctx, double* ms, int n);
 
 /* How the last eigensolve reduced its matrix to tridiagonal form: out[0] 0 one

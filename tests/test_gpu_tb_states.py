@@ -47,7 +47,8 @@ def test_every_order(ctx, norb, nk):
 
 @pytest.mark.parametrize("scale", [1e-140, 1e140])
 def test_scale(ctx, scale):
-    """Entries whose squares leave the range of a double."""
+    """Units in which the sums of squares that decide on convergence are still
+    normal numbers, but nothing of higher order is."""
     m = tb.random_square(6, seed=3)
     from dataclasses import replace
     big = replace(m, h_r=m.h_r * scale)
@@ -55,6 +56,7 @@ def test_scale(ctx, scale):
     e, u = ctx.tb_states_at(k, model=big)
     e1, _ = ctx.tb_states_at(k, model=m)
     assert np.abs(e / scale - e1).max() < 1e-12 * np.abs(e1).max()
+    _check(m, k, e / scale, u)
 
 
 @pytest.mark.parametrize("norb", [2, 6, 16])
