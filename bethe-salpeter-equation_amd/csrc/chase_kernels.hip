@@ -89,15 +89,19 @@ __device__ inline Refl column_refl(double2& x, bool tail) {
                                      __builtin_amdgcn_readlane(__double2loint(x.y), 0)));
     };
     sums();
-    int up = 0;
-    // (the sums are the wave's, so every lane takes the same turn)
-    while (up < 960 && __any(cabs2(alpha) + ss < 1e-290) && __any(x.x != 0.0 || x.y != 0.0)) {
-        x = cmk(ldexp(x.x, 480), ldexp(x.y, 480));
-        up += 480;
-        sums();
-    }
+    // (the sums are the wave's, so every lane takes the same turn; asked behind
+    // the reflector, whose square root and divisions a sweep waits for anyway)
     Refl r = make_refl(alpha, ss);
-    if (up) r.beta = ldexp(r.beta, -up);
+    if (__builtin_expect(__any(cabs2(alpha) + ss < 1e-290), 0)) {
+        int up = 0;
+        while (up < 960 && __any(x.x != 0.0 || x.y != 0.0) && __any(cabs2(alpha) + ss < 1e-290)) {
+            x = cmk(ldexp(x.x, 480), ldexp(x.y, 480));
+            up += 480;
+            sums();
+        }
+        r = make_refl(alpha, ss);
+        r.beta = ldexp(r.beta, -up);
+    }
     return r;
 }
 
